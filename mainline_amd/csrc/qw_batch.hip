@@ -9,151 +9,11 @@
 // system per process (src/program_utils/ooqmc.cpp:148-170, src/method/Dmc_method.cpp:328-567).
 #include <numeric>
 
+#include "qw_batch.hpp"
 #include "qw_engine.hpp"
+#include "qw_panel.hpp"
 
 namespace qw {
-
-// One system of a batched launch.
-struct BatchSlot {
-  DevSys S;
-  MixedTables M;
-  DevWalkers W;
-  BigPtrs<float> Pf;
-  BigPtrs<double> Pd;
-  DmcCtl* ctl;
-  unsigned long long* keys;
-  int* vals;
-  int* psrc;
-  int* pdst;
-  unsigned* stepp;
-  unsigned long long seed;
-  int n[2];     // electrons of each spin
-  int ns;       // register tile of the inverse (4..64); 0 = block-per-walker path
-  int u;        // LCAO coefficient loads in flight (per size bucket, tuned)
-  int inv_rows; // 33..64 electrons of a spin: row-per-lane inversion instead of 8x8 blocks
-  int cap;      // basis tile of the block-per-walker sweep
-  // the slot's method: DMC (depth 1, node-crossing moves rejected, weights and branching)
-  // or VMC (depth 2 with delayed rejection, ndecorr sweeps per step)
-  int depth, ndecorr, lmode, pp_mode;
-  int branch_np;  // branching after this step: the feedback interval's steps (0 = none)
-  double tau;
-  // block-per-... layout: walkers (wavefronts) per 256-thread block, the LDS bytes of each,
-  // rows per lane of the one-wavefront sweep above 64 electrons of a spin (2 or 4)
-  int wpb, lds_w, nr;
-  // the slot's FP64 recompute interval (mixed path): a multiple of the batch's launch interval
-  // R, or at least n (once per sweep); the recompute launch after moves [k0, k0 + R) covers
-  // the slot when k0 + R is a multiple of rf or ends the sweep
-  int rf;
-};
-
-constexpr int kBatchWpb = 4;  // walkers (wavefronts) per 256-thread block for <= 64 per spin
-
-// A field of the slot table (constant address space) as the generic reference the kernel
-// bodies take.
-template <typename T>
-__device__ inline const T& gref(const QW_CONST T& r) {
-  return *(const T*)&r;
-}
-
-// Blocks of a slot in a sweep launch (wpb walkers each), and in a recompute launch (a
-// wavefront per walker up to 64 electrons of a spin, a whole block per walker above).
-__device__ inline int batch_blocks(const QW_CONST BatchSlot& B) { return (B.W.nw + B.wpb - 1) / B.wpb; }
-__device__ inline int batch_blocks_inv(const QW_CONST BatchSlot& B) {
-  return B.ns ? (B.W.nw + kBatchWpb - 1) / kBatchWpb : B.W.nw;
-}
-
-// Whether slot B recomputes spin s after the moves [k0, k0 + R) (host and device).
-__host__ __device__ inline bool batch_recomputes(int rf, int n, int k0, int R) {
-  return (k0 + R) % rf == 0 || k0 + R >= n;
-}
-
-// The slot of block `blk` among the slots of method depth `depth` with a sweep `sw` and moves
-// k0.. of spin s (INV: and a recompute after the R moves from k0), and the slot's first block
-// (*b0).  Uniform over the block; nslot is small.
-template <bool INV = false>
-__device__ inline int batch_find(const QW_CONST BatchSlot* sl, int nslot, int s, int k0, int depth, int sw, int blk,
-                                 int* b0, int R = 0) {
-  int acc = 0;
-  for (int i = 0; i < nslot; i++) {
-    if (sl[i].n[s] <= k0 || sl[i].depth != depth || sw >= sl[i].ndecorr) continue;
-    if (INV && !batch_recomputes(sl[i].rf, sl[i].n[s], k0, R)) continue;
-    const int nb = INV ? batch_blocks_inv(sl[i]) : batch_blocks(sl[i]);
-    if (blk < acc + nb) {
-      *b0 = acc;
-      return i;
-    }
-    acc += nb;
-  }
-  return -1;
-}
-
-// Moves k0 .. min(n_s, k0 + R) of spin s, in sweep `sw` of the step, of every slot of method
-// depth DEPTH (1 DMC, 2 VMC) with more than k0 electrons of that spin.  PREC: 0 FP64, 1 mixed
-// (FP32 LCAO and inverse).
-template <int PREC, int DEPTH>
-__global__ __launch_bounds__(256, 2) void k_sweep_batch(const BatchSlot* __restrict__ slots, int nslot, int s, int k0,
-                                                        int R, int sw) {
-  extern __shared__ double ldsb[];
-  const QW_CONST BatchSlot* sl = cptr(slots);
-  int b0 = 0;
-  const int i = batch_find(sl, nslot, s, k0, DEPTH, sw, (int)blockIdx.x, &b0);
-  if (i < 0) return;
-  const QW_CONST BatchSlot& B = sl[i];
-  const int n = B.n[s];
-  SweepArgs A{s, k0, min(n, k0 + R), B.tau, B.seed, 0u, (unsigned)sw, DEPTH == 1 ? 1 : 0, 0, B.stepp};
-  A.dets = A.k1 == n && sw == B.ndecorr - 1;
-  const int t = (int)threadIdx.x, blk = (int)blockIdx.x - b0;
-  char* lds = (char*)ldsb;
-  if (B.ns == 0) {
-    // more than 64 electrons of a spin: B.wpb walkers per block, a wavefront each
-    const int lane = t & 63, wid = t >> 6;
-    if (wid >= B.wpb) return;
-    const int w = blk * B.wpb + wid;
-    char* base = lds + (size_t)wid * B.lds_w;
-    if constexpr (PREC == 0) {
-      if (B.nr == 2)
-        sweep_w_body<double, double, DEPTH, 2, kBatchWpb>(gref(B.S), gref(B.W), gref(B.Pd), A, B.cap, w, lane, base);
-      else
-        sweep_w_body<double, double, DEPTH, 4, kBatchWpb>(gref(B.S), gref(B.W), gref(B.Pd), A, B.cap, w, lane, base);
-    } else {
-      if (B.nr == 2)
-        sweep_w_body<float, float, DEPTH, 2, kBatchWpb>(gref(B.S), gref(B.W), gref(B.Pf), A, B.cap, w, lane, base);
-      else
-        sweep_w_body<float, float, DEPTH, 4, kBatchWpb>(gref(B.S), gref(B.W), gref(B.Pf), A, B.cap, w, lane, base);
-    }
-    return;
-  }
-  const int lane = t & 63, wid = t >> 6, w = blk * kBatchWpb + wid;
-#define QW_MX(NS, U) \
-  sweep_mx_body<NS, DEPTH, LCAO_FP32, U, kBatchWpb, false>(gref(B.S), gref(B.M), gref(B.W), A, w, lane, wid, lds)
-#define QW_FP(NS, U) sweep_fp64_body<NS, DEPTH, U, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds)
-#define QW_CASES(X, U0, U1, U2)                 \
-  switch (B.ns * 100 + B.u) {                   \
-    case 400 + U0: X(4, U0); break;             \
-    case 400 + U1: X(4, U1); break;             \
-    case 400 + U2: X(4, U2); break;             \
-    case 800 + U0: X(8, U0); break;             \
-    case 800 + U1: X(8, U1); break;             \
-    case 800 + U2: X(8, U2); break;             \
-    case 1600 + U0: X(16, U0); break;           \
-    case 1600 + U1: X(16, U1); break;           \
-    case 1600 + U2: X(16, U2); break;           \
-    case 3200 + U0: X(32, U0); break;           \
-    case 3200 + U1: X(32, U1); break;           \
-    case 3200 + U2: X(32, U2); break;           \
-    case 6400 + U0: X(64, U0); break;           \
-    case 6400 + U1: X(64, U1); break;           \
-    default: X(64, U2); break;                  \
-  }
-  if constexpr (PREC == 0) {
-    QW_CASES(QW_FP, 2, 4, 8)
-  } else {
-    QW_CASES(QW_MX, 4, 8, 16)
-  }
-#undef QW_CASES
-#undef QW_FP
-#undef QW_MX
-}
 
 // FP64 recompute of spin s's inverse for the slots with moves k0.. of spin s (after their
 // FP32 updates): four walkers per block with a wavefront each up to 64 electrons of a spin,
@@ -402,7 +262,6 @@ struct qw_batch {
       B.M = e.MT;
       B.W = e.W;
       B.Pf = BigPtrs<float>{e.W.invf, e.W.mof, {e.MT.Cf[0], e.MT.Cf[1]}, e.MT.spline};
-      B.Pd = BigPtrs<double>{e.W.inv, e.W.mo, {e.S.C[0], e.S.C[1]}, e.S.spline};
       B.ctl = e.dctl;
       B.keys = e.keys;
       B.vals = e.vals;
@@ -413,7 +272,7 @@ struct qw_batch {
       B.n[0] = e.T.nup;
       B.n[1] = e.T.ndn;
       B.ns = e.big ? 0 : e.ns;
-      B.cap = precision == QW_PREC_FP64 ? kCapF64 : kCapF32;
+      B.cap = kCapF32;
       const int bi = bucket_of(B.ns);
       B.u = (B.ns && bi < (int)buckets.size()) ? bucket_u[bi] : (precision == QW_PREC_FP64 ? 4 : 8);
       B.inv_rows = e.inv_rows ? 1 : 0;
@@ -424,16 +283,22 @@ struct qw_batch {
       B.tau = m.timestep;
       B.branch_np = (step_mode && m.method == 1 && mb.ip + 1 == mb.np) ? mb.np : 0;
       B.rf = std::max(e.refresh, refresh);
-      if (B.ns) {
+      if (precision == QW_PREC_FP64 && B.depth == 1) {
+        const int nmax = std::max(e.T.nup, e.T.ndn), w = B.ns ? 1 : nmax <= 128 ? 2 : 4;
+        B.wpb = B.ns ? kPanelWpb : 1;
+        lds_sweep = std::max(lds_sweep, panel_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, B.ns ? B.ns : 64 * w, w,
+                                                        B.wpb));
+      } else if (B.ns) {
         const size_t per =
             precision == QW_PREC_FP64
-                ? ((sweep_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.ns, kCapF64, 8, B.depth) + 15) & ~(size_t)15)
+                ? lds_round16(sweep_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.ns, kCapF64, 8, B.depth))
                 : sweep_mx_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.ns, LCAO_FP32, e.MT.ldchi, B.depth);
         B.wpb = kBatchWpb;
         lds_sweep = std::max(lds_sweep, (size_t)kBatchWpb * per);
       } else {
-        const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, B.cap,
-                                             precision == QW_PREC_FP64 ? 8 : 4);
+        const bool f64 = precision == QW_PREC_FP64;
+        const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, f64 ? kCapF64 : B.cap,
+                                             f64 ? sizeof(double) : sizeof(float));
         // walkers per block while their LDS leaves room for two blocks per compute unit
         B.wpb = (int)std::max<size_t>(1, std::min<size_t>(kBatchWpb, (80u << 10) / per));
         B.lds_w = (int)per;
@@ -473,12 +338,8 @@ struct qw_batch {
     const unsigned g = sweep_grid(s, k0, DEPTH, sw);
     if (!g) return;
     launch(0, [&] {
-      if (precision == QW_PREC_FP64)
-        hipLaunchKernelGGL((k_sweep_batch<0, DEPTH>), dim3(g), dim3(256), lds_sweep, stream, d_slots, nslot(), s, k0,
-                           R, sw);
-      else
-        hipLaunchKernelGGL((k_sweep_batch<1, DEPTH>), dim3(g), dim3(256), lds_sweep, stream, d_slots, nslot(), s, k0,
-                           R, sw);
+      (precision == QW_PREC_FP64 ? launch_sweep_batch_f64 : launch_sweep_batch_mx)(DEPTH, g, lds_sweep, stream, d_slots,
+                                                                                   nslot(), s, k0, R, sw);
     });
   }
   void recompute(int s, int k0, int depth, int sw) {

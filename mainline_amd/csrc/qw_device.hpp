@@ -19,10 +19,11 @@ __device__ inline const QW_CONST T* cptr(const T* p) {
   return (const QW_CONST T*)p;
 }
 
-// Compact shell record for LDS staging: rc = min(shell cutoff, object cutoff);
+// Compact shell record for LDS staging: rc2 = the smallest number whose square root reaches
+// min(shell cutoff, object cutoff), so r2 < rc2 says exactly what sqrt(r2) < cutoff says;
 // meta = atom | sym << 10 | nf << 14 | table << 18.
 struct ShellLds {
-  double rc;
+  double rc2;
   int meta;
   int f0;
 };
@@ -64,6 +65,11 @@ struct DevSys {
   // are eit_a0[t] .. eit_a0[t+1]-1 in type order (positions eit_pos, charges eit_Z), their
   // objects eit[eit_o0[t] .. eit_o0[t+1]-1]
   int n_eit;
+  // 1: the usual trial function: a Jastrow of one CUTOFF_CUSP and one POLYPADE object of at most
+  // four functions (the same coefficients for like and unlike spins) between electrons, in this
+  // order, and one such POLYPADE object per atom type, evaluated without loops over objects and
+  // functions; and shells of S, P, 5D, 6D and 10F symmetry only
+  int usual;
   const JRad<double>* eit;
   const JRad<float>* eitf;
   const int* eit_a0;
@@ -384,7 +390,9 @@ __device__ __attribute__((noinline)) void shell_poly_val(int sym, double f, doub
 
 // Values of one spline shell at distance vector (x,y,z), r: writes nf functions x 5
 // components to out[c*ld + i] (S, P, 5D, 6D, 10F; src/basis_function/Cubic_spline_calc.cpp:353-700).
-template <typename T>
+// FG = false: the caller's shells are S, P, 5D, 6D or 10F only (no out-of-line call, across which
+// a kernel's live registers would have to be saved).
+template <typename T, bool FG = true>
 __device__ inline void shell_lap(int sym, double f, double fd, double f2, double x, double y, double z, T* out, int ld) {
   auto put = [&](int i, double v0, double v1, double v2, double v3, double v4) {
     out[i] = (T)v0;
@@ -454,7 +462,7 @@ __device__ inline void shell_lap(int sym, double f, double fd, double f2, double
       put(9, v3 * f, h * x + v2 * y, h * y + v2 * x, h * z + f * x * y, v3 * f2 + 8. * h);
       break;
     default:  // 7F, 7F_crystal, 9G, 9G_pyscf, 15G
-      shell_poly_lap<T>(sym, f, fd, f2, x, y, z, out, ld);
+      if constexpr (FG) shell_poly_lap<T>(sym, f, fd, f2, x, y, z, out, ld);
       break;
   }
 }

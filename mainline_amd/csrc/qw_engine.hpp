@@ -24,6 +24,7 @@
 #include "qw_multidet.hpp"
 #include "qw_parm.hpp"
 #include "qw_setup.hpp"
+#include "qw_sweep.hpp"
 
 using namespace qw;
 
@@ -52,6 +53,14 @@ constexpr int kRefreshDefault = 32;
 // spin and an update O(n^2) a move, so a fixed 32 would make the recompute the larger part
 // (eight recomputes per sweep at 256 a spin).
 inline int default_refresh(int n) { return n <= 64 ? kRefreshDefault : (n / 2 + 31) / 32 * 32; }
+
+// The smallest x with sqrt(x) >= rc (correctly rounded square roots).
+inline double cutoff_squared(double rc) {
+  double x = rc * rc;
+  while (std::sqrt(x) < rc) x = std::nextafter(x, HUGE_VAL);
+  while (x > 0 && std::sqrt(std::nextafter(x, 0.0)) >= rc) x = std::nextafter(x, 0.0);
+  return x;
+}
 
 inline int pick_ns(int n) {
   int ns = 4;
@@ -89,6 +98,16 @@ std::vector<JRad<R>> jrad_table(const std::vector<JObj>& objs) {
   }
   if (out.empty()) out.push_back(JRad<R>{});
   return out;
+}
+
+// Whether the Jastrow has the form DevSys::usual names (objects of one e-i type: o0[t]..o0[t+1]).
+inline bool usual_jastrow(const std::vector<JObj>& ee, const std::vector<JObj>& eit, const std::vector<int>& o0) {
+  if (ee.size() != 2 || ee[0].kind != 0 || ee[1].kind != 1 || ee[1].nf > 4) return false;
+  for (int i = 0; i < ee[1].nf; i++)
+    if (ee[1].cl[i] != ee[1].cu[i]) return false;
+  for (size_t t = 0; t + 1 < o0.size(); t++)
+    if (o0[t + 1] - o0[t] != 1 || eit[o0[t]].kind != 1 || eit[o0[t]].nf > 4) return false;
+  return o0.size() > 1;
 }
 
 struct qw_engine {
@@ -364,6 +383,9 @@ struct qw_engine {
       }
       if (eit.empty()) eit.push_back(JObj{});
       S.n_eit = (int)rep.size();
+      S.usual = usual_jastrow(T.ee, eit, o0) ? 1 : 0;
+      for (const ShellDesc& d : T.shells)
+        if (d.sym > SK_10F) S.usual = 0;
       S.eit = upload(jrad_table<double>(eit));
       S.eitf = upload(jrad_table<float>(eit));
       S.eit_a0 = upload(a0);
@@ -376,7 +398,7 @@ struct qw_engine {
       std::vector<ShellLds> shl(T.shells.size());
       for (size_t i = 0; i < T.shells.size(); i++) {
         const ShellDesc& d = T.shells[i];
-        shl[i].rc = std::min(d.rcut, d.objthr);
+        shl[i].rc2 = cutoff_squared(std::min(d.rcut, d.objthr));
         shl[i].meta = d.atom | (d.sym << 10) | (d.nf << 14) | (d.table << 18);
         shl[i].f0 = d.f0;
       }
@@ -511,9 +533,6 @@ struct qw_engine {
   // ---- kernels
   // LDS: tiles of basis values (5 x chunk_nf doubles) and active-function indices (chunk_nf ints)
   size_t lds_rows() const { return 5 * (size_t)S.chunk_nf * sizeof(double) + (size_t)S.chunk_nf * sizeof(int); }
-  size_t lds_sweep(int depth) const {
-    return sweep_lds_bytes(S.ne, S.na, S.nsh, S.ntab, ns, kCapF64, sizeof(double), depth);
-  }
   size_t lds_local() const {
     return (7 * (size_t)S.ne + 5 * (size_t)S.chunk_nf) * sizeof(double) + (size_t)S.chunk_nf * sizeof(int);
   }
@@ -577,10 +596,6 @@ struct qw_engine {
   }
   void run_sweep(int s, int k0, int k1, double tau, unsigned sweep, int depth, int restrict_nodes, int dets) {
     SweepArgs A{s, k0, k1, tau, seed, step, sweep, restrict_nodes, dets, dstep};
-    if (big) {
-      big_sweep(A, depth);
-      return;
-    }
     if (md) {
       const size_t lds = sweep_md_lds_bytes(S.ne, S.ndet, S.nsig, S.nsp, S.chunk_nf, depth);
       launch("k_sweep", [&] {
@@ -589,33 +604,16 @@ struct qw_engine {
       });
       return;
     }
-    if (precision != QW_PREC_FP64) {
-      mixed_sweep(*this, A, depth);
+    if (precision == QW_PREC_FP64) {
+      const int u = pick_u();
+      tuned_launch([&] {
+        if (depth == 1) launch_sweep_f64(S, W, A, u, stream);
+        else launch_sweep_vmc64(S, W, A, ns, u, stream);
+      });
       return;
     }
-    const int u = pick_u();
-    if (depth == 1) {
-      if (u == 2) sweep_fp64<1, 2>(A);
-      else if (u == 8) sweep_fp64<1, 8>(A);
-      else sweep_fp64<1, 4>(A);
-    } else {
-      if (u == 2) sweep_fp64<2, 2>(A);
-      else if (u == 8) sweep_fp64<2, 8>(A);
-      else sweep_fp64<2, 4>(A);
-    }
-  }
-  template <int DEPTH, int U>
-  void sweep_fp64(const SweepArgs& A) {
-    auto go = [&](auto kern) {
-      tuned_launch([&] { hipLaunchKernelGGL(kern, dim3(nw), dim3(64), lds_sweep(DEPTH), stream, S, W, A); });
-    };
-    switch (ns) {
-      case 4: go(k_sweep<4, DEPTH, U>); break;
-      case 8: go(k_sweep<8, DEPTH, U>); break;
-      case 16: go(k_sweep<16, DEPTH, U>); break;
-      case 32: go(k_sweep<32, DEPTH, U>); break;
-      default: go(k_sweep<64, DEPTH, U>); break;
-    }
+    if (big) big_sweep(A, depth);
+    else mixed_sweep(*this, A, depth);
   }
 
   // ---- online tuning of the sweep launch: LCAO coefficient loads in flight (U) and, on the
@@ -643,7 +641,7 @@ struct qw_engine {
   }
   int pick_u() {
     if (tune_u) return tune_u;
-    if (!tune_enabled || capturing || big || (precision != QW_PREC_FP64 && precision != QW_PREC_MIXED_FP32))
+    if (!tune_enabled || capturing || (big && precision != QW_PREC_FP64) || (precision != QW_PREC_FP64 && precision != QW_PREC_MIXED_FP32))
       return u_default();
     tune_cur = cands()[tune_n % cands().size()];
     return tune_cur;
@@ -764,34 +762,14 @@ struct qw_engine {
     lu_refresh(0);
     lu_refresh(1);
   }
-  template <typename TI, typename R>
-  void big_sweep_t(const SweepArgs& A, int depth, const BigPtrs<TI>& P, int cap) {
-    // one wavefront per walker, lanes over two (<= 128 per spin) or four rows
-    const size_t lds = sweep_w_lds_bytes(S.ne, S.na, S.nsh, S.ntab, S.nsp, cap, sizeof(TI));
-    const bool nr2 = std::max(T.nup, T.ndn) <= 2 * kWave;
-    launch("k_sweep", [&] {
-      if (depth == 1) {
-        if (nr2) hipLaunchKernelGGL((k_sweep_w<TI, R, 1, 2>), dim3(nw), dim3(kWave), lds, stream, S, W, P, A, cap);
-        else hipLaunchKernelGGL((k_sweep_w<TI, R, 1, 4>), dim3(nw), dim3(kWave), lds, stream, S, W, P, A, cap);
-      } else {
-        if (nr2) hipLaunchKernelGGL((k_sweep_w<TI, R, 2, 2>), dim3(nw), dim3(kWave), lds, stream, S, W, P, A, cap);
-        else hipLaunchKernelGGL((k_sweep_w<TI, R, 2, 4>), dim3(nw), dim3(kWave), lds, stream, S, W, P, A, cap);
-      }
-    });
-  }
+  // mixed path above 64 electrons of a spin: moves, then the recompute, per interval
   void big_sweep(const SweepArgs& A0, int depth) {
-    if (precision == QW_PREC_FP64) {
-      BigPtrs<double> P{W.inv, W.mo, {S.C[0], S.C[1]}, S.spline};
-      big_sweep_t<double, double>(A0, depth, P, kCapF64);
-      return;
-    }
-    BigPtrs<float> P{W.invf, W.mof, {MT.Cf[0], MT.Cf[1]}, MT.spline};
     for (int k0 = A0.k0; k0 < A0.k1; k0 += refresh) {
       SweepArgs A = A0;
       A.k0 = k0;
       A.k1 = std::min(A0.k1, k0 + refresh);
       A.dets = A0.dets && A.k1 == A0.k1;
-      big_sweep_t<float, float>(A, depth, P, kCapF32);
+      launch("k_sweep", [&] { launch_sweep_mx_big(S, MT, W, A, depth, stream); });
       lu_refresh(A.s);
     }
   }

@@ -4,9 +4,10 @@
 //                evaluation); src/orbitals/MO_matrix_cutoff.h:480-560
 //   k_inv<NS>    pivoted inversion, log|det|, sign and transposed inverse per walker and spin;
 //                src/program_utils/MatrixAlgebrac.cpp:108-224,316-421
-//   k_sweep<NS,D> single-electron moves of one spin channel: drift, proposal, ratio, Jastrow,
-//                acceptance, Sherman-Morrison update with the inverse held in registers;
+//   k_sweep<NS,U> VMC moves of one spin channel (delayed rejection): drift, proposal, ratio,
+//                Jastrow, acceptance, Sherman-Morrison update with the inverse held in registers;
 //                src/method/Split_sample.cpp:302-540, src/program_utils/MatrixAlgebrac.cpp:766-838
+//                (DMC moves: qw_panel.hpp; the mixed path: qw_mixed.hpp and qw_big.hpp)
 //   k_local      local energy (kinetic, Coulomb, nonlocal pseudopotential), DMC weight, block
 //                sums; src/system/System.cpp:53-140, Molecular_system.cpp:209-284,
 //                Pseudopotential.cpp:596-815, src/method/Dmc_method.cpp:801-824
@@ -551,7 +552,7 @@ __global__ __launch_bounds__(64, 3) void k_inv_blk(DevSys S, const TIN* mo, TI* 
   k_inv_blk_body<1>(S, mo, inv_out, logdet_out, sgn_out, w, s, (int)threadIdx.x, L);
 }
 
-// ---------------------------------------------------------------- k_sweep
+// ---------------------------------------------------------------- sweeps
 struct SweepArgs {
   int s, k0, k1;
   double tau;

@@ -63,7 +63,7 @@ __device__ inline int basis_active(const DevSys& S, const SysLds& V, const doubl
       const ShellLds d = V.sh[sh];
       const double* ap = V.apos + 4 * shl_atom(d.meta);
       const double x = p[0] - ap[0], y = p[1] - ap[1], z = p[2] - ap[2];
-      act = sqrt(x * x + y * y + z * z) < d.rc;
+      act = x * x + y * y + z * z < d.rc2;
     }
     const unsigned long long m = __ballot(act);
     if (act) V.actl[nact + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = sh;
