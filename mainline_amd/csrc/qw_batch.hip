@@ -11,6 +11,7 @@
 
 #include "qw_batch.hpp"
 #include "qw_engine.hpp"
+#include "qw_local.hpp"
 #include "qw_panel.hpp"
 
 namespace qw {
@@ -73,9 +74,11 @@ __global__ __launch_bounds__(64) void k_local_batch(const BatchSlot* __restrict_
   A.seed = B.seed;
   A.ctl = B.ctl;
   if constexpr (PREC == 0)
-    local_body<double, false, PP>(gref(B.S), gref(B.W), A, (int)blockIdx.x - b0, (int)threadIdx.x, ldsl);
+    if (B.S.usual) local_body<double, false, PP, true>(gref(B.S), gref(B.W), A, (int)blockIdx.x - b0, (int)threadIdx.x, ldsl);
+    else local_body<double, false, PP, false>(gref(B.S), gref(B.W), A, (int)blockIdx.x - b0, (int)threadIdx.x, ldsl);
   else
-    local_body<float, false, PP>(gref(B.S), gref(B.W), A, (int)blockIdx.x - b0, (int)threadIdx.x, ldsl);
+    if (PP && B.S.usual) local_body<float, false, PP, true>(gref(B.S), gref(B.W), A, (int)blockIdx.x - b0, (int)threadIdx.x, ldsl);
+    else local_body<float, false, PP, false>(gref(B.S), gref(B.W), A, (int)blockIdx.x - b0, (int)threadIdx.x, ldsl);
 }
 
 // Trial energy, effective timestep and the pair comb of each branching slot (one block each):
@@ -306,7 +309,7 @@ struct qw_batch {
         lds_sweep = std::max(lds_sweep, (size_t)B.wpb * per);
       }
       any_pp |= e.S.has_pp != 0;
-      lds_local = std::max(lds_local, e.S.has_pp ? e.lds_local() : e.lds_local_nopp());
+      lds_local = std::max(lds_local, local_lds_bytes(e.S));
       slots.push_back(B);
     }
     if ((int)slots.size() > slot_cap) {

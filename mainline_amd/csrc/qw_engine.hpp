@@ -306,6 +306,14 @@ struct qw_engine {
     S.tab_sp = upload(T.tab_spacing);
     for (int s = 0; s < 2; s++) {
       S.C[s] = upload(T.C[s]);
+      S.Ct[s] = nullptr;
+      if (S.has_pp) {
+        const size_t n = (size_t)T.nmo[s];
+        std::vector<double> ct((size_t)T.nb * n);
+        for (size_t b = 0; b < (size_t)T.nb; b++)
+          for (size_t j = 0; j < n; j++) ct[j * T.nb + b] = T.C[s][b * n + j];
+        S.Ct[s] = upload(ct);
+      }
       std::vector<float> cf(T.C[s].begin(), T.C[s].end());
       S.Cf[s] = upload(cf);
     }
@@ -533,12 +541,6 @@ struct qw_engine {
   // ---- kernels
   // LDS: tiles of basis values (5 x chunk_nf doubles) and active-function indices (chunk_nf ints)
   size_t lds_rows() const { return 5 * (size_t)S.chunk_nf * sizeof(double) + (size_t)S.chunk_nf * sizeof(int); }
-  size_t lds_local() const {
-    return (7 * (size_t)S.ne + 5 * (size_t)S.chunk_nf) * sizeof(double) + (size_t)S.chunk_nf * sizeof(int);
-  }
-  // without a pseudopotential: positions, determinant gradients and laplacians only
-  size_t lds_local_nopp() const { return 7 * (size_t)S.ne * sizeof(double); }
-
   void run_mo_rows() {
     launch("k_mo_rows", [&] {
       hipLaunchKernelGGL(k_mo_rows, dim3((unsigned)((size_t)nw * S.ne)), dim3(64), lds_rows(), stream, S, W, nw);
@@ -701,19 +703,7 @@ struct qw_engine {
     });
   }
   void run_local(const LocalArgs& A) {
-    if (md) {
-      const size_t lds = lds_local() + ((size_t)5 * S.ndet + S.nsp + 2) * sizeof(double);
-      launch("k_local", [&] { hipLaunchKernelGGL((k_local<double, true>), dim3(nw), dim3(64), lds, stream, S, W, A); });
-      return;
-    }
-    if (precision != QW_PREC_FP64) {
-      mixed_local(*this, A);
-      return;
-    }
-    launch("k_local", [&] {
-      if (S.has_pp) hipLaunchKernelGGL(k_local<double>, dim3(nw), dim3(64), lds_local(), stream, S, W, A);
-      else hipLaunchKernelGGL((k_local<double, false, false>), dim3(nw), dim3(64), lds_local_nopp(), stream, S, W, A);
-    });
+    launch("k_local", [&] { launch_local(S, W, A, precision == QW_PREC_FP64, stream); });
   }
   // ---- more than 64 electrons per spin
   // working matrices of k_inv_panel (more than 128 electrons of a spin)

@@ -7,10 +7,8 @@
 //   k_sweep<NS,U> VMC moves of one spin channel (delayed rejection): drift, proposal, ratio,
 //                Jastrow, acceptance, Sherman-Morrison update with the inverse held in registers;
 //                src/method/Split_sample.cpp:302-540, src/program_utils/MatrixAlgebrac.cpp:766-838
-//                (DMC moves: qw_panel.hpp; the mixed path: qw_mixed.hpp and qw_big.hpp)
-//   k_local      local energy (kinetic, Coulomb, nonlocal pseudopotential), DMC weight, block
-//                sums; src/system/System.cpp:53-140, Molecular_system.cpp:209-284,
-//                Pseudopotential.cpp:596-815, src/method/Dmc_method.cpp:801-824
+//                (DMC moves: qw_panel.hpp; the mixed path: qw_mixed.hpp and qw_big.hpp; the
+//                local energy: qw_local.hpp)
 //   k_branch     trial energy, effective timestep, fixed-population pair branching;
 //                src/method/Dmc_method.cpp:776-797,961-995
 //   k_copy       walker state copies decided by k_branch
@@ -93,94 +91,6 @@ __device__ inline double lcao_val_n(const DevSys& S, int s, int n, const double 
 __device__ inline double lcao_val(const DevSys& S, int s, const double p[3], double* chi, int* flist, int lane) {
   return lcao_val_n(S, s, s ? S.ndn : S.nup, p, chi, flist, lane);
 }
-
-// Basis values at the points p[0..nq-1] (NQ >= nq) over the union of their active shells of
-// shells sh0..sh1-1: chi[i*ld + b] for point i and packed function b (exactly zero where the
-// shell is outside its cutoff for that point), flist[b] the function index.  Returns the
-// number of packed functions.
-template <int NQ>
-__device__ inline int basis_val_multi(const DevSys& S, const double (*p)[3], int nq, int sh0, int sh1, double* chi,
-                                      int ld, int* flist, int lane) {
-  int base = 0;
-  for (int s0 = sh0; s0 < sh1; s0 += kWave) {
-    const int sh = s0 + lane;
-    ShellDesc d;
-    double x[NQ], y[NQ], z[NQ], r[NQ];
-    bool act[NQ];
-    bool any = false;
-    if (sh < sh1) {
-      d = S.shells[sh];
-      const double* ap = S.atom_pos + 3 * d.atom;
-#pragma unroll
-      for (int i = 0; i < NQ; i++) {
-        act[i] = false;
-        if (i >= nq) continue;
-        x[i] = p[i][0] - ap[0];
-        y[i] = p[i][1] - ap[1];
-        z[i] = p[i][2] - ap[2];
-        r[i] = sqrt(x[i] * x[i] + y[i] * y[i] + z[i] * z[i]);
-        act[i] = r[i] < d.rcut && r[i] < d.objthr;
-        any |= act[i];
-      }
-    }
-    int tot;
-    const int at = base + wave_excl_scan(any ? d.nf : 0, lane, &tot);
-    if (any) {
-#pragma unroll
-      for (int i = 0; i < NQ; i++) {
-        if (i >= nq) break;
-        double* cq = chi + i * ld + at;
-        if (act[i]) {
-          int iv = (int)(r[i] * S.tab_inv[d.table]);
-          iv = iv < 0 ? 0 : (iv >= S.nint ? S.nint - 1 : iv);
-          const double* c = S.spline + ((size_t)d.table * S.nint + iv) * 4;
-          double h = r[i] - iv * S.tab_sp[d.table];
-          double f = c[0] + h * (c[1] + h * (c[2] + h * c[3]));
-          shell_val<double>(d.sym, f, x[i], y[i], z[i], cq);
-        } else {
-          for (int k = 0; k < d.nf; k++) cq[k] = 0.0;
-        }
-      }
-      for (int k = 0; k < d.nf; k++) flist[at + k] = d.f0 + k;
-    }
-    base += tot;
-  }
-  return base;
-}
-
-// MO j (lane j < n) at the points p[0..nq-1]: phi[i].  A function outside its cutoff for a
-// point adds an exact zero there, so phi[i] equals lcao_val at p[i] bit for bit; each
-// coefficient load serves every point.
-template <int NQ>
-__device__ inline void lcao_val_multi(const DevSys& S, int s, const double (*p)[3], int nq, double* chi, int* flist,
-                                      double phi[NQ], int lane) {
-  const int n = s ? S.ndn : S.nup, ld = S.chunk_nf;
-#pragma unroll
-  for (int i = 0; i < NQ; i++) phi[i] = 0;
-  for (int ch = 0; ch < S.nchunk; ch++) {
-    int sh0 = S.chunk_sh0[ch], sh1 = S.chunk_sh0[ch + 1];
-    __syncthreads();
-    const int nact = basis_val_multi<NQ>(S, p, nq, sh0, sh1, chi, ld, flist, lane);
-    __syncthreads();
-    if (lane < n) {
-      const double* Cp = S.C[s] + lane;
-      double a[NQ];
-#pragma unroll
-      for (int i = 0; i < NQ; i++) a[i] = 0;
-#pragma unroll 4
-      for (int b = 0; b < nact; b++) {
-        const double c = Cp[(size_t)flist[b] * n];
-#pragma unroll
-        for (int i = 0; i < NQ; i++) a[i] += c * chi[i * ld + b];
-      }
-#pragma unroll
-      for (int i = 0; i < NQ; i++) phi[i] += a[i];
-    }
-  }
-}
-
-// Quadrature points of a nonlocal pseudopotential term evaluated together in k_local.
-constexpr int kPPBatch = 4;
 
 // ---------------------------------------------------------------- k_mo_rows
 static __global__ __launch_bounds__(64) void k_mo_rows(DevSys S, DevWalkers W, int nw) {
@@ -985,310 +895,6 @@ __device__ inline void md_contract(const DevSys& S, const double* invw, int s, i
   }
 #pragma unroll
   for (int c = 0; c < NC; c++) out[c] = wsum(part[c]) / den;
-}
-
-// MD: several determinants (FP64): determinant parts and quadrature ratios are weighted sums
-// over the determinants (md_contract), from their inverses in W.invd.
-// PP = false compiles the nonlocal pseudopotential out (systems without one): the kernel then
-// needs far fewer registers and runs more waves per SIMD; the arithmetic is the same.
-// The local energy of walker w by one 64-thread block (lds: the block's LDS).
-template <typename TM, bool MD = false, bool PP = true>
-__device__ __forceinline__ void local_body(const DevSys& S, const DevWalkers& W, const LocalArgs& A, int w, int lane,
-                                           double* lds) {
-  if (w >= W.nw) return;
-  const int ne = S.ne, nsp = S.nsp;
-  double* pos = lds;
-  double* gD = pos + 3 * ne;
-  double* lD = gD + 3 * ne;
-  double* chi = lD + ne;
-  int* flist = (int*)(chi + 5 * S.chunk_nf);
-  // MD: determinant weights, their log/sign, and MO values at a quadrature point
-  double* bw = (double*)(flist + ((S.chunk_nf + 1) & ~1));
-  double* mdl = bw + (MD ? S.ndet : 0);
-  double* phq = mdl + (MD ? 4 * S.ndet : 0);
-  for (int i = lane; i < 3 * ne; i += kWave) pos[i] = W.pos[(size_t)w * ne * 3 + i];
-  const TM* mog = mo_cache<TM>(W) + (size_t)w * ne * 5 * nsp;
-  double md_den = 1, md_l0 = 0, md_s0 = 1;
-  const double* md_inv = nullptr;
-  if constexpr (MD) {
-    for (int i = lane; i < 2 * S.ndet; i += kWave) {
-      mdl[i] = W.ldd[(size_t)w * 2 * S.ndet + i];
-      mdl[2 * S.ndet + i] = W.sgd[(size_t)w * 2 * S.ndet + i];
-    }
-    __syncthreads();
-    md_den = md_weights(S, mdl, mdl + 2 * S.ndet, bw, md_l0, md_s0, lane);
-    md_inv = W.invd + (size_t)w * 2 * S.ndet * S.nsig * S.nsig;
-    __syncthreads();
-    for (int e = 0; e < ne; e++) {
-      const int s = e < S.nup ? 0 : 1, k = e - (s ? S.nup : 0);
-      double t[4];
-      md_contract<4>(S, md_inv, s, k, (const double*)mog + ((size_t)e * 5 + 1) * nsp, nsp, bw, md_den, t, lane);
-      if (lane == 0) {
-        gD[3 * e] = t[0];
-        gD[3 * e + 1] = t[1];
-        gD[3 * e + 2] = t[2];
-        lD[e] = t[3];
-      }
-    }
-  }
-  // determinant gradient / laplacian per electron: lane k owns row k of its spin's inverse
-  if (A.use_dgl && !MD) {
-    for (int e = lane; e < ne; e += kWave) {
-      const double* d = W.dgl + ((size_t)w * ne + e) * 4;
-      gD[3 * e] = d[0];
-      gD[3 * e + 1] = d[1];
-      gD[3 * e + 2] = d[2];
-      lD[e] = d[3];
-    }
-  }
-  // otherwise from the inverse and the MO cache: electron by electron, lanes over the MOs, so
-  // every row is read coalesced
-  for (int s = 0; s < 2 && !A.use_dgl && !MD; s++) {
-    const int n = s ? S.ndn : S.nup, off = s ? S.nup : 0;
-    const TM* ig = inv_store<TM>(W) + ((size_t)w * 2 + s) * nsp * nsp;
-    for (int k = 0; k < n; k++) {
-      const int e = off + k;
-      double t1 = 0, t2 = 0, t3 = 0, t4 = 0;
-      for (int j = lane; j < n; j += kWave) {
-        const double iv = ig[(size_t)k * nsp + j];
-        t1 += mog[((size_t)e * 5 + 1) * nsp + j] * iv;
-        t2 += mog[((size_t)e * 5 + 2) * nsp + j] * iv;
-        t3 += mog[((size_t)e * 5 + 3) * nsp + j] * iv;
-        t4 += mog[((size_t)e * 5 + 4) * nsp + j] * iv;
-      }
-      t1 = wsum(t1);
-      t2 = wsum(t2);
-      t3 = wsum(t3);
-      t4 = wsum(t4);
-      if (lane == 0) {
-        gD[3 * e] = t1;
-        gD[3 * e + 1] = t2;
-        gD[3 * e + 2] = t3;
-        lD[e] = t4;
-      }
-    }
-  }
-  __syncthreads();
-  // Jastrow per electron (lanes over electrons), kinetic energy, Coulomb
-  double ke = 0, utot = 0, vei = 0, vee = 0;
-  for (int i = lane; i < ne; i += kWave) {
-    const double* pi = pos + 3 * i;
-    double gx = 0, gy = 0, gz = 0, l = 0, u = 0;
-    // Coulomb (FP64)
-    const QW_CONST double* epos = cptr(S.eit_pos);
-    for (int k = 0; k < S.na; k++) {
-      const QW_CONST double* ap = epos + 3 * k;
-      double x = pi[0] - ap[0], y = pi[1] - ap[1], z = pi[2] - ap[2];
-      double r, ri;
-      dist_inv(x * x + y * y + z * z, r, ri);
-      vei += cptr(S.eit_Z)[k] * ri;
-    }
-    for (int j = 0; j < i; j++) {
-      double x = pi[0] - pos[3 * j], y = pi[1] - pos[3 * j + 1], z = pi[2] - pos[3 * j + 2];
-      double r, ri;
-      dist_inv(x * x + y * y + z * z, r, ri);
-      vee += ri;
-    }
-    // Jastrow: FP64 on the FP64 path, FP32 pair terms on the mixed path
-    if constexpr (sizeof(TM) == sizeof(double)) {
-      jastrow_local<double>(S, S.ee, S.eit, pos, i, u, gx, gy, gz, l);
-    } else {
-      float uf = 0, gxf = 0, gyf = 0, gzf = 0, lf = 0;
-      jastrow_local<float>(S, S.eef, S.eitf, pos, i, uf, gxf, gyf, gzf, lf);
-      u = uf;
-      gx = gxf;
-      gy = gyf;
-      gz = gzf;
-      l = lf;
-    }
-    utot += u;
-    double dot = gD[3 * i] * gx + gD[3 * i + 1] * gy + gD[3 * i + 2] * gz;
-    double lap = lD[i] + (l + (gx * gx + gy * gy + gz * gz)) + 2 * dot;
-    ke += -0.5 * lap;
-    if (A.mode == 0) {
-      double* og = A.out_grad + ((size_t)w * ne + i) * 3;
-      og[0] = gD[3 * i] + gx;
-      og[1] = gD[3 * i + 1] + gy;
-      og[2] = gD[3 * i + 2] + gz;
-      A.out_lap[(size_t)w * ne + i] = lap;
-    }
-  }
-  ke = wsum(ke);
-  utot = wsum(utot);
-  double vloc = -wsum(vei) + S.vii + wsum(vee);
-
-  // nonlocal pseudopotential (src/system/Pseudopotential.cpp:596-815)
-  double vnl = 0;
-  if (PP && S.has_pp) {
-    double rot[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
-    if (A.mode == 0) {
-      if (A.rot)
-        for (int i = 0; i < 9; i++) rot[i] = A.rot[i];
-    } else {
-      random_rotation(A.seed, (unsigned)w, step_of(A.step, A.stepp), rot);
-    }
-    for (int a = 0; a < S.na; a++) {
-      const int pk = cptr(S.atom_pp)[a];
-      if (pk < 0) continue;
-      const QW_CONST PPType& P = cptr(S.pp)[pk];
-      const QW_CONST double* ap = cptr(S.atom_pos) + 3 * a;
-      for (int e0 = 0; e0 < ne; e0 += kWave) {
-        const int e = e0 + lane;
-        bool want = false;
-        double vl[kMaxPPL];
-        if (e < ne) {
-          double x = pos[3 * e] - ap[0], y = pos[3 * e + 1] - ap[1], z = pos[3 * e + 2] - ap[2];
-          double r = sqrt(x * x + y * y + z * z);
-          pp_radial(P, cptr(S.atom_Z)[a], r, vl);
-          if (A.pp_mode == 0) {
-            want = r < P.cutoff;
-          } else {
-            double strength = 0;
-            for (int l = 0; l < P.L - 1; l++) strength += 10.0 * (2 * l + 1) * fabs(vl[l]);
-            strength = fmin(1.0, strength);
-            double rr = A.mode == 0 ? A.pp_rand[((size_t)w * S.na + a) * ne + e]
-                                    : uniform(A.seed, (unsigned)w, step_of(A.step, A.stepp), (unsigned)(a * ne + e), TAG_PP);
-            want = strength > rr;
-          }
-          vnl += vl[P.L - 1];  // local channel for every electron
-          if (A.tneg && !want) A.tneg[((size_t)w * S.na + a) * ne + e] = 0.0;
-        }
-        unsigned long long mask = __ballot(want);
-        while (mask) {
-          const int b = __ffsll((long long)mask) - 1;
-          mask &= mask - 1;
-          const int ee = e0 + b;
-          const int s = ee < S.nup ? 0 : 1, k = ee - (s ? S.nup : 0), n = s ? S.ndn : S.nup;
-          const double* re = pos + 3 * ee;
-          double od[3] = {re[0] - ap[0], re[1] - ap[1], re[2] - ap[2]};
-          double orr = sqrt(od[0] * od[0] + od[1] * od[1] + od[2] * od[2]);
-          double v[kMaxPPL];
-          pp_radial(P, cptr(S.atom_Z)[a], orr, v);
-          if (A.pp_mode == 1) {
-            double strength = 0;
-            for (int l = 0; l < P.L - 1; l++) strength += 10.0 * (2 * l + 1) * fabs(v[l]);
-            strength = fmin(1.0, strength);
-            if (fabs(strength) > 0)
-              for (int l = 0; l < P.L - 1; l++) v[l] /= strength;
-          }
-          double gtmp[3];
-          const double u_old = jastrow_e_val(S, ee, re, pos, lane);
-          (void)gtmp;
-          const double ivk =
-              (!MD && lane < n) ? (double)inv_store<TM>(W)[(((size_t)w * 2 + s) * nsp + k) * nsp + lane] : 0.0;
-          double nl = 0, nneg = 0;
-          // the quadrature points kPPBatch at a time: one pass of the basis, the LCAO
-          // (each coefficient load serving every point) and the Jastrow pairs per batch,
-          // each point's value bitwise that of a pass of its own
-          for (int q0 = 0; q0 < P.aip; q0 += kPPBatch) {
-            const int nq = P.aip - q0 < kPPBatch ? P.aip - q0 : kPPBatch;
-            double np_[kPPBatch][3], cs[kPPBatch];
-#pragma unroll
-            for (int i = 0; i < kPPBatch; i++) {
-              const int q = i < nq ? q0 + i : q0;
-              double qx = P.q[q][0] * rot[0] + P.q[q][1] * rot[3] + P.q[q][2] * rot[6];
-              double qy = P.q[q][0] * rot[1] + P.q[q][1] * rot[4] + P.q[q][2] * rot[7];
-              double qz = P.q[q][0] * rot[2] + P.q[q][1] * rot[5] + P.q[q][2] * rot[8];
-              np_[i][0] = re[0] + (qx * orr - od[0]);
-              np_[i][1] = re[1] + (qy * orr - od[1]);
-              np_[i][2] = re[2] + (qz * orr - od[2]);
-              double nd[3] = {np_[i][0] - ap[0], np_[i][1] - ap[1], np_[i][2] - ap[2]};
-              double nr = sqrt(nd[0] * nd[0] + nd[1] * nd[1] + nd[2] * nd[2]);
-              cs[i] = (nd[0] * od[0] + nd[1] * od[1] + nd[2] * od[2]) / (nr * orr);
-            }
-            double Rq[kPPBatch], uq[kPPBatch];
-            if constexpr (MD) {
-              for (int i = 0; i < nq; i++) {
-                const double phm = lcao_val_n(S, s, S.nmo[s], np_[i], chi, flist, lane);
-                __syncthreads();
-                if (lane < S.nmo[s]) phq[lane] = phm;
-                __syncthreads();
-                md_contract<1>(S, md_inv, s, k, phq, nsp, bw, md_den, &Rq[i], lane);
-              }
-            } else {
-              double phi[kPPBatch];
-              lcao_val_multi<kPPBatch>(S, s, np_, nq, chi, flist, phi, lane);
-#pragma unroll
-              for (int i = 0; i < kPPBatch; i++) Rq[i] = i < nq ? wsum(ivk * phi[i]) : 0.0;
-            }
-            jastrow_e_val_multi<kPPBatch>(S, ee, np_, nq, pos, uq, lane);
-            for (int i = 0; i < nq; i++) {
-              double ratio = Rq[i] * exp(uq[i] - u_old) * P.w[q0 + i];
-              double ts = 0;
-              for (int l = 0; l < P.L - 1; l++) ts += (2 * l + 1) * v[l] * legendre(cs[i], l);
-              const double vxx = ts * ratio;
-              nl += vxx;
-              if (vxx < 0.0) nneg -= vxx;
-            }
-          }
-          if (lane == 0) {
-            vnl += nl;
-            if (A.tneg) A.tneg[((size_t)w * S.na + a) * ne + ee] = nneg;
-          }
-        }
-      }
-    }
-    vnl = wsum(vnl);
-  }
-  const double etot = ke + vloc + vnl;
-  if (lane == 0) {
-    double* el = W.elast + 4 * (size_t)w;
-    el[0] = ke;
-    el[1] = vloc;
-    el[2] = vnl;
-    el[3] = etot;
-    if (A.mode == 0) {
-      if constexpr (MD) {
-        A.out_logpsi[w] = md_l0 + log(fabs(md_den)) + utot;
-        A.out_sign[w] = md_s0 * (md_den < 0 ? -1.0 : 1.0);
-      } else {
-        A.out_logpsi[w] = W.logdet[2 * w] + W.logdet[2 * w + 1] + utot;
-        A.out_sign[w] = W.sgn[2 * w] * W.sgn[2 * w + 1];
-      }
-      A.out_eparts[3 * w] = ke;
-      A.out_eparts[3 * w + 1] = vloc;
-      A.out_eparts[3 * w + 2] = vnl;
-    } else if (A.mode == 3) {
-      W.eold[w] = etot;
-    } else {
-      double wt = W.weight[w];
-      if (A.mode == 2) {
-        const DmcCtl& C = *A.ctl;
-        double teffac = C.teff / 2.0;
-        double eo = W.eold[w];
-        double fbet = fmax(C.etrial - etot, C.etrial - eo);
-        if (fbet > C.cut_stop) teffac = 0;
-        else if (fbet > C.cut_start) teffac = teffac * (1. - (fbet - C.cut_start) / (C.cut_stop - C.cut_start));
-        wt *= exp(teffac * (C.etrial * 2 - etot - eo));
-        if (wt > C.max_weight) wt = C.max_weight;
-        W.weight[w] = wt;
-      }
-      W.eold[w] = etot;
-      double* bs = W.bsum + kBsum * (size_t)w;
-      bs[0] += wt;
-      bs[1] += wt * etot;
-      bs[2] += wt * ke;
-      bs[3] += wt * vloc;
-      bs[4] += wt * vnl;
-      bs[5] += 1;
-      // unweighted first and second moments (per-point variances of the block log)
-      bs[6] += etot;
-      bs[7] += etot * etot;
-      bs[8] += ke;
-      bs[9] += ke * ke;
-      bs[10] += vloc;
-      bs[11] += vloc * vloc;
-      bs[12] += vnl;
-      bs[13] += vnl * vnl;
-      bs[14] += wt * wt;
-    }
-  }
-}
-
-template <typename TM, bool MD = false, bool PP = true>
-__global__ __launch_bounds__(64) void k_local(DevSys S, DevWalkers W, LocalArgs A) {
-  extern __shared__ double lds[];
-  local_body<TM, MD, PP>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, lds);
 }
 
 // ---------------------------------------------------------------- k_tmove

@@ -1,0 +1,28 @@
+// Launches of the local energy (qw_local.hpp).
+#include "qw_local.hpp"
+#include "qw_sweep.hpp"
+
+namespace qw {
+
+void launch_local(const DevSys& S, const DevWalkers& W, const LocalArgs& A, bool f64, hipStream_t st) {
+  const size_t lds = local_lds_bytes(S);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(64), lds, st, S, W, A); };
+  const bool u = S.usual != 0;
+  if (S.ndet > 1) {
+    if (u) go(k_local<double, true, true, true>);
+    else go(k_local<double, true, true, false>);
+  } else if (f64 && S.has_pp) {
+    if (u) go(k_local<double, false, true, true>);
+    else go(k_local<double, false, true, false>);
+  } else if (f64) {
+    if (u) go(k_local<double, false, false, true>);
+    else go(k_local<double, false, false, false>);
+  } else if (S.has_pp) {
+    if (u) go(k_local<float, false, true, true>);
+    else go(k_local<float, false, true, false>);
+  } else {
+    go(k_local<float, false, false, false>);
+  }
+}
+
+}  // namespace qw

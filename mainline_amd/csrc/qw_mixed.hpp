@@ -524,4 +524,3 @@ __global__ __launch_bounds__(64 * WPB, WPB == 1 ? 2 : 1) void k_sweep_mx(DevSys 
 void mixed_setup(qw_engine& e);
 void mixed_refresh_all(qw_engine& e);
 void mixed_sweep(qw_engine& e, const qw::SweepArgs& A, int depth);
-void mixed_local(qw_engine& e, const qw::LocalArgs& A);

@@ -25,6 +25,7 @@
 // atoms) 1.24 -> 0.92 ms; 256 electrons, 1024 walkers 173 -> 27 ms.  Two and four waves per SIMD
 // measured 4 % and 18 % slower than three at 64 electrons (four spill).
 #pragma once
+#include "qw_jastrow.hpp"
 #include "qw_kernels.hpp"
 
 namespace qw {
@@ -118,57 +119,6 @@ __device__ inline void walker_sum8(double v[8], double* red, int lane, int wv) {
 }
 
 // ---------------------------------------------------------------- Jastrow
-// Value and (d/dr)/r of the usual Jastrow (one CUTOFF_CUSP and one POLYPADE object of up to four
-// functions between electrons, one such POLYPADE object per atom type; S.usual) for one pair.
-// Functions beyond an object's count have zero coefficients.  All the denominators of a pair
-// share one reciprocal: 1/a and 1/b are b/(ab) and a/(ab).
-__device__ inline void pair_ee64(const QW_CONST JRad<double>& c, const QW_CONST JRad<double>& o, double cc, double r,
-                                 double ri, double& u, double& gf) {
-  // cusp
-  const double yc = r * c.rcinv, yc2 = yc * yc;
-  const double pp = yc - yc2 + yc * yc2 * (1.0 / 3.0);
-  const double d4 = fma(c.gamma, pp, 1.0);
-  // polynomial Pade
-  const double zz = r * o.rcinv, zz2 = zz * zz;
-  const double zpp = zz2 * (6.0 - 8.0 * zz + 3.0 * zz2);
-  const double d0 = fma(o.beta[0], zpp, 1.0), d1 = fma(o.beta[1], zpp, 1.0);
-  const double d2 = fma(o.beta[2], zpp, 1.0), d3 = fma(o.beta[3], zpp, 1.0);
-  const double d01 = d0 * d1, d23 = d2 * d3, dp = d01 * d23;
-  const double inv = rcp_nr(dp * d4);
-  const double pade = inv * dp, ip = inv * d4;
-  const double i01 = ip * d23, i23 = ip * d01;
-  const double p0 = i01 * d1, p1 = i01 * d0, p2 = i23 * d3, p3 = i23 * d2;
-  const double s0 = o.cl[0] * p0 + o.cl[1] * p1 + o.cl[2] * p2 + o.cl[3] * p3;
-  const double s1 = o.cbl[0] * p0 * p0 + o.cbl[1] * p1 * p1 + o.cbl[2] * p2 * p2 + o.cbl[3] * p3 * p3;
-  const double ppd = 1.0 - 2.0 * yc + yc2;
-  const double zppd = 12.0 * zz * (1.0 - 2.0 * zz + zz2);
-  if (r < c.rcut) {
-    u += cc * (c.rcut * (pp * pade - c.pade0));
-    gf += cc * (ppd * pade * pade * ri);
-  }
-  if (r < o.rcut) {
-    u += (1.0 - zpp) * s0;
-    gf -= zppd * ri * o.rcinv * s1;
-  }
-}
-__device__ inline void pair_ei64(const QW_CONST JRad<double>& o, double r, double ri, double& u, double& gf) {
-  const double zz = r * o.rcinv, zz2 = zz * zz;
-  const double zpp = zz2 * (6.0 - 8.0 * zz + 3.0 * zz2);
-  const double d0 = fma(o.beta[0], zpp, 1.0), d1 = fma(o.beta[1], zpp, 1.0);
-  const double d2 = fma(o.beta[2], zpp, 1.0), d3 = fma(o.beta[3], zpp, 1.0);
-  const double d01 = d0 * d1, d23 = d2 * d3;
-  const double ip = rcp_nr(d01 * d23);
-  const double i01 = ip * d23, i23 = ip * d01;
-  const double p0 = i01 * d1, p1 = i01 * d0, p2 = i23 * d3, p3 = i23 * d2;
-  const double s0 = o.cl[0] * p0 + o.cl[1] * p1 + o.cl[2] * p2 + o.cl[3] * p3;
-  const double s1 = o.cbl[0] * p0 * p0 + o.cbl[1] * p1 * p1 + o.cbl[2] * p2 * p2 + o.cbl[3] * p3 * p3;
-  const double zppd = 12.0 * zz * (1.0 - 2.0 * zz + zz2);
-  if (r < o.rcut) {
-    u += (1.0 - zpp) * s0;
-    gf -= zppd * ri * o.rcinv * s1;
-  }
-}
-
 // This thread's share (partners t, t + NT, ...) of the Jastrow terms of electron e at p: value
 // and gradient.  pos: LDS positions; epos: atoms in e-i type order, 3 doubles each.
 template <int NT, bool JP>
@@ -185,7 +135,7 @@ __device__ inline void jastrow_share(const DevSys& S, int e, const double p[3], 
       double r, ri, gf = 0, l = 0;
       dist_inv(x * x + y * y + z * z, r, ri);
       if constexpr (JP) {
-        pair_ei64(cptr(S.eit)[o0], r, ri, u, gf);
+        pair_ei64<true, false>(cptr(S.eit)[o0], r, ri, u, gf, l);
       } else {
         for (int o = o0; o < o1; o++)
           with_jrad<double, false>(cptr(S.eit)[o], [&](const auto& ev) { ev(0.0, r, ri, u, gf, l); });
@@ -204,7 +154,7 @@ __device__ inline void jastrow_share(const DevSys& S, int e, const double p[3], 
     const bool unlike = (j < S.nup) != eup;
     if constexpr (JP) {
       const QW_CONST JRad<double>* ee = cptr(S.ee);
-      pair_ee64(ee[0], ee[1], unlike ? ee[0].cu[0] : ee[0].cl[0], r, ri, u, gf);
+      pair_ee64<true, false>(ee[0], ee[1], unlike ? ee[0].cu[0] : ee[0].cl[0], r, ri, u, gf, l);
     } else {
       for (int o = 0; o < S.nee; o++)
         with_jrad<double, false>(cptr(S.ee)[o], [&](const auto& ev) { ev(unlike ? 1.0 : 0.0, r, ri, u, gf, l); });

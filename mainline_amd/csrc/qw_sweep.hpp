@@ -1,4 +1,4 @@
-// Sweep launches compiled in translation units of their own.
+// Sweep and local-energy launches compiled in translation units of their own.
 #pragma once
 #include "qw_kernels.hpp"
 #include "qw_mixed.hpp"
@@ -17,5 +17,8 @@ void launch_sweep_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W,
                      int mode, int choice, hipStream_t st);
 void launch_sweep_mx_big(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int depth,
                          hipStream_t st);
+
+// The local energy of every walker (f64: FP64 caches).
+void launch_local(const DevSys& S, const DevWalkers& W, const LocalArgs& A, bool f64, hipStream_t st);
 
 }  // namespace qw
