@@ -12,7 +12,7 @@
 #include "qw_batch.hpp"
 #include "qw_engine.hpp"
 #include "qw_local.hpp"
-#include "qw_panel.hpp"
+#include "qw_panel_mx.hpp"
 
 namespace qw {
 
@@ -292,12 +292,12 @@ struct qw_batch {
         lds_sweep = std::max(lds_sweep, panel_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, B.ns ? B.ns : 64 * w, w,
                                                         B.wpb));
       } else if (B.ns) {
-        const size_t per =
-            precision == QW_PREC_FP64
-                ? lds_round16(sweep_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.ns, kCapF64, 8, B.depth))
-                : sweep_mx_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.ns, LCAO_FP32, e.MT.ldchi, B.depth);
         B.wpb = kBatchWpb;
-        lds_sweep = std::max(lds_sweep, (size_t)kBatchWpb * per);
+        if (precision == QW_PREC_FP64)
+          lds_sweep = std::max(lds_sweep, kBatchWpb * lds_round16(sweep_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab,
+                                                                                  e.ns, kCapF64, 8, B.depth)));
+        else
+          lds_sweep = std::max(lds_sweep, panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, B.depth, 0, e.S.nsp));
       } else {
         const bool f64 = precision == QW_PREC_FP64;
         const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, f64 ? kCapF64 : B.cap,

@@ -1,11 +1,24 @@
 // Batched sweeps of the mixed path.
 #include "qw_batch.hpp"
+#include "qw_panel_mx.hpp"
 
 namespace qw {
 
+template <int DEPTH, bool JP>
+__device__ __forceinline__ void batch_small(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A,
+                                            int ns, int w, int lane, char* sh, char* own, int u) {
+  switch (ns) {
+    case 4: sweep_mxp_body<4, DEPTH, JP, false>(S, M, W, A, w, lane, sh, nullptr, own, u); break;
+    case 8: sweep_mxp_body<8, DEPTH, JP, false>(S, M, W, A, w, lane, sh, nullptr, own, u); break;
+    case 16: sweep_mxp_body<16, DEPTH, JP, false>(S, M, W, A, w, lane, sh, nullptr, own, u); break;
+    case 32: sweep_mxp_body<32, DEPTH, JP, false>(S, M, W, A, w, lane, sh, nullptr, own, u); break;
+    default: sweep_mxp_body<64, DEPTH, JP, false>(S, M, W, A, w, lane, sh, nullptr, own, u); break;
+  }
+}
+
 // The mixed path (FP32 LCAO and inverse).
 template <int DEPTH>
-__global__ __launch_bounds__(256, 2) void k_sweep_batch_mx(const BatchSlot* __restrict__ slots, int nslot, int s, int k0,
+__global__ __launch_bounds__(256, 3) void k_sweep_batch_mx(const BatchSlot* __restrict__ slots, int nslot, int s, int k0,
                                                         int R, int sw) {
   extern __shared__ double ldsb[];
   const QW_CONST BatchSlot* sl = cptr(slots);
@@ -16,6 +29,7 @@ __global__ __launch_bounds__(256, 2) void k_sweep_batch_mx(const BatchSlot* __re
   const int n = B.n[s];
   SweepArgs A{s, k0, min(n, k0 + R), B.tau, B.seed, 0u, (unsigned)sw, DEPTH == 1 ? 1 : 0, 0, B.stepp};
   A.dets = A.k1 == n && sw == B.ndecorr - 1;
+  A.keep = !batch_recomputes(B.rf, n, k0, R);
   const int t = (int)threadIdx.x, blk = (int)blockIdx.x - b0;
   char* lds = (char*)ldsb;
   if (B.ns == 0) {
@@ -30,30 +44,15 @@ __global__ __launch_bounds__(256, 2) void k_sweep_batch_mx(const BatchSlot* __re
       sweep_w_body<float, float, DEPTH, 4, kBatchWpb>(gref(B.S), gref(B.W), gref(B.Pf), A, B.cap, w, lane, base);
     return;
   }
-  const int lane = t & 63, wid = t >> 6, w = blk * kBatchWpb + wid;
-#define QW_MX(NS, U) \
-  sweep_mx_body<NS, DEPTH, LCAO_FP32, U, kBatchWpb, false>(gref(B.S), gref(B.M), gref(B.W), A, w, lane, wid, lds)
-#define QW_CASES(X, U0, U1, U2)                 \
-  switch (B.ns * 100 + B.u) {                   \
-    case 400 + U0: X(4, U0); break;             \
-    case 400 + U1: X(4, U1); break;             \
-    case 400 + U2: X(4, U2); break;             \
-    case 800 + U0: X(8, U0); break;             \
-    case 800 + U1: X(8, U1); break;             \
-    case 800 + U2: X(8, U2); break;             \
-    case 1600 + U0: X(16, U0); break;           \
-    case 1600 + U1: X(16, U1); break;           \
-    case 1600 + U2: X(16, U2); break;           \
-    case 3200 + U0: X(32, U0); break;           \
-    case 3200 + U1: X(32, U1); break;           \
-    case 3200 + U2: X(32, U2); break;           \
-    case 6400 + U0: X(64, U0); break;           \
-    case 6400 + U1: X(64, U1); break;           \
-    default: X(64, U2); break;                  \
-  }
-  QW_CASES(QW_MX, 4, 8, 16)
-#undef QW_CASES
-#undef QW_MX
+  // up to 64: four walkers per block share the tables
+  panel_mx_stage<false>(gref(B.S), gref(B.M), s, lds, t, 64 * kBatchWpb);
+  __syncthreads();
+  const int wid = t >> 6, w = blk * kBatchWpb + wid;
+  if (w >= B.W.nw) return;
+  char* own = lds + panel_mx_shared_lds(B.S.na, B.S.nsh, B.S.ntab, 0, B.S.nsp) +
+              (size_t)wid * panel_mx_walker_lds(B.S.nsh, B.ns, DEPTH);
+  if (B.S.usual) batch_small<DEPTH, true>(gref(B.S), gref(B.M), gref(B.W), A, B.ns, w, t & 63, lds, own, B.u);
+  else batch_small<DEPTH, false>(gref(B.S), gref(B.M), gref(B.W), A, B.ns, w, t & 63, lds, own, B.u);
 }
 
 void launch_sweep_batch_mx(int depth, unsigned grid, size_t lds, hipStream_t st, const BatchSlot* slots, int nslot,

@@ -471,6 +471,7 @@ struct SweepArgs {
   int restrict_nodes;
   int dets;  // write the determinant gradient / laplacian ratios of spin s to W.dgl at the end
   const unsigned* stepp;  // device step counter (replaces `step` when set; graph replays)
+  int keep;               // mixed path: the updated inverse is needed after the launch (no recompute follows)
 };
 __device__ inline unsigned step_of(unsigned step, const unsigned* stepp) { return stepp ? *stepp : step; }
 

@@ -280,84 +280,34 @@ __global__ __launch_bounds__(64) void k_mo_rows_mx(DevSys S, MixedTables M, DevW
 }
 
 // ---------------------------------------------------------------- k_sweep_mx
-// Basis functions per LDS tile batch in the FP32 sweep (one walker per block), and with the
-// coefficients staged in LDS (several walkers per block, where LDS is shared by all of them).
-constexpr int kCapF32 = 256;
-constexpr int kCapCL = 64;
-// Walkers per block of the LDS-staged variant: two waves per SIMD of one compute unit.
-constexpr int kWpbCL = 8;
 constexpr size_t kLdsMax = 163840;  // LDS per workgroup on gfx950
 
 __host__ __device__ inline size_t lds_round16(size_t b) { return (b + 15) & ~(size_t)15; }
 
-// Per-walker LDS of k_sweep_mx: positions | (several walkers per block: active-shell list) |
-// basis tile (FP32 sparse: 5 x cap floats + cap row offsets; MFMA: 5 x ldchi floats + 5 x 64
-// accumulator exchange + ldchi ints) | inverse row and value row broadcast (2 x NS floats).
-__host__ __device__ inline size_t sweep_mx_walker_lds(int ne, int nsh, int ns, int mode, int ldchi, int wpb,
-                                                      int depth) {
-  const int cap = wpb > 1 ? kCapCL : kCapF32;
-  const size_t tile = mode == LCAO_FP32 ? (size_t)5 * cap * 4 + (size_t)cap * 4
-                                        : (size_t)(5 * ldchi + 5 * 64) * 4 + (size_t)ldchi * 4;
-  return lds_round16((size_t)3 * ne * sizeof(double)) + (wpb > 1 ? lds_round16((size_t)nsh * 4) : 0) +
-         sweep_rand_bytes(ns, depth) + tile + (size_t)2 * ns * 4 + 16;
-}
-// LDS of k_sweep_mx: (several walkers per block: the spin's coefficients, nb x nsp floats) |
-// system tables | per-walker regions.
-__host__ __device__ inline size_t sweep_mx_lds_bytes(int ne, int na, int nsh, int ntab, int ns, int mode, int ldchi,
-                                                     int depth, int nb = 0, int nsp = 0, int wpb = 1) {
-  return (wpb > 1 ? lds_round16((size_t)nb * nsp * 4) : 0) + lds_round16(sys_lds_bytes(na, nsh, ntab)) +
-         (size_t)wpb * sweep_mx_walker_lds(ne, nsh, ns, mode, ldchi, wpb, depth);
+// LDS of k_sweep_mx: system tables | positions | random numbers | basis tile (5 x ldchi floats +
+// 5 x 64 accumulator exchange + ldchi ints) | inverse row and value row broadcast (2 x NS floats).
+__host__ __device__ inline size_t sweep_mx_lds_bytes(int ne, int na, int nsh, int ntab, int ns, int ldchi, int depth) {
+  return lds_round16(sys_lds_bytes(na, nsh, ntab)) + lds_round16((size_t)3 * ne * sizeof(double)) +
+         sweep_rand_bytes(ns, depth) + (size_t)(5 * ldchi + 5 * 64) * 4 + (size_t)ldchi * 4 + (size_t)2 * ns * 4 + 16;
 }
 
-// Moves of electrons [k0, k1) of spin s for WPB walkers per block (one wavefront each); all
-// FP32 except positions, drift/proposal, acceptance and log|det| (FP64).  With WPB > 1 the
-// block first stages the spin's MO coefficients in LDS, so the LCAO of every move reads LDS
-// instead of L2; the walkers then run independently (wavefront-level barriers only).  The
-// arithmetic is the same for every WPB and U.
-// The sweep of walker w by wavefront `wid` of a block of WPB wavefronts (lds0: the block's LDS).
-// STAGE: the block shares system tables and the LDS-staged coefficients (the layout above);
-// otherwise each wavefront has a whole region of its own (sweep_mx_lds_bytes with one walker)
-// and runs exactly as a one-walker block does, with wavefront-level barriers.
-template <int NS, int DEPTH, int MODE, int U, int WPB, bool STAGE>
+// Moves of electrons [k0, k1) of spin s, one walker per block, with the LCAO on the matrix cores
+// (the BF16 modes); all FP32 except positions, drift/proposal, acceptance and log|det| (FP64).
+// The FP32 LCAO's sweep is qw_panel_mx.hpp.
+template <int NS, int DEPTH, int MODE>
 __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables& M, const DevWalkers& W,
-                                              const SweepArgs& A, int w, int lane, int wid, char* lds0) {
-  static_assert(WPB == 1 || MODE == LCAO_FP32, "several walkers per block: FP32 LCAO only");
-  static_assert(!STAGE || WPB > 1, "staged coefficients are shared by several walkers");
-  const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
-  char* base = lds0;
-  float* Cl = (float*)base;
-  if constexpr (STAGE) base += lds_round16((size_t)S.nb * nsp * 4);
-  if constexpr (!STAGE && WPB > 1)
-    base += (size_t)wid * sweep_mx_lds_bytes(ne, S.na, S.nsh, S.ntab, NS, MODE, M.ldchi, DEPTH);
-  SysLds V;
-  base = sys_lds_carve(S, base, V);
-  if constexpr (STAGE) {
-    // stage the coefficients (16-byte chunks while aligned) and the system tables
-    const int tid = (int)threadIdx.x, nt = 64 * WPB, nc = S.nb * n;
-    const float4* src4 = reinterpret_cast<const float4*>(M.Cf[s]);
-    float4* dst4 = reinterpret_cast<float4*>(Cl);
-    for (int i = tid; i < nc / 4; i += nt) dst4[i] = src4[i];
-    for (int i = (nc / 4) * 4 + tid; i < nc; i += nt) Cl[i] = M.Cf[s][i];
-    stage_sys(S, V, tid, nt);
-    base += (size_t)wid * sweep_mx_walker_lds(ne, S.nsh, NS, MODE, M.ldchi, WPB, DEPTH);
-    __syncthreads();
-  } else {
-    stage_sys(S, V, lane);
-  }
+                                              const SweepArgs& A, int w, int lane, char* lds0) {
   if (w >= W.nw) return;
+  const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
+  SysLds V;
+  char* base = sys_lds_carve(S, lds0, V);
+  stage_sys(S, V, lane);
   double* pos = (double*)base;
-  char* q = base + lds_round16((size_t)3 * ne * sizeof(double));
-  if constexpr (STAGE) {
-    V.actl = (int*)q;
-    q += lds_round16((size_t)S.nsh * 4);
-  }
-  constexpr int cap = STAGE ? kCapCL : kCapF32;
-  double* rnd = (double*)q;
-  q += sweep_rand_bytes(NS, DEPTH);
-  float* chi = (float*)q;
-  float* phis = chi + 5 * (MODE == LCAO_FP32 ? cap : M.ldchi);  // MFMA modes only
-  int* flist = (int*)(MODE == LCAO_FP32 ? phis : phis + 5 * 64);
-  float* rowb = (float*)(flist + (MODE == LCAO_FP32 ? cap : M.ldchi));
+  double* rnd = (double*)(base + lds_round16((size_t)3 * ne * sizeof(double)));
+  float* chi = (float*)((char*)rnd + sweep_rand_bytes(NS, DEPTH));
+  float* phis = chi + 5 * M.ldchi;
+  int* flist = (int*)(phis + 5 * 64);
+  float* rowb = (float*)(flist + M.ldchi);
   float* phib = rowb + NS;
   for (int i = lane; i < 3 * ne; i += kWave) pos[i] = W.pos[(size_t)w * ne * 3 + i];
   sweep_randoms<DEPTH>(A, (unsigned)w, off, rnd, lane);
@@ -384,7 +334,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
     m2 = mog[(e0 * 5 + 2) * nsp + lane];
     m3 = mog[(e0 * 5 + 3) * nsp + lane];
   }
-  walker_sync<WPB>();
+  __syncthreads();
   for (int k = A.k0; k < A.k1; k++) {
     const int e = off + k;
     double r0[3] = {pos[3 * e], pos[3 * e + 1], pos[3 * e + 2]};
@@ -392,7 +342,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
 #pragma unroll
       for (int j = 0; j < NS; j++) rowb[j] = inv[j];
     }
-    walker_sync<WPB>();
+    __syncthreads();
     const float rk = lane < n ? rowb[lane] : 0.f;
     float gj0[3];
     const float u0 = jastrow_e_freg(S, e, r0, pe, gj0, lane, V.epos, 4);
@@ -408,12 +358,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
       double dr[3], rn[3], dn[3];
       lim_drift(d0, t, dr);
       for (int d = 0; d < 3; d++) rn[d] = r0[d] + (rq[d] * st + dr[d]);
-      if constexpr (MODE == LCAO_FP32 && STAGE)
-        mo_lap_point<float, float, U, WPB>(S, V, M.spline, (const float*)Cl, n, rn, chi, flist, cap, phi, lane);
-      else if constexpr (MODE == LCAO_FP32)
-        mo_lap_point<float, float, U, WPB>(S, V, M.spline, M.Cf[s], n, rn, chi, flist, cap, phi, lane);
-      else
-        lcao_lap_mx<MODE>(S, M, s, rn, chi, phis, flist, phi, lane);
+      lcao_lap_mx<MODE>(S, M, s, rn, chi, phis, flist, phi, lane);
       float t0 = wsumf(rk * phi[0]);
       float t1 = wsumf(rk * phi[1]), t2 = wsumf(rk * phi[2]), t3 = wsumf(rk * phi[3]);
       float gj[3];
@@ -456,7 +401,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
     }
     if (accepted) {
       if (lane < NS) phib[lane] = lane < n ? phi[0] : 0.f;
-      walker_sync<WPB>();
+      __syncthreads();
       if (lane < n) {
         // four independent partial sums: the dot product is not one serial FMA chain
         float tq[4] = {0, 0, 0, 0};
@@ -496,7 +441,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
       m2 = mog[(e1 * 5 + 2) * nsp + lane];
       m3 = mog[(e1 * 5 + 3) * nsp + lane];
     }
-    walker_sync<WPB>();
+    __syncthreads();
   }
   float* igw = W.invf + ((size_t)w * 2 + s) * nsp * nsp;
   inv_row_store<NS>(igw, lane, n, nsp, inv);
@@ -510,13 +455,10 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
   }
 }
 
-template <int NS, int DEPTH, int MODE, int U, int WPB>
-__global__ __launch_bounds__(64 * WPB, WPB == 1 ? 2 : 1) void k_sweep_mx(DevSys S, MixedTables M, DevWalkers W,
-                                                                          SweepArgs A) {
+template <int NS, int DEPTH, int MODE>
+__global__ __launch_bounds__(64, 2) void k_sweep_mx(DevSys S, MixedTables M, DevWalkers W, SweepArgs A) {
   extern __shared__ double ldsd[];
-  const int lane = (int)threadIdx.x & (kWave - 1), wid = WPB == 1 ? 0 : (int)(threadIdx.x / kWave);
-  sweep_mx_body<NS, DEPTH, MODE, U, WPB, (WPB > 1)>(S, M, W, A, (int)blockIdx.x * WPB + wid, lane, wid,
-                                                    (char*)ldsd);
+  sweep_mx_body<NS, DEPTH, MODE>(S, M, W, A, (int)blockIdx.x, (int)threadIdx.x, (char*)ldsd);
 }
 
 }  // namespace qw

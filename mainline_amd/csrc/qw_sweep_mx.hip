@@ -1,44 +1,59 @@
 // Launches of the mixed-precision sweeps, one kernel per size class, method depth and LCAO mode.
 #include "qw_big.hpp"
 #include "qw_mixed.hpp"
+#include "qw_panel_mx.hpp"
 #include "qw_sweep.hpp"
 
 namespace qw {
 
 namespace {
-template <int DEPTH, int MODE, int U, int WPB>
-void mixed_u(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int ns, hipStream_t st) {
-  const size_t lds = sweep_mx_lds_bytes(S.ne, S.na, S.nsh, S.ntab, ns, MODE, M.ldchi, DEPTH, S.nb, S.nsp, WPB);
-  const unsigned grid = (unsigned)((W.nw + WPB - 1) / WPB);
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WPB), lds, st, S, M, W, A); };
-  switch (ns) {
-    case 4: go(k_sweep_mx<4, DEPTH, MODE, U, WPB>); break;
-    case 8: go(k_sweep_mx<8, DEPTH, MODE, U, WPB>); break;
-    case 16: go(k_sweep_mx<16, DEPTH, MODE, U, WPB>); break;
-    case 32: go(k_sweep_mx<32, DEPTH, MODE, U, WPB>); break;
-    default: go(k_sweep_mx<64, DEPTH, MODE, U, WPB>); break;
+// FP32 LCAO (qw_panel_mx.hpp)
+template <int NS, int DEPTH, bool JP, bool STAGE>
+void go_p(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st) {
+  const size_t lds = panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, STAGE ? S.nb : 0, S.nsp);
+  hipLaunchKernelGGL((k_sweep_mxp<NS, DEPTH, JP, STAGE>), dim3((unsigned)((W.nw + kPanelWpb - 1) / kPanelWpb)),
+                     dim3(64 * kPanelWpb), lds, st, S, M, W, A, u);
+}
+template <int NS, int DEPTH>
+void panel(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int choice, hipStream_t st) {
+  if (choice >= 100) {
+    if (S.usual) go_p<NS, DEPTH, true, true>(S, M, W, A, choice - 100, st);
+    else go_p<NS, DEPTH, false, true>(S, M, W, A, choice - 100, st);
+  } else {
+    if (S.usual) go_p<NS, DEPTH, true, false>(S, M, W, A, choice, st);
+    else go_p<NS, DEPTH, false, false>(S, M, W, A, choice, st);
   }
 }
+// LCAO on the matrix cores
+template <int NS, int DEPTH, int MODE>
+void go_m(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, hipStream_t st) {
+  const size_t lds = sweep_mx_lds_bytes(S.ne, S.na, S.nsh, S.ntab, NS, M.ldchi, DEPTH);
+  hipLaunchKernelGGL((k_sweep_mx<NS, DEPTH, MODE>), dim3(W.nw), dim3(64), lds, st, S, M, W, A);
+}
+template <int NS, int DEPTH>
+void by_mode(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int mode, int choice,
+             hipStream_t st) {
+  if (mode == LCAO_BF16X6) go_m<NS, DEPTH, LCAO_BF16X6>(S, M, W, A, st);
+  else if (mode == LCAO_BF16X3) go_m<NS, DEPTH, LCAO_BF16X3>(S, M, W, A, st);
+  else panel<NS, DEPTH>(S, M, W, A, choice, st);
+}
 template <int DEPTH>
-void mixed_mode(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int ns, int mode,
-                int choice, hipStream_t st) {
-  if (mode == LCAO_BF16X6) mixed_u<DEPTH, LCAO_BF16X6, 8, 1>(S, M, W, A, ns, st);
-  else if (mode == LCAO_BF16X3) mixed_u<DEPTH, LCAO_BF16X3, 8, 1>(S, M, W, A, ns, st);
-  else switch (choice) {
-    case 4: mixed_u<DEPTH, LCAO_FP32, 4, 1>(S, M, W, A, ns, st); break;
-    case 16: mixed_u<DEPTH, LCAO_FP32, 16, 1>(S, M, W, A, ns, st); break;
-    case 104: mixed_u<DEPTH, LCAO_FP32, 4, kWpbCL>(S, M, W, A, ns, st); break;
-    case 108: mixed_u<DEPTH, LCAO_FP32, 8, kWpbCL>(S, M, W, A, ns, st); break;
-    case 116: mixed_u<DEPTH, LCAO_FP32, 16, kWpbCL>(S, M, W, A, ns, st); break;
-    default: mixed_u<DEPTH, LCAO_FP32, 8, 1>(S, M, W, A, ns, st); break;
+void by_size(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int ns, int mode, int choice,
+             hipStream_t st) {
+  switch (ns) {
+    case 4: by_mode<4, DEPTH>(S, M, W, A, mode, choice, st); break;
+    case 8: by_mode<8, DEPTH>(S, M, W, A, mode, choice, st); break;
+    case 16: by_mode<16, DEPTH>(S, M, W, A, mode, choice, st); break;
+    case 32: by_mode<32, DEPTH>(S, M, W, A, mode, choice, st); break;
+    default: by_mode<64, DEPTH>(S, M, W, A, mode, choice, st); break;
   }
 }
 }  // namespace
 
 void launch_sweep_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int depth, int ns,
                      int mode, int choice, hipStream_t st) {
-  if (depth == 1) mixed_mode<1>(S, M, W, A, ns, mode, choice, st);
-  else mixed_mode<2>(S, M, W, A, ns, mode, choice, st);
+  if (depth == 1) by_size<1>(S, M, W, A, ns, mode, choice, st);
+  else by_size<2>(S, M, W, A, ns, mode, choice, st);
 }
 
 void launch_sweep_mx_big(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int depth,
