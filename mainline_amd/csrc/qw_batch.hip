@@ -159,6 +159,8 @@ struct qw_batch {
   int kcount[4] = {0, 0, 0, 0};
   size_t lds_sweep = 0, lds_local = 0;
   bool any_pp = false;  // some slot's system has a pseudopotential
+  bool all_usual = true;  // every slot's Jastrow and shells are the usual ones (DevSys::usual)
+  bool any_big = false;  // mixed path: some slot's system has more than 64 electrons of a spin
   bool g_pp = false;    // any_pp of the recorded graph
   bool capturing = false;
   bool step_mode = false;  // made by qw_batch_open: members join and leave between steps
@@ -251,7 +253,8 @@ struct qw_batch {
   void build_slots(bool step_mode) {
     slots.clear();
     lds_sweep = lds_local = 0;
-    any_pp = false;
+    any_pp = any_big = false;
+    all_usual = true;
     std::vector<size_t> order(mem.size());
     for (size_t k = 0; k < order.size(); k++) order[k] = k;
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return mem[a].e->S.ne > mem[b].e->S.ne; });
@@ -264,7 +267,6 @@ struct qw_batch {
       B.S = e.S;
       B.M = e.MT;
       B.W = e.W;
-      B.Pf = BigPtrs<float>{e.W.invf, e.W.mof, {e.MT.Cf[0], e.MT.Cf[1]}, e.MT.spline};
       B.ctl = e.dctl;
       B.keys = e.keys;
       B.vals = e.vals;
@@ -275,7 +277,6 @@ struct qw_batch {
       B.n[0] = e.T.nup;
       B.n[1] = e.T.ndn;
       B.ns = e.big ? 0 : e.ns;
-      B.cap = kCapF32;
       const int bi = bucket_of(B.ns);
       B.u = (B.ns && bi < (int)buckets.size()) ? bucket_u[bi] : (precision == QW_PREC_FP64 ? 4 : 8);
       B.inv_rows = e.inv_rows ? 1 : 0;
@@ -298,17 +299,21 @@ struct qw_batch {
                                                                                   e.ns, kCapF64, 8, B.depth)));
         else
           lds_sweep = std::max(lds_sweep, panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, B.depth, 0, e.S.nsp));
-      } else {
-        const bool f64 = precision == QW_PREC_FP64;
-        const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, f64 ? kCapF64 : B.cap,
-                                             f64 ? sizeof(double) : sizeof(float));
+      } else if (precision == QW_PREC_FP64) {
+        const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, kCapF64, sizeof(double));
         // walkers per block while their LDS leaves room for two blocks per compute unit
         B.wpb = (int)std::max<size_t>(1, std::min<size_t>(kBatchWpb, (80u << 10) / per));
         B.lds_w = (int)per;
         B.nr = std::max(e.T.nup, e.T.ndn) <= 2 * kWave ? 2 : 4;
         lds_sweep = std::max(lds_sweep, (size_t)B.wpb * per);
+      } else {
+        B.wpb = 1;
+        lds_sweep = std::max(lds_sweep, sweep_mxb_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab,
+                                                            std::max(e.T.nup, e.T.ndn), 2, B.depth));
+        any_big = true;
       }
       any_pp |= e.S.has_pp != 0;
+      all_usual &= e.S.usual != 0;
       lds_local = std::max(lds_local, local_lds_bytes(e.S));
       slots.push_back(B);
     }
@@ -336,13 +341,26 @@ struct qw_batch {
       if (B.n[s] > k0 && B.depth == depth && sw < B.ndecorr) g += (unsigned)((B.W.nw + B.wpb - 1) / B.wpb);
     return g;
   }
+  // the moves [k0, k0 + R), in launches of at most kBigPanel of them where a system above 64
+  // electrons of a spin takes part, each followed by its updates of that system's other rows
   template <int DEPTH>
   void sweep(int s, int k0, int R, int sw) {
-    const unsigned g = sweep_grid(s, k0, DEPTH, sw);
-    if (!g) return;
+    if (!sweep_grid(s, k0, DEPTH, sw)) return;
     launch(0, [&] {
-      (precision == QW_PREC_FP64 ? launch_sweep_batch_f64 : launch_sweep_batch_mx)(DEPTH, g, lds_sweep, stream, d_slots,
-                                                                                   nslot(), s, k0, R, sw);
+      const int step = any_big ? std::min(R, kBigPanel) : R;
+      for (int kk = k0; kk < k0 + R; kk += step) {
+        const int r = std::min(step, k0 + R - kk);
+        const unsigned g = sweep_grid(s, kk, DEPTH, sw);
+        if (!g) break;
+        if (precision == QW_PREC_FP64) launch_sweep_batch_f64(DEPTH, g, lds_sweep, stream, d_slots, nslot(), s, kk, r, sw);
+        else launch_sweep_batch_mx(DEPTH, all_usual, g, lds_sweep, stream, d_slots, nslot(), s, kk, r, sw);
+        unsigned gf = 0;
+        int lo, hi;
+        if (any_big)
+          for (auto& B : slots)
+            if (batch_flushes(B, s, kk, r, DEPTH, sw, &lo, &hi)) gf += (unsigned)B.W.nw;
+        if (gf) launch_flush_batch(gf, stream, d_slots, nslot(), s, kk, r, DEPTH, sw);
+      }
     });
   }
   void recompute(int s, int k0, int depth, int sw) {

@@ -1,7 +1,7 @@
 // The slot table of launches covering several systems (qw_batch.hip), and the batched sweeps'
 // launchers (translation units of their own).
 #pragma once
-#include "qw_big.hpp"
+#include "qw_big_mx.hpp"
 #include "qw_kernels.hpp"
 #include "qw_mixed.hpp"
 
@@ -12,7 +12,6 @@ struct BatchSlot {
   DevSys S;
   MixedTables M;
   DevWalkers W;
-  BigPtrs<float> Pf;
   DmcCtl* ctl;
   unsigned long long* keys;
   int* vals;
@@ -24,14 +23,13 @@ struct BatchSlot {
   int ns;       // register tile of the inverse (4..64); 0 = more than 64 electrons of a spin
   int u;        // LCAO coefficient loads in flight (per size bucket, tuned)
   int inv_rows; // 33..64 electrons of a spin: row-per-lane inversion instead of 8x8 blocks
-  int cap;      // basis tile of the one-wavefront sweep above 64 electrons of a spin (mixed path)
   // the slot's method: DMC (depth 1, node-crossing moves rejected, weights and branching)
   // or VMC (depth 2 with delayed rejection, ndecorr sweeps per step)
   int depth, ndecorr, lmode, pp_mode;
   int branch_np;  // branching after this step: the feedback interval's steps (0 = none)
   double tau;
-  // walkers per 256-thread block; mixed path above 64 electrons of a spin: LDS bytes of each
-  // walker and rows per lane of the one-wavefront sweep (2 or 4)
+  // walkers per 256-thread block; FP64 VMC above 64 electrons of a spin: LDS bytes of each walker
+  // and rows per lane of the one-wavefront sweep (2 or 4)
   int wpb, lds_w, nr;
   // the slot's FP64 recompute interval (mixed path): a multiple of the batch's launch interval
   // R, or at least n (once per sweep); the recompute launch after moves [k0, k0 + R) covers
@@ -80,12 +78,24 @@ __device__ inline int batch_find(const QW_CONST BatchSlot* sl, int nslot, int s,
   return -1;
 }
 
+// Whether slot B (above 64 electrons of a spin, mixed path) applies the updates of the moves
+// [k0, k0 + R) of spin s to other rows, and to which (host and device).
+template <typename SLOT>
+__host__ __device__ inline bool batch_flushes(const SLOT& B, int s, int k0, int R, int depth, int sw, int* lo, int* hi) {
+  if (B.ns != 0 || B.n[s] <= k0 || B.depth != depth || sw >= B.ndecorr) return false;
+  const int n = B.n[s], k1 = n < k0 + R ? n : k0 + R;
+  flush_rows(n, k1, B.rf, sw == B.ndecorr - 1, lo, hi);
+  return *hi > 0;
+}
+
 // Moves k0 .. min(n_s, k0 + R) of spin s, in sweep `sw` of the step, of every slot of method
 // depth `depth` (1 DMC, 2 VMC) with more than k0 electrons of that spin: grid blocks of 256
 // threads with lds bytes each.
 void launch_sweep_batch_f64(int depth, unsigned grid, size_t lds, hipStream_t st, const BatchSlot* slots, int nslot,
                             int s, int k0, int R, int sw);
-void launch_sweep_batch_mx(int depth, unsigned grid, size_t lds, hipStream_t st, const BatchSlot* slots, int nslot,
-                           int s, int k0, int R, int sw);
+void launch_sweep_batch_mx(int depth, bool usual, unsigned grid, size_t lds, hipStream_t st, const BatchSlot* slots,
+                           int nslot, int s, int k0, int R, int sw);
+void launch_flush_batch(unsigned grid, hipStream_t st, const BatchSlot* slots, int nslot, int s, int k0, int R, int depth,
+                        int sw);
 
 }  // namespace qw

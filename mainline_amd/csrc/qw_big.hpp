@@ -21,8 +21,6 @@ constexpr int kBigMaxSpin = 256;
 // Electrons of a spin up to which the inverse recompute is k_inv_grid<16> (the whole matrix in
 // registers); above, k_inv_panel.
 constexpr int kGridMaxSpin = 128;
-// Basis functions per LDS tile batch of the FP32 sweep above 64 electrons of a spin.
-constexpr int kCapF32 = 256;
 
 // Spline table element type that goes with an inverse / MO cache element type.
 template <typename TI>

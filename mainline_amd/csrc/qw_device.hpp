@@ -111,6 +111,8 @@ struct DevWalkers {
   double* invd;    // several determinants: [nw][2][ndet][nsig][nsig] transposed inverses
   double* ldd;     // [nw][2][ndet] log|det|
   double* sgd;     // [nw][2][ndet] sign
+  float* pend;     // mixed path above 64 electrons of a spin: [nw][32][nsp] rows of a launch's updates
+  double* pnri;    // [nw][32] their -1/R (0: no update)
 };
 
 // ---------------------------------------------------------------- wave reductions

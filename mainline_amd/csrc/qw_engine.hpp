@@ -19,6 +19,7 @@
 
 #include "../../include/qwalk_amd.h"
 #include "qw_big.hpp"
+#include "qw_big_mx.hpp"
 #include "qw_kernels.hpp"
 #include "qw_mixed.hpp"
 #include "qw_multidet.hpp"
@@ -439,6 +440,7 @@ struct qw_engine {
       const unsigned long long nm = std::max(T.nup, T.ndn);
       if (nm > kGridMaxSpin) b += N * nm * nm * 8;  // k_inv_panel working matrices
     }
+    if (big && precision != QW_PREC_FP64) b += N * kBigPanel * (nsp * 4 + 8);  // a launch's updates (qw_big_mx.hpp)
     if (md) b += N * 2 * S.ndet * (S.nsig * S.nsig + 2) * 8;
     return b;
   }
@@ -527,6 +529,8 @@ struct qw_engine {
     } else {
       W.invd = W.ldd = W.sgd = nullptr;
     }
+    W.pend = big && precision != QW_PREC_FP64 ? walloc<float>((size_t)n * kBigPanel * nsp) : nullptr;
+    W.pnri = W.pend ? walloc<double>((size_t)n * kBigPanel) : nullptr;
     int P = 1;
     while (P < n) P <<= 1;
     keys = walloc<unsigned long long>(P);
@@ -752,15 +756,25 @@ struct qw_engine {
     lu_refresh(0);
     lu_refresh(1);
   }
-  // mixed path above 64 electrons of a spin: moves, then the recompute, per interval
+  // mixed path above 64 electrons of a spin: per recompute interval launches of at most kBigPanel
+  // moves, each followed by its updates of the rows still used, then the recompute
   void big_sweep(const SweepArgs& A0, int depth) {
+    const int n = A0.s ? T.ndn : T.nup;
     for (int k0 = A0.k0; k0 < A0.k1; k0 += refresh) {
-      SweepArgs A = A0;
-      A.k0 = k0;
-      A.k1 = std::min(A0.k1, k0 + refresh);
-      A.dets = A0.dets && A.k1 == A0.k1;
-      launch("k_sweep", [&] { launch_sweep_mx_big(S, MT, W, A, depth, stream); });
-      lu_refresh(A.s);
+      const int end = std::min(A0.k1, k0 + refresh);
+      for (int kk = k0; kk < end; kk += kBigPanel) {
+        SweepArgs A = A0;
+        A.k0 = kk;
+        A.k1 = std::min(end, kk + kBigPanel);
+        A.dets = A0.dets && A.k1 == A0.k1;
+        int lo, hi;
+        flush_rows(n, A.k1, refresh, A0.dets, &lo, &hi);
+        A.keep = hi > 0;
+        launch("k_sweep", [&] { launch_sweep_mx_big(S, MT, W, A, depth, stream); });
+        if (A.keep)
+          launch("k_flush", [&] { launch_flush_mx(S, W, A.s, A.k0, A.k1 - A.k0, lo, hi, A.dets, stream); });
+      }
+      lu_refresh(A0.s);
     }
   }
 

@@ -17,6 +17,9 @@ void launch_sweep_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W,
                      int mode, int choice, hipStream_t st);
 void launch_sweep_mx_big(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int depth,
                          hipStream_t st);
+// ... of at most 32 moves, whose updates this launch then applies to the rows [lo, hi) outside the
+// moved ones (dets: and writes the determinant parts).
+void launch_flush_mx(const DevSys& S, const DevWalkers& W, int s, int k0, int np, int lo, int hi, int dets, hipStream_t st);
 
 // The local energy of every walker (f64: FP64 caches).
 void launch_local(const DevSys& S, const DevWalkers& W, const LocalArgs& A, bool f64, hipStream_t st);

@@ -1,5 +1,5 @@
 // Launches of the mixed-precision sweeps, one kernel per size class, method depth and LCAO mode.
-#include "qw_big.hpp"
+#include "qw_big_mx.hpp"
 #include "qw_mixed.hpp"
 #include "qw_panel_mx.hpp"
 #include "qw_sweep.hpp"
@@ -58,18 +58,24 @@ void launch_sweep_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W,
 
 void launch_sweep_mx_big(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int depth,
                          hipStream_t st) {
-  // one wavefront per walker, lanes over two (<= 128 per spin) or four rows
-  const BigPtrs<float> P{W.invf, W.mof, {M.Cf[0], M.Cf[1]}, M.spline};
-  const size_t lds = sweep_w_lds_bytes(S.ne, S.na, S.nsh, S.ntab, S.nsp, kCapF32, sizeof(float));
-  const bool nr2 = (S.nup > S.ndn ? S.nup : S.ndn) <= 2 * kWave;
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(kWave), lds, st, S, W, P, A, kCapF32); };
-  if (depth == 1) {
-    if (nr2) go(k_sweep_w<float, float, 1, 2>);
-    else go(k_sweep_w<float, float, 1, 4>);
+  const int n = S.nup > S.ndn ? S.nup : S.ndn, nw = n <= 128 ? 2 : 4;
+  const size_t lds = sweep_mxb_lds_bytes(S.ne, S.na, S.nsh, S.ntab, n, nw, depth);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(64 * nw), lds, st, S, M, W, A); };
+  if (nw == 2) {
+    if (depth == 1) S.usual ? go(k_sweep_mxb<2, 1, true>) : go(k_sweep_mxb<2, 1, false>);
+    else S.usual ? go(k_sweep_mxb<2, 2, true>) : go(k_sweep_mxb<2, 2, false>);
   } else {
-    if (nr2) go(k_sweep_w<float, float, 2, 2>);
-    else go(k_sweep_w<float, float, 2, 4>);
+    if (depth == 1) S.usual ? go(k_sweep_mxb<4, 1, true>) : go(k_sweep_mxb<4, 1, false>);
+    else S.usual ? go(k_sweep_mxb<4, 2, true>) : go(k_sweep_mxb<4, 2, false>);
   }
+}
+
+void launch_flush_mx(const DevSys& S, const DevWalkers& W, int s, int k0, int np, int lo, int hi, int dets,
+                     hipStream_t st) {
+  if ((S.nup > S.ndn ? S.nup : S.ndn) <= 128)
+    hipLaunchKernelGGL(k_flush_mx<128>, dim3(W.nw), dim3(128), 0, st, S, W, s, k0, np, lo, hi, dets);
+  else
+    hipLaunchKernelGGL(k_flush_mx<256>, dim3(W.nw), dim3(256), 0, st, S, W, s, k0, np, lo, hi, dets);
 }
 
 }  // namespace qw
