@@ -7,7 +7,6 @@
 //                       large for one wavefront's registers) and each Sherman-Morrison update
 //                       streams the lane's rows; TI = inverse / MO cache element type, R =
 //                       Jastrow arithmetic
-//   k_mo_rows_big<T>    basis + LCAO of every electron (src/orbitals/MO_matrix_cutoff.h:480-560)
 //   k_inv_grid<G>       FP64 pivoted Gauss-Jordan over a G x G thread grid (up to 128 per spin)
 //   k_inv_panel         the same Gauss-Jordan for 129 to 256 per spin, panel by panel with
 //                       the working matrix in device memory (src/program_utils/MatrixAlgebrac.cpp:
@@ -282,51 +281,6 @@ template <typename TI, typename R, int DEPTH, int NR>
 __global__ __launch_bounds__(64) void k_sweep_w(DevSys S, DevWalkers W, BigPtrs<TI> P, SweepArgs A, int cap) {
   extern __shared__ double lds[];
   sweep_w_body<TI, R, DEPTH, NR, 1>(S, W, P, A, cap, (int)blockIdx.x, (int)threadIdx.x, (char*)lds);
-}
-
-// Basis + LCAO of electron e of walker w (one 256-thread block per electron): wavefront 0
-// evaluates the active functions chunk by chunk, every thread accumulates its MO.
-template <typename T>
-__global__ __launch_bounds__(256) void k_mo_rows_big(DevSys S, const double* wpos, const T* C0, const T* C1,
-                                                     T* mo_out, int nw) {
-  extern __shared__ double lds[];
-  const int t = threadIdx.x, wv = t >> 6, lane = t & 63;
-  const long blk = blockIdx.x;
-  const int w = (int)(blk / S.ne), e = (int)(blk % S.ne);
-  if (w >= nw) return;
-  const int s = e < S.nup ? 0 : 1, n = s ? S.ndn : S.nup, ld = S.chunk_nf, nsp = S.nsp;
-  const T* C = s ? C1 : C0;
-  T* chi = (T*)lds;
-  int* flist = (int*)(chi + 5 * ld);
-  int* nb = flist + ld;
-  double p[3];
-  for (int d = 0; d < 3; d++) p[d] = wpos[((size_t)w * S.ne + e) * 3 + d];
-  T acc[5] = {0, 0, 0, 0, 0};
-  for (int ch = 0; ch < S.nchunk; ch++) {
-    const int sh0 = S.chunk_sh0[ch], sh1 = S.chunk_sh0[ch + 1];
-    __syncthreads();
-    if (wv == 0) {
-      const int na_ = basis_lap_sparse<T>(S, p, sh0, sh1, chi, ld, flist, lane);
-      if (lane == 0) *nb = na_;
-    }
-    __syncthreads();
-    const int nact = *nb;
-    if (t < n) {
-      const T* Cp = C + t;
-      for (int b = 0; b < nact; b++) {
-        const T c = Cp[(size_t)flist[b] * n];
-        acc[0] += c * chi[b];
-        acc[1] += c * chi[ld + b];
-        acc[2] += c * chi[2 * ld + b];
-        acc[3] += c * chi[3 * ld + b];
-        acc[4] += c * chi[4 * ld + b];
-      }
-    }
-  }
-  if (t < n) {
-    T* row = mo_out + ((size_t)w * S.ne + e) * 5 * nsp;
-    for (int c = 0; c < 5; c++) row[(size_t)c * nsp + t] = acc[c];
-  }
 }
 
 // ---------------------------------------------------------------- k_inv_grid

@@ -543,12 +543,8 @@ struct qw_engine {
   }
 
   // ---- kernels
-  // LDS: tiles of basis values (5 x chunk_nf doubles) and active-function indices (chunk_nf ints)
-  size_t lds_rows() const { return 5 * (size_t)S.chunk_nf * sizeof(double) + (size_t)S.chunk_nf * sizeof(int); }
   void run_mo_rows() {
-    launch("k_mo_rows", [&] {
-      hipLaunchKernelGGL(k_mo_rows, dim3((unsigned)((size_t)nw * S.ne)), dim3(64), lds_rows(), stream, S, W, nw);
-    });
+    launch("k_mo_rows", [&] { launch_rows_f64(S, W, stream); });
   }
   // inverse, log|det| and sign of spin `only_spin` (both spins when -1) from the MO value rows
   template <typename TIN, typename TI>
@@ -744,14 +740,9 @@ struct qw_engine {
     });
   }
   void big_refresh_all() {
-    const size_t lds = 5 * (size_t)S.chunk_nf * sizeof(double) + (size_t)S.chunk_nf * sizeof(int) + 16;
     launch("k_mo_rows", [&] {
-      if (precision == QW_PREC_FP64)
-        hipLaunchKernelGGL(k_mo_rows_big<double>, dim3((unsigned)((size_t)nw * S.ne)), dim3(256), lds, stream, S,
-                           (const double*)W.pos, S.C[0], S.C[1], W.mo, nw);
-      else
-        hipLaunchKernelGGL(k_mo_rows_big<float>, dim3((unsigned)((size_t)nw * S.ne)), dim3(256), lds, stream, S,
-                           (const double*)W.pos, MT.Cf[0], MT.Cf[1], W.mof, nw);
+      if (precision == QW_PREC_FP64) launch_rows_f64(S, W, stream);
+      else launch_rows_mx(S, MT, W, stream);
     });
     lu_refresh(0);
     lu_refresh(1);

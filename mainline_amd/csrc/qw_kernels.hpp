@@ -1,14 +1,12 @@
 // Walker-engine kernels (FP64 path).  One 64-lane wavefront = one walker per block.
 //
-//   k_mo_rows    basis + LCAO for every electron of every walker (walker refresh, fixed-config
-//                evaluation); src/orbitals/MO_matrix_cutoff.h:480-560
 //   k_inv<NS>    pivoted inversion, log|det|, sign and transposed inverse per walker and spin;
 //                src/program_utils/MatrixAlgebrac.cpp:108-224,316-421
 //   k_sweep<NS,U> VMC moves of one spin channel (delayed rejection): drift, proposal, ratio,
 //                Jastrow, acceptance, Sherman-Morrison update with the inverse held in registers;
 //                src/method/Split_sample.cpp:302-540, src/program_utils/MatrixAlgebrac.cpp:766-838
-//                (DMC moves: qw_panel.hpp; the mixed path: qw_mixed.hpp and qw_big.hpp; the
-//                local energy: qw_local.hpp)
+//                (DMC moves: qw_panel.hpp; the mixed path: qw_panel_mx.hpp, qw_big_mx.hpp and
+//                qw_mixed.hpp; MO rows: qw_rows.hpp; the local energy: qw_local.hpp)
 //   k_branch     trial energy, effective timestep, fixed-population pair branching;
 //                src/method/Dmc_method.cpp:776-797,961-995
 //   k_copy       walker state copies decided by k_branch
@@ -90,24 +88,6 @@ __device__ inline double lcao_val_n(const DevSys& S, int s, int n, const double 
 }
 __device__ inline double lcao_val(const DevSys& S, int s, const double p[3], double* chi, int* flist, int lane) {
   return lcao_val_n(S, s, s ? S.ndn : S.nup, p, chi, flist, lane);
-}
-
-// ---------------------------------------------------------------- k_mo_rows
-static __global__ __launch_bounds__(64) void k_mo_rows(DevSys S, DevWalkers W, int nw) {
-  extern __shared__ double lds[];
-  const int lane = threadIdx.x;
-  const long blk = blockIdx.x;
-  const int w = (int)(blk / S.ne), e = (int)(blk % S.ne);
-  if (w >= nw) return;
-  const int s = e < S.nup ? 0 : 1, n = S.nmo[s];
-  double p[3];
-  for (int d = 0; d < 3; d++) p[d] = W.pos[((size_t)w * S.ne + e) * 3 + d];
-  double phi[5];
-  lcao_lap_n(S, s, n, p, lds, (int*)(lds + 5 * S.chunk_nf), phi, lane);
-  if (lane < n) {
-    double* row = W.mo + ((size_t)w * S.ne + e) * 5 * S.nsp;
-    for (int c = 0; c < 5; c++) row[c * S.nsp + lane] = phi[c];
-  }
 }
 
 // ---------------------------------------------------------------- k_inv

@@ -1,5 +1,6 @@
-// Launches of the local energy (qw_local.hpp).
+// Launches of the local energy (qw_local.hpp) and of the MO rows (qw_rows.hpp).
 #include "qw_local.hpp"
+#include "qw_rows.hpp"
 #include "qw_sweep.hpp"
 
 namespace qw {
@@ -23,6 +24,15 @@ void launch_local(const DevSys& S, const DevWalkers& W, const LocalArgs& A, bool
   } else {
     go(k_local<float, false, false, false>);
   }
+}
+
+void launch_rows_f64(const DevSys& S, const DevWalkers& W, hipStream_t st) {
+  rows_go<RowsF64>(S, W.pos, S.C[0], S.C[1], nullptr, W.mo, W.nw, st);
+}
+
+void launch_rows_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W, hipStream_t st) {
+  if (std::max(S.nmo[0], S.nmo[1]) <= 64) rows_go<RowsMx>(S, W.pos, M.Cf[0], M.Cf[1], M.spline, W.mof, W.nw, st);
+  else rows_go<RowsF32>(S, W.pos, M.Cf[0], M.Cf[1], nullptr, W.mof, W.nw, st);
 }
 
 }  // namespace qw

@@ -70,44 +70,6 @@ __device__ inline void basis_lap_f32(const DevSys& S, const MixedTables& M, cons
   }
 }
 
-// Sparse FP32 basis evaluation: active functions packed in increasing order (see
-// basis_lap_sparse); returns their count.
-__device__ inline int basis_lap_sparse_f32(const DevSys& S, const MixedTables& M, const double p[3], float* chi,
-                                           int ld, int* flist, int lane) {
-  int base = 0;
-  for (int s0 = 0; s0 < S.nsh; s0 += kWave) {
-    const int sh = s0 + lane;
-    ShellDesc d;
-    float x = 0, y = 0, z = 0, r = 0;
-    bool act = false;
-    if (sh < S.nsh) {
-      d = S.shells[sh];
-      const double* ap = S.atom_pos + 3 * d.atom;
-      x = (float)(p[0] - ap[0]);
-      y = (float)(p[1] - ap[1]);
-      z = (float)(p[2] - ap[2]);
-      r = sqrtf(x * x + y * y + z * z);
-      act = r < (float)d.rcut && r < (float)d.objthr;
-    }
-    int tot;
-    const int at = base + wave_excl_scan(act ? d.nf : 0, lane, &tot);
-    if (act) {
-      float inv = (float)S.tab_inv[d.table];
-      int iv = (int)(r * inv);
-      iv = iv < 0 ? 0 : (iv >= S.nint ? S.nint - 1 : iv);
-      const float4 c = *(const float4*)(M.spline + ((size_t)d.table * S.nint + iv) * 4);
-      float h = r - iv * (float)S.tab_sp[d.table];
-      float f = c.x + h * (c.y + h * (c.z + h * c.w));
-      float fd = (c.y + h * (2.f * c.z + h * (3.f * c.w))) / r;
-      float f2 = 2.f * c.z + 6.f * h * c.w;
-      shell_lap<float>(d.sym, f, fd, f2, x, y, z, chi + at, ld);
-      for (int i = 0; i < d.nf; i++) flist[at + i] = d.f0 + i;
-    }
-    base += tot;
-  }
-  return base;
-}
-
 // FP32 Jastrow value and gradient of electron e at p (distances from FP64 positions);
 // epos: atom positions in e-i type order with stride estride.
 __device__ inline float jastrow_e_f(const DevSys& S, int e, const double p[3], const double* pos, float g[3], int lane,
@@ -167,40 +129,14 @@ __device__ inline float jastrow_e_freg(const DevSys& S, int e, const double p[3]
   return u;
 }
 
-// LCAO of one point in the mixed path.  On return lane j < n holds phi[c] (c = value,
+// LCAO of one point on the matrix cores (the BF16 modes).  On return lane j < n holds phi[c] (c = value,
 // gradient, laplacian) of MO j.  chi: LDS tile 5 x ld floats (FP32 basis values);
 // phis: LDS 5 x 64 floats used to move MFMA accumulators to lane = MO.
 template <int MODE>
 __device__ inline void lcao_lap_mx(const DevSys& S, const MixedTables& M, int s, const double p[3], float* chi,
-                                   float* phis, int* flist, float phi[5], int lane) {
+                                   float* phis, float phi[5], int lane) {
   const int n = s ? S.ndn : S.nup, ld = M.ldchi;
   for (int c = 0; c < 5; c++) phi[c] = 0.f;
-  if (MODE == LCAO_FP32) {
-    {
-      __syncthreads();
-      const int nact = basis_lap_sparse_f32(S, M, p, chi, ld, flist, lane);
-      __syncthreads();
-      if (lane < n) {
-        const float* Cp = M.Cf[s] + lane;
-        float a0 = 0, a1 = 0, a2 = 0, a3 = 0, a4 = 0;
-#pragma unroll 8
-        for (int b = 0; b < nact; b++) {
-          float c = Cp[(size_t)flist[b] * n];
-          a0 += c * chi[b];
-          a1 += c * chi[ld + b];
-          a2 += c * chi[2 * ld + b];
-          a3 += c * chi[3 * ld + b];
-          a4 += c * chi[4 * ld + b];
-        }
-        phi[0] += a0;
-        phi[1] += a1;
-        phi[2] += a2;
-        phi[3] += a3;
-        phi[4] += a4;
-      }
-    }
-    return;
-  }
   // MFMA: D[c][j] += sum_k A[c][k] B[k][j], A = basis values (rows = 5 components, padded to
   // 16), B = coefficient fragments pre-packed per (kstep, tile, lane).  The LDS tile holds
   // all basis functions (ldchi >= nb).
@@ -261,6 +197,7 @@ __device__ inline void lcao_lap_mx(const DevSys& S, const MixedTables& M, int s,
 }
 
 // ---------------------------------------------------------------- k_mo_rows_mx
+// MO rows of the BF16 modes, one electron per block (FP32: qw_rows.hpp).
 template <int MODE>
 __global__ __launch_bounds__(64) void k_mo_rows_mx(DevSys S, MixedTables M, DevWalkers W, int nw) {
   extern __shared__ float ldsf[];
@@ -272,7 +209,7 @@ __global__ __launch_bounds__(64) void k_mo_rows_mx(DevSys S, MixedTables M, DevW
   double p[3];
   for (int d = 0; d < 3; d++) p[d] = W.pos[((size_t)w * S.ne + e) * 3 + d];
   float phi[5];
-  lcao_lap_mx<MODE>(S, M, s, p, ldsf, ldsf + 5 * M.ldchi, (int*)(ldsf + 5 * M.ldchi + 5 * 64), phi, lane);
+  lcao_lap_mx<MODE>(S, M, s, p, ldsf, ldsf + 5 * M.ldchi, phi, lane);
   if (lane < n) {
     float* row = W.mof + ((size_t)w * S.ne + e) * 5 * S.nsp;
     for (int c = 0; c < 5; c++) row[c * S.nsp + lane] = phi[c];
@@ -285,10 +222,10 @@ constexpr size_t kLdsMax = 163840;  // LDS per workgroup on gfx950
 __host__ __device__ inline size_t lds_round16(size_t b) { return (b + 15) & ~(size_t)15; }
 
 // LDS of k_sweep_mx: system tables | positions | random numbers | basis tile (5 x ldchi floats +
-// 5 x 64 accumulator exchange + ldchi ints) | inverse row and value row broadcast (2 x NS floats).
+// 5 x 64 accumulator exchange) | inverse row and value row broadcast (2 x NS floats).
 __host__ __device__ inline size_t sweep_mx_lds_bytes(int ne, int na, int nsh, int ntab, int ns, int ldchi, int depth) {
   return lds_round16(sys_lds_bytes(na, nsh, ntab)) + lds_round16((size_t)3 * ne * sizeof(double)) +
-         sweep_rand_bytes(ns, depth) + (size_t)(5 * ldchi + 5 * 64) * 4 + (size_t)ldchi * 4 + (size_t)2 * ns * 4 + 16;
+         sweep_rand_bytes(ns, depth) + (size_t)(5 * ldchi + 5 * 64) * 4 + (size_t)2 * ns * 4 + 16;
 }
 
 // Moves of electrons [k0, k1) of spin s, one walker per block, with the LCAO on the matrix cores
@@ -306,8 +243,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
   double* rnd = (double*)(base + lds_round16((size_t)3 * ne * sizeof(double)));
   float* chi = (float*)((char*)rnd + sweep_rand_bytes(NS, DEPTH));
   float* phis = chi + 5 * M.ldchi;
-  int* flist = (int*)(phis + 5 * 64);
-  float* rowb = (float*)(flist + M.ldchi);
+  float* rowb = phis + 5 * 64;
   float* phib = rowb + NS;
   for (int i = lane; i < 3 * ne; i += kWave) pos[i] = W.pos[(size_t)w * ne * 3 + i];
   sweep_randoms<DEPTH>(A, (unsigned)w, off, rnd, lane);
@@ -358,7 +294,7 @@ __device__ __forceinline__ void sweep_mx_body(const DevSys& S, const MixedTables
       double dr[3], rn[3], dn[3];
       lim_drift(d0, t, dr);
       for (int d = 0; d < 3; d++) rn[d] = r0[d] + (rq[d] * st + dr[d]);
-      lcao_lap_mx<MODE>(S, M, s, rn, chi, phis, flist, phi, lane);
+      lcao_lap_mx<MODE>(S, M, s, rn, chi, phis, phi, lane);
       float t0 = wsumf(rk * phi[0]);
       float t1 = wsumf(rk * phi[1]), t2 = wsumf(rk * phi[2]), t3 = wsumf(rk * phi[3]);
       float gj[3];

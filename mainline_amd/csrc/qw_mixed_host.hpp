@@ -73,9 +73,9 @@ void mixed_setup(qw_engine& e) {
 }
 
 namespace {
-// LDS: FP32 basis tile (5 x ldchi), MFMA accumulator exchange (5 x 64), active-function list (ldchi ints)
+// LDS: FP32 basis tile (5 x ldchi), MFMA accumulator exchange (5 x 64)
 size_t lds_mx_rows(const qw_engine& e) {
-  return (5 * (size_t)e.MT.ldchi + 5 * 64) * sizeof(float) + (size_t)e.MT.ldchi * sizeof(int);
+  return (5 * (size_t)e.MT.ldchi + 5 * 64) * sizeof(float);
 }
 
 // FP64 recompute of the FP32 inverses of spin `only_spin` (or both when -1) from the current
@@ -94,7 +94,9 @@ void mixed_rows_t(qw_engine& e) {
 
 void mixed_refresh_all(qw_engine& e) {
   switch (lcao_mode(e.precision)) {
-    case LCAO_FP32: mixed_rows_t<LCAO_FP32>(e); break;
+    case LCAO_FP32:
+      e.launch("k_mo_rows", [&] { launch_rows_mx(e.S, e.MT, e.W, e.stream); });
+      break;
     case LCAO_BF16X6: mixed_rows_t<LCAO_BF16X6>(e); break;
     default: mixed_rows_t<LCAO_BF16X3>(e); break;
   }

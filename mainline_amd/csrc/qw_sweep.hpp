@@ -24,4 +24,9 @@ void launch_flush_mx(const DevSys& S, const DevWalkers& W, int s, int k0, int np
 // The local energy of every walker (f64: FP64 caches).
 void launch_local(const DevSys& S, const DevWalkers& W, const LocalArgs& A, bool f64, hipStream_t st);
 
+// MO value, gradient and laplacian rows of every electron at W.pos, in FP64 and on the mixed path
+// (FP32 LCAO).
+void launch_rows_f64(const DevSys& S, const DevWalkers& W, hipStream_t st);
+void launch_rows_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W, hipStream_t st);
+
 }  // namespace qw
