@@ -334,20 +334,16 @@ extern "C" qw_status qw_parm_deriv(qw_engine* e, int K, const double* pos, doubl
     double* d_gd = dalloc((size_t)K * np * ne * 4 * sizeof(double));
     double* d_vg = dalloc((size_t)K * ne * 3 * sizeof(double));
     double* d_vj = nps && np ? dalloc((size_t)K * ne * 3 * sizeof(double)) : nullptr;
-    const size_t lds = (size_t)9 * ne * sizeof(double) + (e->md ? (size_t)5 * e->S.ndet * sizeof(double) : 0);
+    const int pt = e->md ? 1 : parm_split((int)ne), threads = e->md ? 64 : parm_threads((int)ne, pt);
+    const size_t lds = parm_lds_bytes((int)ne, (int)np, threads / 64, e->S.ndet);
     e->launch("k_parm_deriv", [&] {
-      if (e->md)
-        hipLaunchKernelGGL((k_parm_deriv<double, true>), dim3(K), dim3(64), lds, e->stream, e->S, e->W,
-                           (const JParmDev*)e->d_parm, (const JRad<double>*)e->d_punit, (const int*)e->d_patoms,
-                           (int)np, K, d_g, d_gd, d_vg, d_vj);
-      else if (e->precision == QW_PREC_FP64)
-        hipLaunchKernelGGL(k_parm_deriv<double>, dim3(K), dim3(64), lds, e->stream, e->S, e->W,
-                           (const JParmDev*)e->d_parm, (const JRad<double>*)e->d_punit, (const int*)e->d_patoms,
-                           (int)np, K, d_g, d_gd, d_vg, (double*)nullptr);
-      else
-        hipLaunchKernelGGL(k_parm_deriv<float>, dim3(K), dim3(64), lds, e->stream, e->S, e->W,
-                           (const JParmDev*)e->d_parm, (const JRad<double>*)e->d_punit, (const int*)e->d_patoms,
-                           (int)np, K, d_g, d_gd, d_vg, (double*)nullptr);
+      auto go = [&](auto kern, double* vj) {
+        hipLaunchKernelGGL(kern, dim3(K), dim3(threads), lds, e->stream, e->S, e->W, (const JParmDev*)e->d_parm,
+                           (const JRad<double>*)e->d_punit, (const int*)e->d_patoms, (int)np, K, pt, d_g, d_gd, d_vg, vj);
+      };
+      if (e->md) go(k_parm_deriv<double, true>, d_vj);
+      else if (e->precision == QW_PREC_FP64) go(k_parm_deriv<double>, nullptr);
+      else go(k_parm_deriv<float>, nullptr);
     });
     double* d_gs = nps ? dalloc((size_t)K * nps * sizeof(double)) : nullptr;
     double* d_gds = nps ? dalloc((size_t)K * nps * ne * 4 * sizeof(double)) : nullptr;
