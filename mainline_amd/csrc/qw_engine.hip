@@ -311,75 +311,35 @@ extern "C" qw_status qw_parm_deriv(qw_engine* e, int K, const double* pos, doubl
     const size_t ne = e->S.ne, np = (size_t)e->npar, nps = (size_t)e->nslp, nt = np + nps;
     HIPCHK(hipMemcpyAsync(e->W.pos, pos, (size_t)K * ne * 3 * sizeof(double), hipMemcpyHostToDevice, e->stream));
     e->refresh_all();
-    std::vector<void*> tmp;
-    auto dalloc = [&](size_t bytes) {
-      void* p = nullptr;
-      {
-        std::lock_guard<std::mutex> g(g_devmem_mu);
-        HIPCHK(hipMalloc(&p, std::max<size_t>(bytes, 8)));
-      }
-      tmp.push_back(p);
-      return (double*)p;
-    };
-    struct Free {
-      std::vector<void*>& v;
-      hipStream_t st;
-      ~Free() {
-        (void)hipStreamSynchronize(st);
-        std::lock_guard<std::mutex> g(g_devmem_mu);
-        for (void* p : v) (void)hipFree(p);
-      }
-    } fr{tmp, e->stream};
-    double* d_g = dalloc((size_t)K * np * sizeof(double));
-    double* d_gd = dalloc((size_t)K * np * ne * 4 * sizeof(double));
-    double* d_vg = dalloc((size_t)K * ne * 3 * sizeof(double));
-    double* d_vj = nps && np ? dalloc((size_t)K * ne * 3 * sizeof(double)) : nullptr;
+    // the caller's order: CSF coefficients, then Jastrow parameters
+    typedef qw_engine::EvalScratch Ws;
+    const size_t ng = K * nt, ngd = ng * ne * 4, nv = (size_t)K * ne * 3;
+    Ws ws(e, Ws::part(ng) + Ws::part(ngd) + 2 * Ws::part(nv));
+    double *d_g = ws.take(ng), *d_gd = ws.take(ngd), *d_vg = ws.take(nv), *d_vj = nps && np ? ws.take(nv) : nullptr;
     const int pt = e->md ? 1 : parm_split((int)ne), threads = e->md ? 64 : parm_threads((int)ne, pt);
     const size_t lds = parm_lds_bytes((int)ne, (int)np, threads / 64, e->S.ndet);
     e->launch("k_parm_deriv", [&] {
       auto go = [&](auto kern, double* vj) {
         hipLaunchKernelGGL(kern, dim3(K), dim3(threads), lds, e->stream, e->S, e->W, (const JParmDev*)e->d_parm,
-                           (const JRad<double>*)e->d_punit, (const int*)e->d_patoms, (int)np, K, pt, d_g, d_gd, d_vg, vj);
+                           (const JRad<double>*)e->d_punit, (const int*)e->d_patoms, (int)np, K, pt, (int)nt, (int)nps, d_g, d_gd, d_vg, vj);
       };
       if (e->md) go(k_parm_deriv<double, true>, d_vj);
       else if (e->precision == QW_PREC_FP64) go(k_parm_deriv<double>, nullptr);
       else go(k_parm_deriv<float>, nullptr);
     });
-    double* d_gs = nps ? dalloc((size_t)K * nps * sizeof(double)) : nullptr;
-    double* d_gds = nps ? dalloc((size_t)K * nps * ne * 4 * sizeof(double)) : nullptr;
     if (nps) {
       e->launch("k_parm_det", [&] {
         hipLaunchKernelGGL(k_parm_det, dim3(K), dim3(64), parm_det_lds_bytes((int)ne, e->S.ndet), e->stream, e->S,
                            e->W, (const int*)e->d_csf_d0, (const double*)e->d_csf_w, (int)nps + 1, K,
-                           (const double*)d_vj, d_gs, d_gds);
+                           (const double*)d_vj, (int)nt, d_g, d_gd);
       });
     }
-    std::vector<double> gj((size_t)K * np), gdj((size_t)K * np * ne * 4), gs((size_t)K * nps),
-        gds((size_t)K * nps * ne * 4);
-    if (np) {
-      HIPCHK(hipMemcpyAsync(gj.data(), d_g, gj.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-      HIPCHK(hipMemcpyAsync(gdj.data(), d_gd, gdj.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+    if (nt) {
+      HIPCHK(hipMemcpyAsync(gradient, d_g, ng * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+      HIPCHK(hipMemcpyAsync(gradderiv, d_gd, ngd * sizeof(double), hipMemcpyDeviceToHost, e->stream));
     }
-    if (nps) {
-      HIPCHK(hipMemcpyAsync(gs.data(), d_gs, gs.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-      HIPCHK(hipMemcpyAsync(gds.data(), d_gds, gds.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-    }
-    HIPCHK(hipMemcpyAsync(val_gradient, d_vg, (size_t)K * ne * 3 * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(hipMemcpyAsync(val_gradient, d_vg, nv * sizeof(double), hipMemcpyDeviceToHost, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
-    // the caller's order: CSF coefficients, then Jastrow parameters
-    const size_t row = ne * 4;
-    for (int k = 0; k < K; k++) {
-      for (size_t p = 0; p < nps; p++) {
-        gradient[(size_t)k * nt + p] = gs[(size_t)k * nps + p];
-        std::copy(&gds[((size_t)k * nps + p) * row], &gds[((size_t)k * nps + p) * row] + row,
-                  gradderiv + ((size_t)k * nt + p) * row);
-      }
-      for (size_t p = 0; p < np; p++) {
-        gradient[(size_t)k * nt + nps + p] = gj[(size_t)k * np + p];
-        std::copy(&gdj[((size_t)k * np + p) * row], &gdj[((size_t)k * np + p) * row] + row,
-                  gradderiv + ((size_t)k * nt + nps + p) * row);
-      }
-    }
     // hessian: g_i g_j, except between two CSF coefficients (zero), as the reference's
     // Slater determinant leaves its block zero and extend_parm_deriv fills the rest
     if (hessian)
@@ -403,40 +363,22 @@ extern "C" qw_status qw_eval_fixed(qw_engine* e, int K, const double* pos, const
     const size_t ne = e->S.ne, na = e->S.na;
     HIPCHK(hipMemcpyAsync(e->W.pos, pos, (size_t)K * ne * 3 * sizeof(double), hipMemcpyHostToDevice, e->stream));
     e->refresh_all();
-    std::vector<void*> tmp;
-    auto dalloc = [&](size_t bytes) {
-      void* p = nullptr;
-      {
-        std::lock_guard<std::mutex> g(g_devmem_mu);
-        HIPCHK(hipMalloc(&p, std::max<size_t>(bytes, 8)));
-      }
-      tmp.push_back(p);
-      return p;
-    };
-    struct Free {
-      std::vector<void*>& v;
-      hipStream_t st;
-      ~Free() {
-        (void)hipStreamSynchronize(st);
-        std::lock_guard<std::mutex> g(g_devmem_mu);
-        for (void* p : v) (void)hipFree(p);
-      }
-    } fr{tmp, e->stream};
+    typedef qw_engine::EvalScratch Ws;
+    const size_t nr = pp_mode == 1 && pp_rand ? (size_t)K * na * ne : 0, nv = (size_t)K * ne * 3;
+    Ws ws(e, Ws::part(9) + Ws::part(nr) + 2 * Ws::part(K) + Ws::part(nv) + Ws::part((size_t)K * ne) +
+                 Ws::part((size_t)K * 3));
     double* d_rot = nullptr;
     double* d_rand = nullptr;
     if (rot) {
-      d_rot = (double*)dalloc(9 * sizeof(double));
+      d_rot = ws.take(9);
       HIPCHK(hipMemcpyAsync(d_rot, rot, 9 * sizeof(double), hipMemcpyHostToDevice, e->stream));
     }
-    if (pp_mode == 1 && pp_rand) {
-      d_rand = (double*)dalloc((size_t)K * na * ne * sizeof(double));
-      HIPCHK(hipMemcpyAsync(d_rand, pp_rand, (size_t)K * na * ne * sizeof(double), hipMemcpyHostToDevice, e->stream));
+    if (nr) {
+      d_rand = ws.take(nr);
+      HIPCHK(hipMemcpyAsync(d_rand, pp_rand, nr * sizeof(double), hipMemcpyHostToDevice, e->stream));
     }
-    double* d_lp = (double*)dalloc(K * sizeof(double));
-    double* d_sg = (double*)dalloc(K * sizeof(double));
-    double* d_gr = (double*)dalloc((size_t)K * ne * 3 * sizeof(double));
-    double* d_la = (double*)dalloc((size_t)K * ne * sizeof(double));
-    double* d_ep = (double*)dalloc((size_t)K * 3 * sizeof(double));
+    double *d_lp = ws.take(K), *d_sg = ws.take(K), *d_gr = ws.take(nv), *d_la = ws.take((size_t)K * ne),
+           *d_ep = ws.take((size_t)K * 3);
     LocalArgs A{};
     A.mode = 0;
     A.pp_mode = pp_mode;

@@ -162,6 +162,42 @@ struct qw_engine {
   int tm_mode = 0;  // 0 off, 1 TMOVES, 2 TMOVESSC (for the current run)
   void* scratch = nullptr;  // this device's copy of the allocation-free evaluation's array
 
+  // Device workspace of one evaluation call (its outputs before they are copied out), taken in
+  // parts from one allocation that the engine keeps for the next call up to kEvalKeep bytes: an
+  // allocation and a release per output and call cost more than the kernels of a small call.
+  static constexpr size_t kEvalKeep = (size_t)64 << 20;
+  void* eval_ws = nullptr;
+  size_t eval_cap = 0;
+  void eval_release() {
+    std::lock_guard<std::mutex> g(g_devmem_mu);
+    if (eval_ws) (void)hipFree(eval_ws);
+    eval_ws = nullptr;
+    eval_cap = 0;
+  }
+  struct EvalScratch {
+    qw_engine* e;
+    char* at;
+    static size_t part(size_t n) { return (n * sizeof(double) + 255) / 256 * 256; }
+    EvalScratch(qw_engine* e, size_t bytes) : e(e) {
+      if (bytes > e->eval_cap) {
+        e->eval_release();
+        std::lock_guard<std::mutex> g(g_devmem_mu);
+        HIPCHK(hipMalloc(&e->eval_ws, bytes));
+        e->eval_cap = bytes;
+      }
+      at = (char*)e->eval_ws;
+    }
+    double* take(size_t n) {
+      double* p = (double*)at;
+      at += part(n);
+      return p;
+    }
+    ~EvalScratch() {  // the call's copies have ended before its buffers go
+      (void)hipStreamSynchronize(e->stream);
+      if (e->eval_cap > kEvalKeep) e->eval_release();
+    }
+  };
+
   ~qw_engine() {
     (void)hipSetDevice(device);
     if (stream) (void)hipStreamSynchronize(stream);
@@ -170,6 +206,7 @@ struct qw_engine {
       std::lock_guard<std::mutex> g(g_devmem_mu);
       for (void* p : sys_allocs) (void)hipFree(p);
       for (void* p : walker_allocs) (void)hipFree(p);
+      if (eval_ws) (void)hipFree(eval_ws);
     }
     for (auto& e : evs) pool.push_back(e.a), pool.push_back(e.b);
     for (auto ev : pool) (void)hipEventDestroy(ev);

@@ -249,7 +249,7 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
 // D_j = D_up,j D_dn,j, Psi_S = sum_d c_d D_d, d_c = d/dx, d/dy, d/dz, laplacian of electron e;
 // vj: gradient of the parameterised Jastrow pieces (from k_parm_deriv) or null.
 static __global__ __launch_bounds__(64) void k_parm_det(DevSys S, DevWalkers W, const int* csf_d0, const double* csf_w,
-                                                 int ncsf, int nw, const double* vj, double* grad, double* gd) {
+                                                 int ncsf, int nw, const double* vj, int nt, double* grad, double* gd) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x, w = blockIdx.x;
   if (w >= nw) return;
@@ -283,7 +283,7 @@ static __global__ __launch_bounds__(64) void k_parm_det(DevSys S, DevWalkers W, 
     if (lane == 0) {
       double g = 0;
       for (int j = d0; j < d1; j++) g += csf_w[j] * ed[j] / den;
-      grad[(size_t)w * np + p] = g;
+      grad[(size_t)w * nt + p] = g;
     }
     for (int e = lane; e < ne; e += kWave) {
       const int s = e < S.nup ? 0 : 1, k = e - (s ? S.nup : 0), n = s ? S.ndn : S.nup;
@@ -298,7 +298,7 @@ static __global__ __launch_bounds__(64) void k_parm_det(DevSys S, DevWalkers W, 
       }
       if (vj) acc[3] += 2 * (acc[0] * vj[((size_t)w * ne + e) * 3] + acc[1] * vj[((size_t)w * ne + e) * 3 + 1] +
                              acc[2] * vj[((size_t)w * ne + e) * 3 + 2]);
-      double* out = gd + (((size_t)w * np + p) * ne + e) * 4;
+      double* out = gd + (((size_t)w * nt + p) * ne + e) * 4;
       for (int c = 0; c < 4; c++) out[c] = acc[c];
     }
   }

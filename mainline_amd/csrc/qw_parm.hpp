@@ -43,7 +43,8 @@ inline size_t parm_lds_bytes(int ne, int np, int nwave, int ndet) {
   return ((size_t)9 * ne + (size_t)np * nwave + (ndet > 1 ? (size_t)5 * ndet : 0)) * sizeof(double);
 }
 
-// One block per configuration; outputs grad[nw][np], gd[nw][np][ne][4], vg[nw][ne][3].  The
+// One block per configuration; outputs grad[nw][nt], gd[nw][nt][ne][4] (parameters p0 .. p0 + np of
+// nt), vg[nw][ne][3].  The
 // wavefronts share the electrons of the determinant gradient; `pt` neighbouring lanes share the
 // partners of an electron (parm_split), and their sums meet by lane exchanges.
 // MD: several determinants (the determinant gradient is their weighted sum; one wavefront, pt = 1);
@@ -54,7 +55,8 @@ inline size_t parm_lds_bytes(int ne, int np, int nwave, int ndet) {
 template <typename TM, bool MD = false>
 __global__ __launch_bounds__(MD ? 64 : 512) void k_parm_deriv(DevSys S, DevWalkers W, const JParmDev* P,
                                                               const JRad<double>* U, const int* patoms, int np, int nw,
-                                                              int pt, double* grad, double* gd, double* vg, double* vjo) {
+                                                              int pt, int nt, int p0, double* grad, double* gd,
+                                                              double* vg, double* vjo) {
   extern __shared__ double lds[];
   const int t = threadIdx.x, NT = blockDim.x, lane = t & 63, wv = t >> 6, nwave = NT >> 6, w = blockIdx.x;
   if (w >= nw) return;
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(MD ? 64 : 512) void k_parm_deriv(DevSys S, DevWalke
         l += __shfl_xor(l, m);
       }
       if (part == 0) {
-        double* o = gd + (((size_t)w * np + p) * ne + e) * 4;
+        double* o = gd + (((size_t)w * nt + p0 + p) * ne + e) * 4;
         o[0] = gx;
         o[1] = gy;
         o[2] = gz;
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(MD ? 64 : 512) void k_parm_deriv(DevSys S, DevWalke
   for (int p = t; p < np; p += NT) {
     double g = 0;
     for (int x = 0; x < nwave; x++) g += red[p * nwave + x];
-    grad[(size_t)w * np + p] = g;
+    grad[(size_t)w * nt + p0 + p] = g;
   }
   // cross terms of the laplacian derivative with the gradient of the parameterised Jastrow
   // pieces and of the determinant
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(MD ? 64 : 512) void k_parm_deriv(DevSys S, DevWalke
   for (int i = t; i < np * ne; i += NT) {
     const int e = i % ne;
     const double vx = vj[3 * e] + gD[3 * e], vy = vj[3 * e + 1] + gD[3 * e + 1], vz = vj[3 * e + 2] + gD[3 * e + 2];
-    double* o = gd + ((size_t)w * np * ne + i) * 4;
+    double* o = gd + (((size_t)w * nt + p0) * ne + i) * 4;
     o[3] += 2 * (o[0] * vx + o[1] * vy + o[2] * vz);
   }
 }
