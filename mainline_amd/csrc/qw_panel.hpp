@@ -21,8 +21,9 @@
 // wavefront, one such wave per SIMD at 1024 walkers; now a lane holds 16 doubles of the panel,
 // three waves share a SIMD, the inverse is read and written once per 16 moves, and above 64 of a
 // spin 2 or 4 wavefronts share a walker's basis, LCAO and pair terms.  Measured per launch (one
-// spin channel): 64 electrons, 8192 walkers 6.74 -> 4.39 ms; 32 electrons, 4096 walkers (pseudo-
-// atoms) 1.24 -> 0.92 ms; 256 electrons, 1024 walkers 173 -> 27 ms.  Two and four waves per SIMD
+// spin channel): 64 electrons, 8192 walkers 6.74 -> 4.0 ms; 32 electrons, 4096 walkers (pseudo-
+// atoms) 1.24 -> 0.69 ms; 256 electrons, 1024 walkers 173 -> 24.5 ms.  Of that, splitting the LCAO's
+// functions over lane groups gave 4.39 -> 4.0, 0.92 -> 0.69 and 27 -> 24.5 ms.  Two and four waves per SIMD
 // measured 4 % and 18 % slower than three at 64 electrons (four spill).
 #pragma once
 #include "qw_jastrow.hpp"
@@ -269,11 +270,98 @@ __device__ inline int panel_basis(const DevSys& S, const double* tabs, const dou
   }
   return take;
 }
-__device__ inline void panel_lcao(const double* C, const int* roff, const double* chi, int cap, int nfun, double acc[5],
-                                  int lane, int u) {
-  if (u == 8) lcao_batch<double, 8>(C, roff, chi, cap, nfun, acc, lane);
-  else if (u == 2) lcao_batch<double, 2>(C, roff, chi, cap, nfun, acc, lane);
-  else lcao_batch<double, 4>(C, roff, chi, cap, nfun, acc, lane);
+
+// ---------------------------------------------------------------- LCAO
+// The wavefront's lanes form G groups of 64 / G; group g sums the functions 2g, 2g+1 of every 2G,
+// a lane for the orbitals j, j + 64/G, ... (R of them), and the groups' sums meet at the end.  A
+// function's five values read from LDS then serve R orbitals of a lane instead of one (with every
+// lane reading them for one orbital, LDS took longer than the FMAs), and up to 32 electrons of a
+// spin no lane is idle.
+template <int NS>
+struct PanelLcao {
+  static constexpr int G = NS <= 8 ? 8 : NS <= 32 ? 4 : 2;
+  static constexpr int R = NS <= 16 ? 1 : 2;
+  static constexpr int unit = 2 * G;  // functions of a step
+};
+// Zero values after the nfun functions of a tile, up to a whole unit.
+template <int UNIT>
+__device__ inline void lcao_pad(double* chi, int* roff, int cap, int nfun, int lane) {
+  static_assert(UNIT <= 16, "unit");
+  const int i = lane & 15, c = lane >> 4;
+  if (i < (UNIT - nfun % UNIT) % UNIT) {
+    chi[c * cap + nfun + i] = 0.0;
+    if (c == 0) chi[4 * cap + nfun + i] = 0.0;
+    if (c == 1) roff[nfun + i] = 0;
+  }
+}
+template <int G, int R, int K>
+__device__ inline int lcao_units(const char* Cb, const unsigned lb[R], const int* roff, const double* chi, int cap, int b,
+                                 int nfun, double acc[R][5]) {
+  for (; b + 2 * G * (K - 1) < nfun; b += 2 * G * K) {
+    double cv[K][2][R];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int2 ro = *(const int2*)(roff + b + 2 * G * k);
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        cv[k][0][r] = *reinterpret_cast<const double*>(Cb + ((unsigned)ro.x + lb[r]));
+        cv[k][1][r] = *reinterpret_cast<const double*>(Cb + ((unsigned)ro.y + lb[r]));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all loads issue before the first use
+#pragma unroll
+    for (int k = 0; k < K; k++)
+#pragma unroll
+      for (int c = 0; c < 5; c++) {
+        const f64x2 x = *(const f64x2*)(chi + c * cap + b + 2 * G * k);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          acc[r][c] += cv[k][0][r] * x[0];
+          acc[r][c] += cv[k][1][r] * x[1];
+        }
+      }
+  }
+  return b;
+}
+// Adds a tile to the lane's partial sums; C: the wavefront's first orbital, nm of them.  2u
+// loads in flight at most (the sums do not depend on it).
+template <int G, int R>
+__device__ inline void panel_lcao(const double* C, const int* roff, const double* chi, int cap, int nfun, int nm,
+                                  double acc[R][5], int lane, int u) {
+  constexpr int L = kWave / G;
+  const char* Cb = reinterpret_cast<const char*>(C);
+  unsigned lb[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {  // lanes past the last orbital repeat it
+    const int j = lane % L + L * r;
+    lb[r] = (unsigned)(j < nm ? j : nm - 1) * 8u;
+  }
+  const int g = lane / L;
+  roff += 2 * g;
+  chi += 2 * g;
+  int b = 0;
+  if (u == 8) b = lcao_units<G, R, 8 / R>(Cb, lb, roff, chi, cap, b, nfun, acc);
+  else if (u == 4) b = lcao_units<G, R, 4 / R>(Cb, lb, roff, chi, cap, b, nfun, acc);
+  lcao_units<G, R, 1>(Cb, lb, roff, chi, cap, b, nfun, acc);
+}
+// The groups' sums: orbital `lane` of the wavefront (below 32 orbitals, repeated).
+template <int G, int R>
+__device__ inline void lcao_join(const double acc[R][5], double phi[5]) {
+#pragma unroll
+  for (int c = 0; c < 5; c++) {
+    if constexpr (G == 2 && R == 2) phi[c] = swap32_add(acc[0][c], acc[1][c]);
+    else if constexpr (G == 4 && R == 4)
+      phi[c] = swap16_add(swap32_add(acc[0][c], acc[2][c]), swap32_add(acc[1][c], acc[3][c]));
+    else if constexpr (G == 4 && R == 2)
+      phi[c] = swap16_add(swap32_add(acc[0][c], acc[0][c]), swap32_add(acc[1][c], acc[1][c]));
+    else {
+      static_assert(R == 1, "layout");
+      double v = swap32_add(acc[0][c], acc[0][c]);
+      if constexpr (G >= 4) v = swap16_add(v, v);
+      if constexpr (G == 8) v = dpp_add<kDppRor8>(v);
+      phi[c] = v;
+    }
+  }
 }
 
 // ---------------------------------------------------------------- panel rows
@@ -484,16 +572,20 @@ __device__ __forceinline__ void sweep_panel_body(const DevSys& S, const DevWalke
       const double fd = drift_scale(d0, tau);
       double rn[3];
       for (int d = 0; d < 3; d++) rn[d] = r0[d] + (rq[d] * stau + d0[d] * fd);
-      double phi[5];
-      for (int c = 0; c < 5; c++) phi[c] = 0;
+      typedef PanelLcao<NS> Lc;
+      double phi[5], part[Lc::R][5];
+#pragma unroll
+      for (int x = 0; x < Lc::R; x++)
+        for (int c = 0; c < 5; c++) part[x][c] = 0;
       const int nact = panel_active<NT>(S, shl, apos, rn, list, t);
       wave_sync();
       if constexpr (NW == 1) {
         for (int i0 = 0; i0 < nact;) {
           int nfun;
           const int take = panel_basis<!JP>(S, tabs, apos, rn, list, i0, nact, n, chi, roff, cap, &nfun, lane);
+          lcao_pad<Lc::unit>(chi, roff, cap, nfun, lane);
           wave_sync();
-          if (mine) panel_lcao(Cw, roff, chi, cap, nfun, phi, lane, u);
+          panel_lcao<Lc::G, Lc::R>(Cw, roff, chi, cap, nfun, n, part, lane, u);
           wave_sync();
           i0 += take;
         }
@@ -502,6 +594,7 @@ __device__ __forceinline__ void sweep_panel_body(const DevSys& S, const DevWalke
         for (int i0 = 0;;) {
           int nfun = 0;
           if (i0 < nact) i0 += panel_basis<!JP>(S, tabs, apos, rn, list, i0, nact, n, chi, roff, cap, &nfun, lane);
+          lcao_pad<Lc::unit>(chi, roff, cap, nfun, lane);
           if (lane == 0) {
             cnt[2 * wv] = nfun;
             cnt[2 * wv + 1] = nact - i0;
@@ -512,12 +605,14 @@ __device__ __forceinline__ void sweep_panel_body(const DevSys& S, const DevWalke
           for (int x = 0; x < NW; x++) {
             const int nf = cnt[2 * x];
             more |= cnt[2 * x + 1] > 0;
-            if (mine) panel_lcao(Cw, roff0 + x * cap, chi0 + (size_t)x * 5 * cap, cap, nf, phi, lane, u);
+            if (64 * wv < n)
+              panel_lcao<Lc::G, Lc::R>(Cw, roff0 + x * cap, chi0 + (size_t)x * 5 * cap, cap, nf, n - 64 * wv, part, lane, u);
           }
           if (!more) break;
           __syncthreads();
         }
       }
+      lcao_join<Lc::G, Lc::R>(part, phi);
       jastrow_share<NT, JP>(S, e, rn, pos, epos, v[0], v[1], v[2], v[3], t);
       for (int c = 0; c < 4; c++) v[4 + c] = mine ? rk * phi[c] : 0.0;
       if (t < NS) phib[t] = mine ? phi[0] : 0.0;
