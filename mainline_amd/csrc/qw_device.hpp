@@ -50,6 +50,7 @@ struct JRad {
 struct DevSys {
   int nup, ndn, ne, na, nb, nsh, ntab, nint;
   int nee, nchunk, has_pp, nsp;  // nsp = max(nup, ndn): row length of the MO cache
+  int pp_g;                      // (atom, electron) pairs a wavefront takes together (pp_pairs)
   const double* atom_pos;
   const double* atom_Z;
   const ShellDesc* shells;

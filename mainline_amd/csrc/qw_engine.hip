@@ -129,8 +129,7 @@ qw_status make_engine(SysTables T, const qw_engine_opts* opts, qw_engine** out) 
   if (const char* t = std::getenv("QW_TUNE")) e->tune_enabled = t[0] != '0';
   if (const char* v = std::getenv("QW_INV")) e->inv_rows = std::strcmp(v, "rows") == 0;
   if (const char* c = std::getenv("QW_SWEEP"))
-    for (int x : e->cands())
-      if (x == std::atoi(c)) e->tune_u = x;
+    if (e->sweep_choice_ok(std::atoi(c))) e->tune_u = std::atoi(c);
   *out = e.release();
   return QW_OK;
 }

@@ -24,6 +24,7 @@
 #include "qw_mixed.hpp"
 #include "qw_multidet.hpp"
 #include "qw_parm.hpp"
+#include "qw_pp.hpp"
 #include "qw_setup.hpp"
 #include "qw_sweep.hpp"
 
@@ -313,6 +314,8 @@ struct qw_engine {
     S.nint = T.nint;
     S.nee = (int)T.ee.size();
     S.has_pp = T.pptypes.empty() ? 0 : 1;
+    S.pp_g = 0;
+    for (const PPType& t : T.pptypes) S.pp_g = std::max(S.pp_g, pp_pairs(t.aip));
     // MO cache row: the spin's MO list (its electrons' orbitals with one determinant)
     S.nsp = std::max(T.nmo[0], T.nmo[1]);
     S.nsig = std::max(T.nup, T.ndn);
@@ -670,13 +673,15 @@ struct qw_engine {
   std::vector<int> tune_cands;
   std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> tune_ev;
   int u_default() const { return precision == QW_PREC_FP64 ? 4 : 8; }
+  // (The LDS-staged launches can be forced but are not tried: at 64 electrons of a spin and 8192
+  // walkers one takes 3.3 ms against 1.28, so trying them cost a new engine's first run 14 %.)
   const std::vector<int>& cands() {
-    if (tune_cands.empty()) {
-      if (precision == QW_PREC_FP64) tune_cands = {2, 4, 8};
-      else tune_cands = {4, 8, 16};
-      if (cl_ok) tune_cands.insert(tune_cands.end(), {104, 108, 116});
-    }
+    if (tune_cands.empty()) tune_cands = precision == QW_PREC_FP64 ? std::vector<int>{2, 4, 8} : std::vector<int>{4, 8, 16};
     return tune_cands;
+  }
+  bool sweep_choice_ok(int u) {
+    if (std::count(cands().begin(), cands().end(), u)) return true;
+    return cl_ok && (u == 104 || u == 108 || u == 116);
   }
   int pick_u() {
     if (tune_u) return tune_u;

@@ -11,7 +11,7 @@ namespace qw {
 // Dynamic LDS of k_local: positions, determinant gradients and laplacians; several determinants:
 // their weights, logs and signs; with a pseudopotential the buffers of pp_energy.
 __host__ __device__ inline size_t local_lds_bytes(const DevSys& S) {
-  return ((size_t)7 * S.ne + (S.ndet > 1 ? 5 * (size_t)S.ndet : 0) + 1 + (S.has_pp ? pp_lds_doubles(S.chunk_nf, S.nsp) : 0)) *
+  return ((size_t)7 * S.ne + (S.ndet > 1 ? 5 * (size_t)S.ndet : 0) + 1 + (S.has_pp ? pp_lds_doubles(S.pp_g, S.chunk_nf, S.nsp) : 0)) *
          sizeof(double);
 }
 

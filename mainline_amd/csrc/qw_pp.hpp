@@ -58,8 +58,9 @@ __host__ __device__ inline int pp_pairs(int aip) {
   const int g = 64 / (aip + 1);
   return g < kPPPairs ? g : kPPPairs;
 }
-__host__ __device__ inline size_t pp_lds_doubles(int chunk_nf, int nsp) {
-  return (size_t)kPPPairs * (chunk_nf | 1) + (size_t)kPPPairs * ((nsp + 2) & ~1) + 64 + (64 + kPPPairs);
+// (gmax: pp_pairs of the system's smallest quadrature, DevSys::pp_g).
+__host__ __device__ inline size_t pp_lds_doubles(int gmax, int chunk_nf, int nsp) {
+  return (size_t)gmax * (chunk_nf | 1) + (size_t)gmax * ((nsp + 2) & ~1) + 64 + (64 + kPPPairs);
 }
 
 // Jastrow value of electron e at p, terms of every other electron and atom (this lane's own e, p).
@@ -254,8 +255,8 @@ __device__ inline double pp_energy(const DevSys& S, const DevWalkers& W, const L
                                    double* lds, const double* bw, double md_den, int lane) {
   const int ne = S.ne;
   double* dl = lds;
-  double* rowl = dl + (size_t)kPPPairs * (S.chunk_nf | 1);
-  double* vx = rowl + (size_t)kPPPairs * ((S.nsp + 2) & ~1);
+  double* rowl = dl + (size_t)S.pp_g * (S.chunk_nf | 1);
+  double* vx = rowl + (size_t)S.pp_g * ((S.nsp + 2) & ~1);
   int2* list = (int2*)(vx + 64);
   double rot[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
   if (A.mode == 0) {
