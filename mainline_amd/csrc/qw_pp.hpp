@@ -8,17 +8,21 @@
 // shells near it adding chi_b D_b, and the Jastrow partners, with no sums over lanes and no
 // orbital at all.  The pair's own unmoved position is one more point (its Jastrow value).
 //
-// What bounds it: vector issue of the basis and pair terms (most of it the Jastrow partners of
-// every point).  Contracting the orbitals at every point instead, four points at a time with the
+// What bounds it: the latency of the shells' table rows and coefficients at three wavefronts per
+// SIMD (30 % of the vector issue slots are used); two shells' rows in flight together take 1.27 ms
+// against 1.58 one at a time, three and four 1.56 and 1.75 (registers), eight coefficient loads
+// instead of four 1.40.  Contracting the orbitals at every point instead, four points at a time with the
 // wave over orbitals, partners and shells in turn, held 255 registers (two waves per SIMD; now
 // 123, four) and waited on coefficient loads.  Measured: local energy of the 64-electron
-// pseudopotential molecule, 4096 walkers 4.56 -> 1.82 ms, of N2 (10 electrons, 2048 walkers)
-// 0.232 -> 0.046 ms; 500 configurations of the 64-electron molecule 1.89 -> 0.80 ms.
+// pseudopotential molecule, 4096 walkers 4.56 -> 1.27 ms, of N2 (10 electrons, 2048 walkers)
+// 0.232 -> 0.046 ms; 500 configurations of the 64-electron molecule 1.89 -> 0.62 ms.
 #pragma once
 #include "qw_jastrow.hpp"
 #include "qw_kernels.hpp"
 
 namespace qw {
+
+constexpr int kPPShells = 2;  // shells whose table rows are in flight together
 
 constexpr int kPPPairs = 8;  // pairs whose points the lanes share at most
 
@@ -192,28 +196,45 @@ __device__ inline double pp_pairs_energy(const DevSys& S, const DevWalkers& W, c
     }
     __syncthreads();
     const double* d = dl + (valid ? p : 0) * ldd;
+    // two shells at a time: their records and spline rows are all in flight before the first use
     int atom = -1;
     double x = 0, y = 0, z = 0, r = 0;
-    for (int sh = sh0; sh < sh1; sh++) {
-      const QW_CONST ShellDesc& D = shs[sh];
-      if (D.atom != atom) {
-        atom = D.atom;
-        const QW_CONST double* pa = cptr(S.atom_pos) + 3 * atom;
-        x = pt[0] - pa[0];
-        y = pt[1] - pa[1];
-        z = pt[2] - pa[2];
-        double ri;
-        dist_inv(x * x + y * y + z * z, r, ri);
+    for (int sh = sh0; sh < sh1; sh += kPPShells) {
+      double c[kPPShells][4], hx[kPPShells], xs[kPPShells][3];
+      bool act[kPPShells];
+#pragma unroll
+      for (int i = 0; i < kPPShells; i++) {
+        const bool in = sh + i < sh1;
+        const QW_CONST ShellDesc& D = shs[in ? sh + i : sh];
+        if (D.atom != atom) {
+          atom = D.atom;
+          const QW_CONST double* pa = cptr(S.atom_pos) + 3 * atom;
+          x = pt[0] - pa[0];
+          y = pt[1] - pa[1];
+          z = pt[2] - pa[2];
+          double ri;
+          dist_inv(x * x + y * y + z * z, r, ri);
+        }
+        act[i] = quad && in && r < D.rcut && r < D.objthr;
+        xs[i][0] = x;
+        xs[i][1] = y;
+        xs[i][2] = z;
+        if (act[i]) {
+          int iv = (int)(r * cptr(S.tab_inv)[D.table]);
+          iv = iv < 0 ? 0 : (iv >= S.nint ? S.nint - 1 : iv);
+          const double* cc = S.spline + ((size_t)D.table * S.nint + iv) * 4;
+          hx[i] = r - iv * cptr(S.tab_sp)[D.table];
+          for (int k = 0; k < 4; k++) c[i][k] = cc[k];
+        }
       }
-      const bool act = quad && r < D.rcut && r < D.objthr;
-      if (!wave_any(act)) continue;
-      if (act) {
-        int iv = (int)(r * cptr(S.tab_inv)[D.table]);
-        iv = iv < 0 ? 0 : (iv >= S.nint ? S.nint - 1 : iv);
-        const double* c = S.spline + ((size_t)D.table * S.nint + iv) * 4;
-        const double h = r - iv * cptr(S.tab_sp)[D.table];
-        const double f = c[0] + h * (c[1] + h * (c[2] + h * c[3]));
-        R += shell_dot<!JP>(D.sym, f, x, y, z, d + (D.f0 - f0));
+#pragma unroll
+      for (int i = 0; i < kPPShells; i++) {
+        if (!wave_any(act[i])) continue;
+        const QW_CONST ShellDesc& D = shs[sh + i];
+        if (act[i]) {
+          const double f = c[i][0] + hx[i] * (c[i][1] + hx[i] * (c[i][2] + hx[i] * c[i][3]));
+          R += shell_dot<!JP>(D.sym, f, xs[i][0], xs[i][1], xs[i][2], d + (D.f0 - f0));
+        }
       }
     }
   }
