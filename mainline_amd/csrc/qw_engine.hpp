@@ -650,7 +650,7 @@ struct qw_engine {
       const int u = pick_u();
       tuned_launch([&] {
         if (depth == 1) launch_sweep_f64(S, W, A, u, stream);
-        else launch_sweep_vmc64(S, W, A, ns, u, stream);
+        else launch_sweep_vmc64_big(S, W, A, stream);  // (up to 64 electrons of a spin: vmc_sweeps)
       });
       return;
     }
@@ -940,15 +940,24 @@ struct qw_engine {
     step++;
     R.fbi = std::max(1, m.feedback_interval);
   }
+  // nsw sweeps of both spins in one launch (one determinant, FP64, up to 64 electrons of a spin)
+  void vmc_sweeps(double tau, int nsw) {
+    const SweepArgs A{0, 0, 0, tau, seed, step, 0u, 0, 0, dstep};
+    const int u = pick_u();
+    tuned_launch([&] { launch_sweeps_vmc64(S, W, A, nsw, ns, u, stream); });
+  }
   // one VMC step: ndecorr sweeps of both spin channels, then the local energy
   void vmc_step(const qw_method_desc& m, RunState& R) {
     const int nsw = std::max(1, m.ndecorr);
-    for (int sw = 0; sw < nsw; sw++) {
-      for (int s = 0; s < 2; s++) {
-        int n = s ? T.ndn : T.nup;
-        if (n == 0) continue;
-        run_sweep(s, 0, n, m.timestep, (unsigned)sw, 2, 0, sw == nsw - 1);
-      }
+    if (precision == QW_PREC_FP64 && !md && !big) {
+      vmc_sweeps(m.timestep, nsw);
+    } else {
+      for (int sw = 0; sw < nsw; sw++)
+        for (int s = 0; s < 2; s++) {
+          int n = s ? T.ndn : T.nup;
+          if (n == 0) continue;
+          run_sweep(s, 0, n, m.timestep, (unsigned)sw, 2, 0, sw == nsw - 1);
+        }
     }
     R.moves += (long long)nw * S.ne * (nsw - 1);  // run_advance counts one sweep per step
     R.A.mode = 1;

@@ -2,7 +2,7 @@
 //
 //   k_inv<NS>    pivoted inversion, log|det|, sign and transposed inverse per walker and spin;
 //                src/program_utils/MatrixAlgebrac.cpp:108-224,316-421
-//   k_sweep<NS,U> VMC moves of one spin channel (delayed rejection): drift, proposal, ratio,
+//   k_sweeps<NS,U> VMC moves of a step (delayed rejection): drift, proposal, ratio,
 //                Jastrow, acceptance, Sherman-Morrison update with the inverse held in registers;
 //                src/method/Split_sample.cpp:302-540, src/program_utils/MatrixAlgebrac.cpp:766-838
 //                (DMC moves: qw_panel.hpp; the mixed path: qw_panel_mx.hpp, qw_big_mx.hpp and
@@ -734,10 +734,25 @@ __device__ __forceinline__ void sweep_fp64_body(const DevSys& S, const DevWalker
   }
 }
 
+// The moves of `nsw` sweeps of both spins, one walker per block.  The sweeps of a walker depend only
+// on each other, so one launch takes them all.  What bounds it: the latency of a move's serial chain
+// (small systems leave most SIMDs one wavefront).  Measured, a step of two sweeps: 256 walkers with 2
+// electrons of a spin 179 us in four launches, 150 in one.
 template <int NS, int DEPTH, int U>
-__global__ __launch_bounds__(64, 2) void k_sweep(DevSys S, DevWalkers W, SweepArgs A) {
+__global__ __launch_bounds__(64, 2) void k_sweeps(DevSys S, DevWalkers W, SweepArgs A, int nsw) {
   extern __shared__ double lds[];
-  sweep_fp64_body<NS, DEPTH, U, 1>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, 0, (char*)lds);
+  for (int i = 0; i < 2 * nsw; i++) {
+    A.s = i & 1;
+    A.sweep = (unsigned)(i >> 1);
+    A.k1 = A.s ? S.ndn : S.nup;
+    A.dets = A.sweep + 1 == (unsigned)nsw;
+    if (A.k1 == 0) continue;
+    if (i) {  // the state the last sweep left in device memory, and its LDS
+      __threadfence_block();
+      __syncthreads();
+    }
+    sweep_fp64_body<NS, DEPTH, U, 1>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, 0, (char*)lds);
+  }
 }
 
 // ---------------------------------------------------------------- k_local
