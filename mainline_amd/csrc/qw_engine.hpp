@@ -639,10 +639,13 @@ struct qw_engine {
   void run_sweep(int s, int k0, int k1, double tau, unsigned sweep, int depth, int restrict_nodes, int dets) {
     SweepArgs A{s, k0, k1, tau, seed, step, sweep, restrict_nodes, dets, dstep};
     if (md) {
-      const size_t lds = sweep_md_lds_bytes(S.ne, S.ndet, S.nsig, S.nsp, S.chunk_nf, depth);
+      const size_t with = sweep_md_lds_bytes(S, depth, true);
+      const bool res = with <= kMdResident;
+      const size_t lds = res ? with : sweep_md_lds_bytes(S, depth, false);
       launch("k_sweep", [&] {
-        if (depth == 1) hipLaunchKernelGGL(k_sweep_md<1>, dim3(nw), dim3(64), lds, stream, S, W, A);
-        else hipLaunchKernelGGL(k_sweep_md<2>, dim3(nw), dim3(64), lds, stream, S, W, A);
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nw), dim3(64), lds, stream, S, W, A); };
+        if (depth == 1) res ? go(k_sweep_md<1, true>) : go(k_sweep_md<1, false>);
+        else res ? go(k_sweep_md<2, true>) : go(k_sweep_md<2, false>);
       });
       return;
     }

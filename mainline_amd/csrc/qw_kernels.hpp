@@ -864,19 +864,18 @@ __device__ inline double md_weights(const DevSys& S, const double* ld, const dou
   return wsum(part);
 }
 
-// out[c] = sum_d b_d sum_j inv_d(k, j) v[c][occ_d(j)] / den for NC components (v: LDS rows of
-// length ldv indexed by the spin's MO list), lanes over determinants.
-template <int NC>
-__device__ inline void md_contract(const DevSys& S, const double* invw, int s, int k, const double* v, int ldv,
-                                   const double* b, double den, double out[NC], int lane) {
-  const int nd = S.ndet, n = s ? S.ndn : S.nup, ns = S.nsig;
-  const QW_CONST int* oc = cptr(S.occ) + (size_t)s * nd * ns;
+// out[c] = sum_d b_d sum_j inv_d(k, j) v[c][occ_d(j)] / den for NC components (v: rows of length ldv
+// indexed by the spin's MO list), lanes over determinants.  inv, oc: the spin's inverses and
+// occupations, determinant by determinant (device memory or LDS).
+template <int NC, typename OC>
+__device__ inline void md_contract_at(int nd, int n, int ns, const double* inv, OC oc, int k, const double* v, int ldv,
+                                      const double* b, double den, double out[NC], int lane) {
   double part[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) part[c] = 0;
   for (int d = lane; d < nd; d += kWave) {
-    const double* row = invw + (((size_t)s * nd + d) * ns + k) * ns;
-    const QW_CONST int* o = oc + (size_t)d * ns;
+    const double* row = inv + ((size_t)d * ns + k) * ns;
+    const OC o = oc + (size_t)d * ns;
     double t[NC];
 #pragma unroll
     for (int c = 0; c < NC; c++) t[c] = 0;
@@ -891,6 +890,14 @@ __device__ inline void md_contract(const DevSys& S, const double* invw, int s, i
   }
 #pragma unroll
   for (int c = 0; c < NC; c++) out[c] = wsum(part[c]) / den;
+}
+// The same for spin s of the walker's inverses invw ([2][ndet][ns][ns]).
+template <int NC>
+__device__ inline void md_contract(const DevSys& S, const double* invw, int s, int k, const double* v, int ldv,
+                                   const double* b, double den, double out[NC], int lane) {
+  const int nd = S.ndet, n = s ? S.ndn : S.nup, ns = S.nsig;
+  md_contract_at<NC>(nd, n, ns, invw + (size_t)s * nd * ns * ns, cptr(S.occ) + (size_t)s * nd * ns, k, v, ldv, b, den, out,
+                     lane);
 }
 
 // ---------------------------------------------------------------- k_tmove

@@ -97,37 +97,60 @@ static __global__ __launch_bounds__(64) void k_inv_md(DevSys S, DevWalkers W, in
 
 inline size_t inv_md_lds_bytes(int nsig) { return (size_t)2 * nsig * nsig * sizeof(double) + 16; }
 
-// LDS of k_sweep_md.
-inline size_t sweep_md_lds_bytes(int ne, int ndet, int nsig, int nsp, int chunk_nf, int depth) {
-  return ((size_t)3 * ne + 4 * (size_t)ndet + ndet + 5 * (size_t)nsp + (size_t)ndet * nsig + 5 * (size_t)chunk_nf) *
-             sizeof(double) +
-         (size_t)chunk_nf * sizeof(int) + sweep_rand_bytes(kMdMaxSpin, depth) + 64;
+// LDS of k_sweep_md; RES: with the spin's inverses and occupations.
+inline size_t sweep_md_lds_bytes(const DevSys& S, int depth, bool res) {
+  const size_t nd = S.ndet, ns = S.nsig;
+  return ((sys_lds_bytes(S.na, S.nsh, S.ntab) + 15) & ~(size_t)15) +
+         ((size_t)3 * S.ne + 5 * nd + 5 * (size_t)S.nsp + nd * ns + 5 * (size_t)kCapF64) * sizeof(double) +
+         sweep_rand_bytes(kMdMaxSpin, depth) + (size_t)kCapF64 * sizeof(int) +
+         (res ? nd * ns * ns * sizeof(double) + nd * ns * sizeof(int) : 0) + 16;
 }
+// The inverses stay in LDS for a launch while four walkers of a compute unit fit (one per SIMD).
+constexpr size_t kMdResident = 40960;
 
-template <int DEPTH>
+// What bounds it: the latency of a move's serial chain, one wavefront per walker (1000 walkers leave
+// a SIMD one).  With the system tables, the inverses and the occupations in LDS its gathers over
+// determinants and orbitals no longer wait on device memory: 1000 walkers of N2 with 28
+// determinants, a spin's moves with delayed rejection, 164 -> 142 us.
+template <int DEPTH, bool RES>
 __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepArgs A) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x, w = blockIdx.x;
   if (w >= W.nw) return;
   const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
   const int nd = S.ndet, ns = S.nsig, nm = S.nmo[s];
-  double* pos = lds;
+  SysLds V;
+  double* pos = (double*)sys_lds_carve(S, (char*)lds, V);
   double* ld = pos + 3 * ne;  // [2][nd]
   double* sg = ld + 2 * nd;   // [2][nd]
   double* b = sg + 2 * nd;    // [nd]
-  double* phin = b + nd;      // [5][nsp] MO values at the trial point
+  double* phin = b + nd;      // [5][nsp] MO values at the trial point (before: the old point's gradient)
   double* rowk = phin + 5 * nsp;  // [nd][ns] row k of every inverse before an update
   double* rnd = rowk + (size_t)nd * ns;
   double* chi = rnd + sweep_rand_bytes(kMdMaxSpin, DEPTH) / sizeof(double);
-  int* flist = (int*)(chi + 5 * S.chunk_nf);
+  double* linv = chi + 5 * kCapF64;  // RES: [nd][ns][ns]
+  int* roff = (int*)(linv + (RES ? (size_t)nd * ns * ns : 0));
+  int* locc = roff + kCapF64;  // RES: [nd][ns]
+  stage_sys(S, V, lane);
   for (int i = lane; i < 3 * ne; i += kWave) pos[i] = W.pos[(size_t)w * ne * 3 + i];
   for (int i = lane; i < 2 * nd; i += kWave) {
     ld[i] = W.ldd[(size_t)w * 2 * nd + i];
     sg[i] = W.sgd[(size_t)w * 2 * nd + i];
   }
   sweep_randoms<DEPTH>(A, (unsigned)w, off, rnd, lane);
-  double* invw = W.invd + (size_t)w * 2 * nd * ns * ns;
-  const QW_CONST int* oc = cptr(S.occ) + (size_t)s * nd * ns;
+  double* invg = W.invd + ((size_t)w * 2 + s) * nd * ns * ns;
+  const QW_CONST int* ocg = cptr(S.occ) + (size_t)s * nd * ns;
+  if constexpr (RES) {
+    for (int i = lane; i < nd * ns * ns; i += kWave) linv[i] = invg[i];
+    for (int i = lane; i < nd * ns; i += kWave) locc[i] = ocg[i];
+  }
+  double* inv;
+  if constexpr (RES) inv = linv;
+  else inv = invg;
+  auto contract = [&](auto nc, int k, const double* v, double den, double* out) {
+    if constexpr (RES) md_contract_at<decltype(nc)::value>(nd, n, ns, linv, (const int*)locc, k, v, nsp, b, den, out, lane);
+    else md_contract_at<decltype(nc)::value>(nd, n, ns, invg, ocg, k, v, nsp, b, den, out, lane);
+  };
   double* mog = W.mo + (size_t)w * ne * 5 * nsp;
   const double tau = A.tau, stau = sqrt(tau);
   int nacc = 0;
@@ -136,12 +159,14 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
     const int e = off + k;
     double r0[3] = {pos[3 * e], pos[3 * e + 1], pos[3 * e + 2]};
     double l0, s0;
+    if (lane < nm)
+      for (int c = 1; c < 4; c++) phin[c * nsp + lane] = mog[((size_t)e * 5 + c) * nsp + lane];
     const double den = md_weights(S, ld, sg, b, l0, s0, lane);
     __syncthreads();
     // drift at the old position: determinant part from the cached MO row, Jastrow part fresh
     double gd[3], gj0[3], d0[3];
-    md_contract<3>(S, invw, s, k, mog + ((size_t)e * 5 + 1) * nsp, nsp, b, den, gd, lane);
-    const double u0 = jastrow_e(S, e, r0, pos, gj0, nullptr, lane);
+    contract(std::integral_constant<int, 3>(), k, phin + nsp, den, gd);
+    const double u0 = jastrow_e(S, e, r0, pos, gj0, nullptr, lane, V.epos, 4);
     for (int d = 0; d < 3; d++) d0[d] = gd[d] + gj0[d];
     double phi[5];
     double r1[3], d1[3], ln1 = 0;
@@ -153,16 +178,15 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
       double dr[3], rn[3], dn[3];
       lim_drift(d0, t, dr);
       for (int d = 0; d < 3; d++) rn[d] = r0[d] + (rq[d] * st + dr[d]);
-      lcao_lap_n(S, s, nm, rn, chi, flist, phi, lane);
-      __syncthreads();
+      mo_lap_point<double, double, 8>(S, V, S.spline, S.C[s], nm, rn, chi, roff, kCapF64, phi, lane);
       if (lane < nm)
         for (int c = 0; c < 5; c++) phin[c * nsp + lane] = phi[c];
       __syncthreads();
       double tt[4];
-      md_contract<4>(S, invw, s, k, phin, nsp, b, den, tt, lane);
+      contract(std::integral_constant<int, 4>(), k, phin, den, tt);
       const double t0 = tt[0];
       double gj[3];
-      const double un = jastrow_e(S, e, rn, pos, gj, nullptr, lane);
+      const double un = jastrow_e(S, e, rn, pos, gj, nullptr, lane, V.epos, 4);
       dn[0] = tt[1] / t0 + gj[0];
       dn[1] = tt[2] / t0 + gj[1];
       dn[2] = tt[3] / t0 + gj[2];
@@ -201,17 +225,19 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
       // every determinant: Sherman-Morrison for the replaced row k with its own orbitals
       for (int i = lane; i < nd * n; i += kWave) {
         const int d = i / n, j = i % n;
-        rowk[d * ns + j] = invw[(((size_t)s * nd + d) * ns + k) * ns + j];
+        rowk[d * ns + j] = inv[((size_t)d * ns + k) * ns + j];
       }
       __syncthreads();
       for (int i = lane; i < nd * n; i += kWave) {
         const int d = i / n, r = i % n;
-        const QW_CONST int* o = oc + (size_t)d * ns;
         const double* rk = rowk + d * ns;
         double Rd = 0, tr = 0;
-        double* row = invw + (((size_t)s * nd + d) * ns + r) * ns;
+        double* row = inv + ((size_t)d * ns + r) * ns;
         for (int j = 0; j < n; j++) {
-          const double v = phin[o[j]];
+          int m;
+          if constexpr (RES) m = locc[d * ns + j];
+          else m = ocg[(size_t)d * ns + j];
+          const double v = phin[m];
           Rd += rk[j] * v;
           tr += row[j] * v;
         }
@@ -232,6 +258,8 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
     }
     __syncthreads();
   }
+  if constexpr (RES)
+    for (int i = lane; i < nd * ns * ns; i += kWave) invg[i] = linv[i];
   for (int i = lane; i < 3 * ne; i += kWave) W.pos[(size_t)w * ne * 3 + i] = pos[i];
   for (int i = lane; i < 2 * nd; i += kWave) {
     W.ldd[(size_t)w * 2 * nd + i] = ld[i];
