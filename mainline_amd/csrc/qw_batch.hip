@@ -92,11 +92,12 @@ __global__ __launch_bounds__(1024) void k_branch_batch(const BatchSlot* __restri
               (int)threadIdx.x, L);
 }
 
-// The branching copies of the slots that branched (one block per pair slot of each).
+// The branching copies of the slots that branched (copy_slices blocks per pair slot of each).
 __global__ __launch_bounds__(256) void k_copy_batch(const BatchSlot* __restrict__ slots, int nslot, int np) {
   const QW_CONST BatchSlot* sl = cptr(slots);
   int i = 0, b0 = 0;
-  while (i + 1 < nslot && (int)blockIdx.x >= b0 + sl[i].W.nw / 2 + 1) b0 += sl[i++].W.nw / 2 + 1;
+  auto nb = [&](int q) { return (sl[q].W.nw / 2 + 1) * copy_slices(sl[q].S.ne, sl[q].S.nsp); };
+  while (i + 1 < nslot && (int)blockIdx.x >= b0 + nb(i)) b0 += nb(i++);
   const QW_CONST BatchSlot& B = sl[i];
   if (!np && B.branch_np <= 0) return;
   copy_body(gref(B.S), gref(B.W), B.ctl, B.psrc, B.pdst, (int)blockIdx.x - b0, (int)threadIdx.x);
@@ -411,7 +412,7 @@ struct qw_batch {
   // branching: every slot over np steps, or (np = 0) the slots whose branch_np is set
   void branch(int np) {
     unsigned ncp = 0;
-    for (auto& B : slots) ncp += (unsigned)(B.W.nw / 2 + 1);
+    for (auto& B : slots) ncp += (unsigned)((B.W.nw / 2 + 1) * copy_slices(B.S.ne, B.S.nsp));
     launch(3, [&] {
       hipLaunchKernelGGL(k_branch_batch, dim3(nslot()), dim3(1024), 0, stream, d_slots, nslot(), np);
       hipLaunchKernelGGL(k_copy_batch, dim3(ncp), dim3(256), 0, stream, d_slots, nslot(), np);

@@ -842,7 +842,7 @@ struct qw_engine {
                          seed, 0u, (const unsigned*)dstep);
     });
     launch("k_copy", [&] {
-      hipLaunchKernelGGL(k_copy, dim3(nw / 2 + 1), dim3(256), 0, stream, S, W, (const DmcCtl*)dctl,
+      hipLaunchKernelGGL(k_copy, dim3((unsigned)(nw / 2 + 1) * copy_slices(S.ne, S.nsp)), dim3(256), 0, stream, S, W, (const DmcCtl*)dctl,
                          (const int*)psrc, (const int*)pdst);
     });
   }

@@ -1320,30 +1320,49 @@ static __global__ __launch_bounds__(1024) void k_branch(DevWalkers W, DmcCtl* ct
   branch_body(W, ctl, keys, vals, pair_src, pair_dst, nmoves, do_branch, seed, event_host, eventp, (int)threadIdx.x, L);
 }
 
-// Copies the state of walker pair_src[p] into walker pair_dst[p] for p < ctl->npairs.
+// Blocks that share a pair's copy: one per 16384 values of the MO cache, at most 16 (a block that
+// finds no pair ends at once).  What bounds it: latency up to 128 electrons, device memory above.  One
+// block per pair with one value in flight per thread took 1.77 ms for 1024 walkers of 512 electrons,
+// now 0.63, and 79 us for 8192 of 128 on the mixed path, now 17.
+__host__ __device__ inline int copy_slices(int ne, int nsp) {
+  const int n = (ne * 5 * nsp + 16383) / 16384;
+  return n < 16 ? n : 16;
+}
+// n values by threads t, t + stride, ..., four in flight.
+template <typename T>
+__device__ inline void copy_values(T* dst, const T* src, size_t n, size_t t, size_t stride) {
+  size_t i = t;
+  for (; i + 3 * stride < n; i += 4 * stride) {
+    const T a = src[i], b = src[i + stride], c = src[i + 2 * stride], d = src[i + 3 * stride];
+    dst[i] = a;
+    dst[i + stride] = b;
+    dst[i + 2 * stride] = c;
+    dst[i + 3 * stride] = d;
+  }
+  for (; i < n; i += stride) dst[i] = src[i];
+}
+// Copies the state of walker pair_src[p] into walker pair_dst[p] for p < ctl->npairs; block `blk` is
+// slice blk % copy_slices of pair blk / copy_slices.
 __device__ __forceinline__ void copy_body(const DevSys& S, const DevWalkers& W, const DmcCtl* ctl,
-                                          const int* pair_src, const int* pair_dst, int p, int t) {
+                                          const int* pair_src, const int* pair_dst, int blk, int t) {
+  const int ny = copy_slices(S.ne, S.nsp), p = blk / ny, y = blk % ny;
   if (p >= ctl->npairs) return;
   const int src = pair_src[p], dst = pair_dst[p];
   const int ne = S.ne, nsp = S.nsp;
   const size_t npos = (size_t)ne * 3, ninv = (size_t)2 * nsp * nsp, nmo = (size_t)ne * 5 * nsp;
-  for (size_t i = t; i < npos; i += 256) W.pos[dst * npos + i] = W.pos[src * npos + i];
-  if (W.inv)
-    for (size_t i = t; i < ninv; i += 256) W.inv[dst * ninv + i] = W.inv[src * ninv + i];
-  if (W.invf)
-    for (size_t i = t; i < ninv; i += 256) W.invf[dst * ninv + i] = W.invf[src * ninv + i];
-  if (W.mo)
-    for (size_t i = t; i < nmo; i += 256) W.mo[dst * nmo + i] = W.mo[src * nmo + i];
-  if (W.mof)
-    for (size_t i = t; i < nmo; i += 256) W.mof[dst * nmo + i] = W.mof[src * nmo + i];
+  const size_t t0 = (size_t)256 * y + t, st = (size_t)256 * ny;
+  copy_values(W.pos + dst * npos, W.pos + src * npos, npos, t0, st);
+  if (W.inv) copy_values(W.inv + dst * ninv, W.inv + src * ninv, ninv, t0, st);
+  if (W.invf) copy_values(W.invf + dst * ninv, W.invf + src * ninv, ninv, t0, st);
+  if (W.mo) copy_values(W.mo + dst * nmo, W.mo + src * nmo, nmo, t0, st);
+  if (W.mof) copy_values(W.mof + dst * nmo, W.mof + src * nmo, nmo, t0, st);
   if (W.invd) {
     const size_t nd = (size_t)2 * S.ndet * S.nsig * S.nsig, nl = (size_t)2 * S.ndet;
-    for (size_t i = t; i < nd; i += 256) W.invd[dst * nd + i] = W.invd[src * nd + i];
-    for (size_t i = t; i < nl; i += 256) {
-      W.ldd[dst * nl + i] = W.ldd[src * nl + i];
-      W.sgd[dst * nl + i] = W.sgd[src * nl + i];
-    }
+    copy_values(W.invd + dst * nd, W.invd + src * nd, nd, t0, st);
+    copy_values(W.ldd + dst * nl, W.ldd + src * nl, nl, t0, st);
+    copy_values(W.sgd + dst * nl, W.sgd + src * nl, nl, t0, st);
   }
+  if (y) return;
   if (t < 2) {
     W.logdet[2 * dst + t] = W.logdet[2 * src + t];
     W.sgn[2 * dst + t] = W.sgn[2 * src + t];
