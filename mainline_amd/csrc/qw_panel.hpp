@@ -482,7 +482,8 @@ __device__ inline void panel_sync() {
     __syncthreads();
 }
 // The moves of walker w's spin A.s by NW wavefronts (t: thread of the walker).  sh: the block's
-// shared LDS tables, own: the walker's region.  u: coefficient loads in flight in the LCAO.
+// shared LDS tables, own: the walker's region.  u: half the coefficient loads in flight in the
+// LCAO.
 template <int NW, int NS, bool JP>
 __device__ __forceinline__ void sweep_panel_body(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int w, int t,
                                                  char* sh, char* own, int u) {

@@ -5,8 +5,8 @@
 
 namespace qw {
 
-// The DMC moves A of every walker in FP64 (up to 256 electrons of a spin); u: coefficient loads
-// in flight in the LCAO (2, 4 or 8; every choice gives the same results).
+// The DMC moves A of every walker in FP64 (up to 256 electrons of a spin); u: coefficient loads in
+// flight in the LCAO, halved (2, 4 or 8; every choice gives the same results).
 void launch_sweep_f64(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st);
 // The VMC moves in FP64: nsw sweeps of both spins (A: their common arguments) up to 64 electrons of
 // a spin (ns: register tile of the inverse), and one spin's sweep above.
