@@ -133,7 +133,9 @@ __device__ __forceinline__ void sweep_mxb_body(const DevSys& S, const MixedTable
   double* tabs = epos + 3 * S.na;
   double* draw = (double*)(base + lds_round16((size_t)(3 * ne + 6 * S.na + 2 * S.ntab) * 8));  // [np][DEPTH][4]
   float* prow = (float*)(draw + kBigPanel * 4 * DEPTH);
-  float* ph = prow + kBigPanel * ldp;  // [4][64 NW], over the lists
+  // [4][64 NW], over the lists: every wavefront reads the values of a stage, so a block barrier lies
+  // between those reads and the next stage's (or move's) lists
+  float* ph = prow + kBigPanel * ldp;
   int2* list0 = (int2*)ph;
   float* chi0 = (float*)((char*)ph + big_list_bytes(S.nsh, NW));
   int* roff0 = (int*)(chi0 + (size_t)NB * 5 * cap);
@@ -209,6 +211,7 @@ __device__ __forceinline__ void sweep_mxb_body(const DevSys& S, const MixedTable
     bool accepted = false;
     double acc_first = 0, g2first = 0;
     for (int dep = 1; dep <= DEPTH && !accepted; dep++) {
+      if (dep > 1) __syncthreads();  // the first stage's values are read (accepted is the block's)
       const double tt = dep == 1 ? tau : tau * 0.5, st = dep == 1 ? stau : sqrt(tau * 0.5);
       double dr[3], rn[3], dn[3];
       const double* dw = draw + 4 * ((k - A.k0) * DEPTH + dep - 1);
