@@ -103,10 +103,15 @@ std::vector<JRad<R>> jrad_table(const std::vector<JObj>& objs) {
 }
 
 // Whether the Jastrow has the form DevSys::usual names (objects of one e-i type: o0[t]..o0[t+1]).
+// Its FP64 pair terms divide by the product of all the denominators 1 + beta z (1 + gamma p) of a
+// pair.  z and p are positive, so a denominator can vanish only with a negative beta (gamma), and in
+// use only beyond its own object's cutoff: there the other object must not be in use still (its
+// terms would become NaN).
 inline bool usual_jastrow(const std::vector<JObj>& ee, const std::vector<JObj>& eit, const std::vector<int>& o0) {
   if (ee.size() != 2 || ee[0].kind != 0 || ee[1].kind != 1 || ee[1].nf > 4) return false;
   for (int i = 0; i < ee[1].nf; i++)
-    if (ee[1].cl[i] != ee[1].cu[i]) return false;
+    if (ee[1].cl[i] != ee[1].cu[i] || (ee[1].beta[i] < 0 && ee[1].rcut < ee[0].rcut)) return false;
+  if (ee[0].gamma < 0 && ee[0].rcut < ee[1].rcut) return false;
   for (size_t t = 0; t + 1 < o0.size(); t++)
     if (o0[t + 1] - o0[t] != 1 || eit[o0[t]].kind != 1 || eit[o0[t]].nf > 4) return false;
   return o0.size() > 1;

@@ -2,7 +2,8 @@
 // up to four functions between electrons, one such POLYPADE object per atom type (the formulas of
 // CuspEval and PolyEval).  Functions beyond an object's count have zero coefficients.  All the
 // denominators of a pair share one reciprocal (1/a and 1/b are b/(ab) and a/(ab)): a double
-// reciprocal costs a quarter-rate estimate and four multiply-adds, and a pair has five.
+// reciprocal costs a quarter-rate estimate and four multiply-adds, and a pair has five.  None of them
+// vanishes where another object is inside its cutoff (the rule that sets DevSys::usual).
 // GRAD: add (d/dr)/r to gf; LAP: add the laplacian to l.
 #pragma once
 #include "qw_device.hpp"
