@@ -64,12 +64,6 @@ inline double cutoff_squared(double rc) {
   return x;
 }
 
-inline int pick_ns(int n) {
-  int ns = 4;
-  while (ns < n) ns <<= 1;
-  return ns;
-}
-
 // Device forms of the Jastrow radial objects (constants folded, see JRad).
 template <typename R>
 std::vector<JRad<R>> jrad_table(const std::vector<JObj>& objs) {
@@ -644,13 +638,13 @@ struct qw_engine {
   void run_sweep(int s, int k0, int k1, double tau, unsigned sweep, int depth, int restrict_nodes, int dets) {
     SweepArgs A{s, k0, k1, tau, seed, step, sweep, restrict_nodes, dets, dstep};
     if (md) {
-      const size_t with = sweep_md_lds_bytes(S, depth, true);
-      const bool res = with <= kMdResident;
-      const size_t lds = res ? with : sweep_md_lds_bytes(S, depth, false);
+      const bool sys = sweep_md_lds_bytes(S, depth, false, true) <= kLdsMax;
+      const bool res = sys && sweep_md_lds_bytes(S, depth, true, true) <= kMdResident;
+      const size_t lds = sweep_md_lds_bytes(S, depth, res, sys);
       launch("k_sweep", [&] {
         auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nw), dim3(64), lds, stream, S, W, A); };
-        if (depth == 1) res ? go(k_sweep_md<1, true>) : go(k_sweep_md<1, false>);
-        else res ? go(k_sweep_md<2, true>) : go(k_sweep_md<2, false>);
+        if (depth == 1) res ? go(k_sweep_md<1, true, true>) : sys ? go(k_sweep_md<1, false, true>) : go(k_sweep_md<1, false, false>);
+        else res ? go(k_sweep_md<2, true, true>) : sys ? go(k_sweep_md<2, false, true>) : go(k_sweep_md<2, false, false>);
       });
       return;
     }

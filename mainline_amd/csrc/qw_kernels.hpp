@@ -565,6 +565,13 @@ __device__ inline void write_det_parts(const DevSys& S, const DevWalkers& W, int
   o[3] = t[3];
 }
 
+// Size class (register tile) of up to 64 electrons of a spin.
+inline int pick_ns(int n) {
+  int ns = 4;
+  while (ns < n) ns <<= 1;
+  return ns;
+}
+
 // Basis functions per LDS tile batch in the FP64 sweep.
 constexpr int kCapF64 = 128;
 

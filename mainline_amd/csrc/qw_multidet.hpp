@@ -97,12 +97,12 @@ static __global__ __launch_bounds__(64) void k_inv_md(DevSys S, DevWalkers W, in
 
 inline size_t inv_md_lds_bytes(int nsig) { return (size_t)2 * nsig * nsig * sizeof(double) + 16; }
 
-// LDS of k_sweep_md; RES: with the spin's inverses and occupations.
-inline size_t sweep_md_lds_bytes(const DevSys& S, int depth, bool res) {
-  const size_t nd = S.ndet, ns = S.nsig;
-  return ((sys_lds_bytes(S.na, S.nsh, S.ntab) + 15) & ~(size_t)15) +
-         ((size_t)3 * S.ne + 5 * nd + 5 * (size_t)S.nsp + nd * ns + 5 * (size_t)kCapF64) * sizeof(double) +
-         sweep_rand_bytes(kMdMaxSpin, depth) + (size_t)kCapF64 * sizeof(int) +
+// LDS of k_sweep_md; RES: with the spin's inverses and occupations; SYS: with the system tables.
+inline size_t sweep_md_lds_bytes(const DevSys& S, int depth, bool res, bool sys) {
+  const size_t nd = S.ndet, ns = S.nsig, cap = sys ? kCapF64 : S.chunk_nf;
+  return (sys ? (sys_lds_bytes(S.na, S.nsh, S.ntab) + 15) & ~(size_t)15 : 0) +
+         ((size_t)3 * S.ne + 5 * nd + 5 * (size_t)S.nsp + nd * ns + 5 * cap) * sizeof(double) +
+         sweep_rand_bytes(kMdMaxSpin, depth) + cap * sizeof(int) +
          (res ? nd * ns * ns * sizeof(double) + nd * ns * sizeof(int) : 0) + 16;
 }
 // The inverses stay in LDS for a launch while four walkers of a compute unit fit (one per SIMD).
@@ -112,15 +112,20 @@ constexpr size_t kMdResident = 40960;
 // a SIMD one).  With the system tables, the inverses and the occupations in LDS its gathers over
 // determinants and orbitals no longer wait on device memory: 1000 walkers of N2 with 28
 // determinants, a spin's moves with delayed rejection, 164 -> 142 us.
-template <int DEPTH, bool RES>
+// SYS = false: the tables of thousands of shells stay in device memory, the basis goes shell chunk by
+// shell chunk.
+template <int DEPTH, bool RES, bool SYS>
 __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepArgs A) {
   extern __shared__ double lds[];
   const int lane = threadIdx.x, w = blockIdx.x;
   if (w >= W.nw) return;
   const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
   const int nd = S.ndet, ns = S.nsig, nm = S.nmo[s];
+  static_assert(SYS || !RES, "resident inverses come with the system tables");
+  const int cap = SYS ? kCapF64 : S.chunk_nf;
   SysLds V;
-  double* pos = (double*)sys_lds_carve(S, (char*)lds, V);
+  double* pos = lds;
+  if constexpr (SYS) pos = (double*)sys_lds_carve(S, (char*)lds, V);
   double* ld = pos + 3 * ne;  // [2][nd]
   double* sg = ld + 2 * nd;   // [2][nd]
   double* b = sg + 2 * nd;    // [nd]
@@ -128,10 +133,10 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
   double* rowk = phin + 5 * nsp;  // [nd][ns] row k of every inverse before an update
   double* rnd = rowk + (size_t)nd * ns;
   double* chi = rnd + sweep_rand_bytes(kMdMaxSpin, DEPTH) / sizeof(double);
-  double* linv = chi + 5 * kCapF64;  // RES: [nd][ns][ns]
+  double* linv = chi + 5 * cap;  // RES: [nd][ns][ns]
   int* roff = (int*)(linv + (RES ? (size_t)nd * ns * ns : 0));
-  int* locc = roff + kCapF64;  // RES: [nd][ns]
-  stage_sys(S, V, lane);
+  int* locc = roff + cap;  // RES: [nd][ns]
+  if constexpr (SYS) stage_sys(S, V, lane);
   for (int i = lane; i < 3 * ne; i += kWave) pos[i] = W.pos[(size_t)w * ne * 3 + i];
   for (int i = lane; i < 2 * nd; i += kWave) {
     ld[i] = W.ldd[(size_t)w * 2 * nd + i];
@@ -151,6 +156,10 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
     if constexpr (RES) md_contract_at<decltype(nc)::value>(nd, n, ns, linv, (const int*)locc, k, v, nsp, b, den, out, lane);
     else md_contract_at<decltype(nc)::value>(nd, n, ns, invg, ocg, k, v, nsp, b, den, out, lane);
   };
+  auto jastrow = [&](int e, const double* p, double* g) {
+    if constexpr (SYS) return jastrow_e(S, e, p, pos, g, nullptr, lane, V.epos, 4);
+    else return jastrow_e(S, e, p, pos, g, nullptr, lane, S.eit_pos, 3);
+  };
   double* mog = W.mo + (size_t)w * ne * 5 * nsp;
   const double tau = A.tau, stau = sqrt(tau);
   int nacc = 0;
@@ -166,7 +175,7 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
     // drift at the old position: determinant part from the cached MO row, Jastrow part fresh
     double gd[3], gj0[3], d0[3];
     contract(std::integral_constant<int, 3>(), k, phin + nsp, den, gd);
-    const double u0 = jastrow_e(S, e, r0, pos, gj0, nullptr, lane, V.epos, 4);
+    const double u0 = jastrow(e, r0, gj0);
     for (int d = 0; d < 3; d++) d0[d] = gd[d] + gj0[d];
     double phi[5];
     double r1[3], d1[3], ln1 = 0;
@@ -178,7 +187,12 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
       double dr[3], rn[3], dn[3];
       lim_drift(d0, t, dr);
       for (int d = 0; d < 3; d++) rn[d] = r0[d] + (rq[d] * st + dr[d]);
-      mo_lap_point<double, double, 8>(S, V, S.spline, S.C[s], nm, rn, chi, roff, kCapF64, phi, lane);
+      if constexpr (SYS) {
+        mo_lap_point<double, double, 8>(S, V, S.spline, S.C[s], nm, rn, chi, roff, cap, phi, lane);
+      } else {
+        lcao_lap_n(S, s, nm, rn, chi, roff, phi, lane);
+        __syncthreads();
+      }
       if (lane < nm)
         for (int c = 0; c < 5; c++) phin[c * nsp + lane] = phi[c];
       __syncthreads();
@@ -186,7 +200,7 @@ __global__ __launch_bounds__(64) void k_sweep_md(DevSys S, DevWalkers W, SweepAr
       contract(std::integral_constant<int, 4>(), k, phin, den, tt);
       const double t0 = tt[0];
       double gj[3];
-      const double un = jastrow_e(S, e, rn, pos, gj, nullptr, lane, V.epos, 4);
+      const double un = jastrow(e, rn, gj);
       dn[0] = tt[1] / t0 + gj[0];
       dn[1] = tt[2] / t0 + gj[1];
       dn[2] = tt[3] / t0 + gj[2];

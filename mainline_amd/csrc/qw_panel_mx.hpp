@@ -1,9 +1,11 @@
 // Mixed-precision sweep of one spin channel, up to 64 electrons of a spin, with the inverse updated
 // panel by panel (FP32 LCAO; the arithmetic of qw_mixed.hpp's sweep, bit for bit).
 //
-//   k_sweep_mxp<NS, DEPTH, JP, STAGE>  single-electron moves (src/method/Split_sample.cpp:302-540,
+//   k_sweep_mxp<NS, DEPTH, JP, STAGE, SHL>  single-electron moves (src/method/Split_sample.cpp:302-540,
 //       src/program_utils/MatrixAlgebrac.cpp:766-838), one wavefront per walker, four walkers per
-//       block sharing the system tables
+//       block sharing the system tables; SHL = false: one walker per block with the shell records in
+//       device memory, for systems of so many shells that four walkers' tables and lists do not fit
+//       (from about 2400 shells on, 1500 with a thousand atoms)
 //
 // Only the rows of the next 16 electrons are held (four lanes per row, each with every fourth
 // value: the four partial sums of the update's dot product), and take every accepted move's
@@ -283,7 +285,7 @@ __device__ inline void mx_flush(float* ig, const float* mo0, int nsp, int n, int
 
 // The moves of walker w's spin A.s by one wavefront.  sh: the block's shared LDS, own: the
 // walker's region, Cl: the spin's coefficients in LDS (STAGE).  u: coefficient loads in flight.
-template <int NS, int DEPTH, bool JP, bool STAGE>
+template <int NS, int DEPTH, bool JP, bool STAGE, bool SHL = true>
 __device__ __forceinline__ void sweep_mxp_body(const DevSys& S, const MixedTables& M, const DevWalkers& W,
                                                const SweepArgs& A, int w, int lane, char* sh, const float* Cl, char* own,
                                                int u) {
@@ -293,7 +295,9 @@ __device__ __forceinline__ void sweep_mxp_body(const DevSys& S, const MixedTable
   const double* apos = (const double*)sh;
   const double* epos = apos + 3 * S.na;
   const double* tabs = epos + 3 * S.na;
-  const ShellLds* shl = (const ShellLds*)(tabs + 2 * S.ntab);
+  const ShellLds* shl;
+  if constexpr (SHL) shl = (const ShellLds*)(tabs + 2 * S.ntab);
+  else shl = S.shl;
   float* chi = (float*)own;
   int* roff = (int*)(chi + 5 * cap);
   int2* list = (int2*)(roff + cap);
@@ -525,9 +529,9 @@ __device__ __forceinline__ void sweep_mxp_body(const DevSys& S, const MixedTable
 }
 
 // The block's shared LDS: the tables of panel_stage, and with STAGE the spin's coefficients.
-template <bool STAGE>
+template <bool STAGE, bool SHL = true>
 __device__ inline const float* panel_mx_stage(const DevSys& S, const MixedTables& M, int s, char* sh, int t, int nt) {
-  panel_stage(S, sh, 1, t, nt);
+  panel_stage(S, sh, SHL ? 1 : 2, t, nt);
   float* Cl = (float*)(sh + lds_round16(panel_shared_lds(S.na, S.nsh, S.ntab, 1)));
   if constexpr (STAGE) {
     const int nc = S.nb * (s ? S.ndn : S.nup);
@@ -541,18 +545,19 @@ __device__ inline const float* panel_mx_stage(const DevSys& S, const MixedTables
 
 // Four waves per SIMD (128 registers, 8 spilled at 64 electrons of a spin) for the usual DMC sweep;
 // the delayed-rejection and general forms would spill a hundred there and run three.
-template <int NS, int DEPTH, bool JP, bool STAGE>
-__global__ __launch_bounds__(64 * kPanelWpb, DEPTH == 1 && JP ? 4 : 3) void k_sweep_mxp(DevSys S, MixedTables M, DevWalkers W, SweepArgs A,
-                                                                   int u) {
+template <int NS, int DEPTH, bool JP, bool STAGE, bool SHL = true>
+__global__ __launch_bounds__(64 * (SHL ? kPanelWpb : 1), DEPTH == 1 && JP ? 4 : 3) void k_sweep_mxp(
+    DevSys S, MixedTables M, DevWalkers W, SweepArgs A, int u) {
   extern __shared__ double ldsp[];
+  constexpr int wpb = SHL ? kPanelWpb : 1;
   char* sh = (char*)ldsp;
-  const float* Cl = panel_mx_stage<STAGE>(S, M, A.s, sh, (int)threadIdx.x, 64 * kPanelWpb);
+  const float* Cl = panel_mx_stage<STAGE, SHL>(S, M, A.s, sh, (int)threadIdx.x, 64 * wpb);
   __syncthreads();
-  const int wid = (int)threadIdx.x >> 6, w = (int)blockIdx.x * kPanelWpb + wid;
+  const int wid = (int)threadIdx.x >> 6, w = (int)blockIdx.x * wpb + wid;
   if (w >= W.nw) return;
-  char* own = sh + panel_mx_shared_lds(S.na, S.nsh, S.ntab, STAGE ? S.nb : 0, S.nsp) +
+  char* own = sh + panel_mx_shared_lds(S.na, SHL ? S.nsh : 0, S.ntab, STAGE ? S.nb : 0, S.nsp) +
               (size_t)wid * panel_mx_walker_lds(S.nsh, NS, DEPTH);
-  sweep_mxp_body<NS, DEPTH, JP, STAGE>(S, M, W, A, w, (int)threadIdx.x & 63, sh, Cl, own, u);
+  sweep_mxp_body<NS, DEPTH, JP, STAGE, SHL>(S, M, W, A, w, (int)threadIdx.x & 63, sh, Cl, own, u);
 }
 
 }  // namespace qw

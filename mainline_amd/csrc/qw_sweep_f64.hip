@@ -24,7 +24,10 @@ void by_form(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int u, hi
 
 void launch_sweep_f64(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st) {
   const int n = S.nup > S.ndn ? S.nup : S.ndn;
-  if (n <= 4) by_form<1, 4>(S, W, A, u, st);
+  // thousands of shells (from about 2400 on): the tables and lists of four walkers do not fit one
+  // block, and the two-wavefront form, which leaves the shell records in device memory, takes any size
+  if (n <= 64 && panel_lds_bytes(S.ne, S.na, S.nsh, S.ntab, pick_ns(n), 1, kPanelWpb) > kLdsMax) by_form<2, 128>(S, W, A, u, st);
+  else if (n <= 4) by_form<1, 4>(S, W, A, u, st);
   else if (n <= 8) by_form<1, 8>(S, W, A, u, st);
   else if (n <= 16) by_form<1, 16>(S, W, A, u, st);
   else if (n <= 32) by_form<1, 32>(S, W, A, u, st);
