@@ -299,7 +299,7 @@ struct qw_batch {
           lds_sweep = std::max(lds_sweep, kBatchWpb * lds_round16(sweep_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab,
                                                                                   e.ns, kCapF64, 8, B.depth)));
         else
-          lds_sweep = std::max(lds_sweep, panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, B.depth, 0, e.S.nsp));
+          lds_sweep = std::max(lds_sweep, panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, B.depth, 0, e.S.nsp, e.S.usual));
       } else if (precision == QW_PREC_FP64) {
         const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, kCapF64, sizeof(double));
         // walkers per block while their LDS leaves room for two blocks per compute unit
@@ -310,7 +310,7 @@ struct qw_batch {
       } else {
         B.wpb = 1;
         lds_sweep = std::max(lds_sweep, sweep_mxb_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab,
-                                                            std::max(e.T.nup, e.T.ndn), 2, B.depth));
+                                                            std::max(e.T.nup, e.T.ndn), 2, B.depth, e.S.usual));
         any_big = true;
       }
       any_pp |= e.S.has_pp != 0;

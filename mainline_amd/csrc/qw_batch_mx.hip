@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256, JP ? 4 : 3) void k_sweep_batch_mx(const BatchS
   const int wid = t >> 6, w = blk * kBatchWpb + wid;
   if (w >= B.W.nw) return;
   char* own = lds + panel_mx_shared_lds(B.S.na, B.S.nsh, B.S.ntab, 0, B.S.nsp) +
-              (size_t)wid * panel_mx_walker_lds(B.S.nsh, B.ns, DEPTH);
+              (size_t)wid * panel_mx_walker_lds(B.S.nsh, B.ns, DEPTH, JP || B.S.usual);
   if (JP || B.S.usual) batch_small<DEPTH, true>(gref(B.S), gref(B.M), gref(B.W), A, B.ns, w, t & 63, lds, own, B.u);
   else batch_small<DEPTH, false>(gref(B.S), gref(B.M), gref(B.W), A, B.ns, w, t & 63, lds, own, B.u);
 }

@@ -26,7 +26,6 @@
 namespace qw {
 
 constexpr int kBigPanel = 32;  // moves of one launch at most
-constexpr int kCapBig = 128;   // basis functions per wavefront's tile
 
 // floats per panel row: 16-byte chunks, an odd number of them (a lane per row: no bank conflicts)
 __host__ __device__ inline int big_ldp(int n) { return 4 * ((n + 3) / 4 | 1); }
@@ -38,9 +37,10 @@ __host__ __device__ inline size_t big_list_bytes(int nsh, int nw) {
 // LDS of one walker: positions, atoms, spacings | draws | panel rows | lists or value rows |
 // basis tiles | sums exchanged between the wavefronts.  192 electrons: 26.3 KB, six walkers per
 // compute unit.
-__host__ __device__ inline size_t sweep_mxb_lds_bytes(int ne, int na, int nsh, int ntab, int nmax, int nw, int depth) {
+__host__ __device__ inline size_t sweep_mxb_lds_bytes(int ne, int na, int nsh, int ntab, int nmax, int nw, int depth,
+                                                           bool usual) {
   return lds_round16((size_t)(3 * ne + 6 * na + 2 * ntab) * 8) + (size_t)kBigPanel * 32 * depth +
-         (size_t)kBigPanel * big_ldp(nmax) * 4 + big_list_bytes(nsh, nw) + (size_t)(nw - 1) * kCapBig * 24 + 128;
+         (size_t)kBigPanel * big_ldp(nmax) * 4 + big_list_bytes(nsh, nw) + (size_t)(nw - 1) * cap_mx(usual) * 24 + 128;
 }
 
 // jastrow_e_t<float, false> for the usual Jastrow: the same terms in the same order.
@@ -123,7 +123,7 @@ template <int NW, int DEPTH, bool JP>
 __device__ __forceinline__ void sweep_mxb_body(const DevSys& S, const MixedTables& M, const DevWalkers& W,
                                                const SweepArgs& A, int w, int t, char* base) {
   static_assert(NW == 2 || NW == 4, "wavefronts per walker");
-  constexpr int NR = NW, NB = NW - 1, cap = kCapBig, NT = 64 * NW;
+  constexpr int NR = NW, NB = NW - 1, cap = cap_mx(JP), NT = 64 * NW;
   const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
   const int ldp = big_ldp(S.nup > S.ndn ? S.nup : S.ndn), np = A.k1 - A.k0;

@@ -72,6 +72,7 @@ struct DevSys {
   // order, and one such POLYPADE object per atom type, evaluated without loops over objects and
   // functions; and shells of S, P, 5D, 6D and 10F symmetry only
   int usual;
+  int fg;  // 1: shells of F or G symmetry among them (7F, 7F_crystal, 9G, 9G_pyscf, 15G)
   const JRad<double>* eit;
   const JRad<float>* eitf;
   const int* eit_a0;

@@ -432,8 +432,9 @@ struct qw_engine {
       if (eit.empty()) eit.push_back(JObj{});
       S.n_eit = (int)rep.size();
       S.usual = usual_jastrow(T.ee, eit, o0) ? 1 : 0;
+      S.fg = 0;
       for (const ShellDesc& d : T.shells)
-        if (d.sym > SK_10F) S.usual = 0;
+        if (d.sym > SK_10F) S.usual = 0, S.fg = 1;
       S.eit = upload(jrad_table<double>(eit));
       S.eitf = upload(jrad_table<float>(eit));
       S.eit_a0 = upload(a0);

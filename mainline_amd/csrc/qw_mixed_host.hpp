@@ -68,7 +68,7 @@ void mixed_setup(qw_engine& e) {
   // the LDS-staged sweep variant is a tuning candidate where its LDS fits one workgroup
   int maxlds = 0;
   if (hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, e.device) != hipSuccess) maxlds = 0;
-  const size_t need = panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, 2, e.S.nb, e.S.nsp);
+  const size_t need = panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, 2, e.S.nb, e.S.nsp, e.S.usual);
   e.cl_ok = e.precision == QW_PREC_MIXED_FP32 && !e.big && need <= std::min<size_t>(kLdsMax, (size_t)maxlds);
 }
 

@@ -45,19 +45,23 @@ __device__ inline int lane_col(int q, int i) {
   return PanelMx<NS>::TPR == 4 ? 4 * i + q : 4 * (i >> 1) + 2 * q + (i & 1);
 }
 
-constexpr int kCapMx = 128;    // basis functions per LDS tile
+// Basis functions per LDS tile.  The general form's shells may be F and G, each a long serial loop that
+// every batch of shells repeats, so its tile takes twice the functions (six atoms of 29 functions, 7F
+// and 9G among them, 1024 walkers: a spin's VMC moves 0.98 -> 0.79 ms; without such shells no slower).
+__host__ __device__ constexpr int cap_mx(bool usual) { return usual ? 128 : 256; }
 constexpr int kMxStage = 4;    // updates staged in LDS at a time when a panel ends
 
 __host__ __device__ inline size_t panel_mx_shared_lds(int na, int nsh, int ntab, int stage_nb, int nsp) {
   return lds_round16(panel_shared_lds(na, nsh, ntab, 1)) + lds_round16((size_t)stage_nb * nsp * 4);
 }
-__host__ __device__ inline size_t panel_mx_walker_lds(int nsh, int ns, int depth) {
-  return (size_t)kCapMx * (5 * 4 + 4) + lds_round16((size_t)(nsh + 64) * 8) + (size_t)((ns <= 32 ? ns : 16) * depth * 4) * 8 +
+__host__ __device__ inline size_t panel_mx_walker_lds(int nsh, int ns, int depth, bool usual) {
+  return (size_t)cap_mx(usual) * (5 * 4 + 4) + lds_round16((size_t)(nsh + 64) * 8) + (size_t)((ns <= 32 ? ns : 16) * depth * 4) * 8 +
          lds_round16((size_t)2 * ns * 4) + (ns > 32 ? (size_t)kMxStage * 2 * ns * 4 : 0) + 64;
 }
 // stage_nb: the basis size when the coefficients are staged in LDS, else 0.
-__host__ __device__ inline size_t panel_mx_lds_bytes(int na, int nsh, int ntab, int ns, int depth, int stage_nb, int nsp) {
-  return panel_mx_shared_lds(na, nsh, ntab, stage_nb, nsp) + (size_t)kPanelWpb * panel_mx_walker_lds(nsh, ns, depth);
+__host__ __device__ inline size_t panel_mx_lds_bytes(int na, int nsh, int ntab, int ns, int depth, int stage_nb, int nsp,
+                                                          bool usual) {
+  return panel_mx_shared_lds(na, nsh, ntab, stage_nb, nsp) + (size_t)kPanelWpb * panel_mx_walker_lds(nsh, ns, depth, usual);
 }
 
 // PolyEval with the like and unlike coefficients equal (no choice per lane), and CuspEval with the
@@ -290,7 +294,7 @@ __device__ __forceinline__ void sweep_mxp_body(const DevSys& S, const MixedTable
                                                const SweepArgs& A, int w, int lane, char* sh, const float* Cl, char* own,
                                                int u) {
   typedef PanelMx<NS> D;
-  constexpr int P = D::P, TPR = D::TPR, EPT = D::EPT, cap = kCapMx;
+  constexpr int P = D::P, TPR = D::TPR, EPT = D::EPT, cap = cap_mx(JP);
   const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
   const double* apos = (const double*)sh;
   const double* epos = apos + 3 * S.na;
@@ -556,7 +560,7 @@ __global__ __launch_bounds__(64 * (SHL ? kPanelWpb : 1), DEPTH == 1 && JP ? 4 : 
   const int wid = (int)threadIdx.x >> 6, w = (int)blockIdx.x * wpb + wid;
   if (w >= W.nw) return;
   char* own = sh + panel_mx_shared_lds(S.na, SHL ? S.nsh : 0, S.ntab, STAGE ? S.nb : 0, S.nsp) +
-              (size_t)wid * panel_mx_walker_lds(S.nsh, NS, DEPTH);
+              (size_t)wid * panel_mx_walker_lds(S.nsh, NS, DEPTH, JP);
   sweep_mxp_body<NS, DEPTH, JP, STAGE, SHL>(S, M, W, A, w, (int)threadIdx.x & 63, sh, Cl, own, u);
 }
 

@@ -29,18 +29,25 @@ constexpr int kRowsWaves = 4;  // wavefronts of a block
 template <int KIND>
 struct RowsT {
   typedef float T;
-  static constexpr int cap = 128;  // functions of a tile
 };
 template <>
 struct RowsT<RowsF64> {
   typedef double T;
-  static constexpr int cap = 96;
 };
+// Functions of a tile.  FG: F and G shells, each a long serial loop that every batch of shells repeats:
+// a large tile (no larger than the basis, so that small systems keep four wavefronts per SIMD) and one
+// electron per wavefront.  Six atoms of 29 functions with 7F and 9G shells, 24 electrons: 512
+// configurations 276 -> 146 us, 1024 walkers 696 -> 268 us.
+template <int KIND, bool FG>
+__host__ __device__ inline int rows_cap(int nb) {
+  if constexpr (FG) return nb < 256 ? (nb + 1) & ~1 : 256;
+  else return KIND == RowsF64 ? 96 : 128;
+}
 
 // LDS of a wavefront: G tiles of values and coefficient offsets, G lists.
-template <int KIND, int G>
-__host__ __device__ inline size_t rows_wave_lds(int nsh) {
-  return G * ((size_t)RowsT<KIND>::cap * (5 * sizeof(typename RowsT<KIND>::T) + 4) +
+template <int KIND, int G, bool FG>
+__host__ __device__ inline size_t rows_wave_lds(int nb, int nsh) {
+  return G * ((size_t)rows_cap<KIND, FG>(nb) * (5 * sizeof(typename RowsT<KIND>::T) + 4) +
               (size_t)((nsh < kRowsWin ? nsh : kRowsWin) + 3) / 4 * 16);
 }
 
@@ -78,7 +85,7 @@ template <int KIND, bool FG>
 __device__ inline int rows_batch(const DevSys& S, const float* splf, const double p[3], const int* list, int i0, int nact,
                                  int n, typename RowsT<KIND>::T* chi, int* roff, int* nfun, int lane) {
   typedef typename RowsT<KIND>::T T;
-  constexpr int cap = RowsT<KIND>::cap;
+  const int cap = rows_cap<KIND, FG>(S.nb);
   const int i = i0 + lane;
   ShellLds d;
   int nf = 0;
@@ -172,10 +179,11 @@ __global__ __launch_bounds__(64 * kRowsWaves, 3) void k_rows(DevSys S, const dou
                                                              typename RowsT<KIND>::T* mo_out, int nw) {
   static_assert(NR == 1 || G == 1, "several electrons or several orbitals per lane");
   typedef typename RowsT<KIND>::T T;
-  constexpr int cap = RowsT<KIND>::cap, LE = kWave / G;
+  constexpr int LE = kWave / G;
+  const int cap = rows_cap<KIND, FG>(S.nb);
   extern __shared__ double ldsr[];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  char* own = (char*)ldsr + (size_t)wid * rows_wave_lds<KIND, G>(S.nsh);
+  char* own = (char*)ldsr + (size_t)wid * rows_wave_lds<KIND, G, FG>(S.nb, S.nsh);
   T* chi0 = (T*)own;
   int* roff0 = (int*)(chi0 + (size_t)G * 5 * cap);
   int* list0 = roff0 + G * cap;
@@ -254,23 +262,24 @@ inline void rows_go(const DevSys& S, const double* pos, const typename RowsT<KIN
   const size_t total = (size_t)nw * S.ne;
   auto go = [&](auto kern, int G, size_t lds) {
     const size_t blocks = (total + kRowsWaves * G - 1) / (kRowsWaves * G);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(64 * kRowsWaves), kRowsWaves * lds, st,
+    // whole rounds of four blocks per compute unit; with F and G shells (three) an electron per wavefront
+    const size_t most = S.fg ? 65536 : 4096;
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min(blocks, most)), dim3(64 * kRowsWaves), kRowsWaves * lds, st,
                        S, pos, C0, C1, splf, out, nw);
   };
-#define ROWS(NR, G) (S.usual ? go(k_rows<KIND, NR, G, false>, G, rows_wave_lds<KIND, G>(S.nsh)) \
-                             : go(k_rows<KIND, NR, G, true>, G, rows_wave_lds<KIND, G>(S.nsh)))
+#define ROWS(NR, G, FG) go(k_rows<KIND, NR, G, FG>, G, rows_wave_lds<KIND, G, FG>(S.nb, S.nsh))
   if constexpr (KIND != RowsF32) {
     // several electrons per wavefront fill the lanes of small systems (32 orbitals, 32000 electrons:
     // 163 -> 112 us), as long as that leaves four wavefronts per SIMD (1024 electrons of a
     // 2-orbital system: 7 us one at a time, 12 us four at a time)
     constexpr size_t kFill = 4096;
-    if (n <= 16 && total >= 4 * kFill) return ROWS(1, 4);
-    if (n <= 32 && total >= 2 * kFill) return ROWS(1, 2);
-    if (n <= 64) return ROWS(1, 1);
+    if (n <= 16 && total >= 4 * kFill && !S.fg) return ROWS(1, 4, false);
+    if (n <= 32 && total >= 2 * kFill && !S.fg) return ROWS(1, 2, false);
+    if (n <= 64) return S.fg ? ROWS(1, 1, true) : ROWS(1, 1, false);
   }
   if constexpr (KIND != RowsMx) {
-    if (n <= 128) ROWS(2, 1);
-    else ROWS(4, 1);
+    if (n <= 128) S.fg ? ROWS(2, 1, true) : ROWS(2, 1, false);
+    else S.fg ? ROWS(4, 1, true) : ROWS(4, 1, false);
   }
 #undef ROWS
 }

@@ -10,19 +10,19 @@ namespace {
 // FP32 LCAO (qw_panel_mx.hpp)
 template <int NS, int DEPTH, bool JP, bool STAGE>
 void go_p(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st) {
-  const size_t lds = panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, STAGE ? S.nb : 0, S.nsp);
+  const size_t lds = panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, STAGE ? S.nb : 0, S.nsp, JP);
   hipLaunchKernelGGL((k_sweep_mxp<NS, DEPTH, JP, STAGE>), dim3((unsigned)((W.nw + kPanelWpb - 1) / kPanelWpb)),
                      dim3(64 * kPanelWpb), lds, st, S, M, W, A, u);
 }
 // the form for thousands of shells: one instantiation for every size and trial function
 template <int DEPTH>
 void go_shells(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st) {
-  const size_t lds = panel_mx_shared_lds(S.na, 0, S.ntab, 0, S.nsp) + panel_mx_walker_lds(S.nsh, 64, DEPTH);
+  const size_t lds = panel_mx_shared_lds(S.na, 0, S.ntab, 0, S.nsp) + panel_mx_walker_lds(S.nsh, 64, DEPTH, false);
   hipLaunchKernelGGL((k_sweep_mxp<64, DEPTH, false, false, false>), dim3(W.nw), dim3(64), lds, st, S, M, W, A, u);
 }
 template <int NS, int DEPTH>
 void panel(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int choice, hipStream_t st) {
-  if (panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, 0, S.nsp) > kLdsMax) go_shells<DEPTH>(S, M, W, A, choice, st);
+  if (panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, 0, S.nsp, S.usual) > kLdsMax) go_shells<DEPTH>(S, M, W, A, choice, st);
   else if (choice >= 100) {
     if (S.usual) go_p<NS, DEPTH, true, true>(S, M, W, A, choice - 100, st);
     else go_p<NS, DEPTH, false, true>(S, M, W, A, choice - 100, st);
@@ -66,7 +66,7 @@ void launch_sweep_mx(const DevSys& S, const MixedTables& M, const DevWalkers& W,
 void launch_sweep_mx_big(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int depth,
                          hipStream_t st) {
   const int n = S.nup > S.ndn ? S.nup : S.ndn, nw = n <= 128 ? 2 : 4;
-  const size_t lds = sweep_mxb_lds_bytes(S.ne, S.na, S.nsh, S.ntab, n, nw, depth);
+  const size_t lds = sweep_mxb_lds_bytes(S.ne, S.na, S.nsh, S.ntab, n, nw, depth, S.usual);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(64 * nw), lds, st, S, M, W, A); };
   if (nw == 2) {
     if (depth == 1) S.usual ? go(k_sweep_mxb<2, 1, true>) : go(k_sweep_mxb<2, 1, false>);
