@@ -204,8 +204,11 @@ __host__ __device__ inline size_t panel_walker_lds(int ne, int nsh, int ns, int 
 __host__ __device__ inline size_t panel_lds_bytes(int ne, int na, int nsh, int ntab, int ns, int nw, int wpb) {
   return (panel_shared_lds(na, nsh, ntab, nw) + 15) / 16 * 16 + (size_t)wpb * panel_walker_lds(ne, nsh, ns, nw);
 }
-// Walkers per block: four wavefronts share the tables.
+// Walkers per block: up to four wavefronts share the tables, fewer where four would leave compute units
+// without a block (256 walkers of 8 electrons 286 -> 268 us a step pair, of 128 electrons 4.36 -> 4.11 ms;
+// 512: 293 -> 286 us and 4.42 -> 4.29 ms; from 769 on the same).
 constexpr int kPanelWpb = 4;
+inline int panel_wpb(int nw) { return nw > 768 ? kPanelWpb : nw > 512 ? 3 : nw > 256 ? 2 : 1; }
 
 // ---------------------------------------------------------------- basis
 // Active shells of point p among this thread's shells t, t + NT, ...: (meta, f0) appended to the
@@ -739,7 +742,7 @@ __global__ __launch_bounds__(NW == 1 ? 64 * kPanelWpb : 64 * NW, 3) void k_sweep
                                                                                    int u) {
   extern __shared__ double ldsp[];
   char* sh = (char*)ldsp;
-  constexpr int wpb = NW == 1 ? kPanelWpb : 1, nt = 64 * NW * wpb;
+  const int nt = (int)blockDim.x, wpb = NW == 1 ? nt >> 6 : 1;
   panel_stage(S, sh, NW, (int)threadIdx.x, nt);
   __syncthreads();
   const int wid = NW == 1 ? (int)threadIdx.x >> 6 : 0, t = NW == 1 ? (int)threadIdx.x & 63 : (int)threadIdx.x;

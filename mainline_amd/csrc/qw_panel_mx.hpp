@@ -60,8 +60,8 @@ __host__ __device__ inline size_t panel_mx_walker_lds(int nsh, int ns, int depth
 }
 // stage_nb: the basis size when the coefficients are staged in LDS, else 0.
 __host__ __device__ inline size_t panel_mx_lds_bytes(int na, int nsh, int ntab, int ns, int depth, int stage_nb, int nsp,
-                                                          bool usual) {
-  return panel_mx_shared_lds(na, nsh, ntab, stage_nb, nsp) + (size_t)kPanelWpb * panel_mx_walker_lds(nsh, ns, depth, usual);
+                                                          bool usual, int wpb = kPanelWpb) {
+  return panel_mx_shared_lds(na, nsh, ntab, stage_nb, nsp) + (size_t)wpb * panel_mx_walker_lds(nsh, ns, depth, usual);
 }
 
 // PolyEval with the like and unlike coefficients equal (no choice per lane), and CuspEval with the
@@ -553,9 +553,9 @@ template <int NS, int DEPTH, bool JP, bool STAGE, bool SHL = true>
 __global__ __launch_bounds__(64 * (SHL ? kPanelWpb : 1), DEPTH == 1 && JP ? 4 : 3) void k_sweep_mxp(
     DevSys S, MixedTables M, DevWalkers W, SweepArgs A, int u) {
   extern __shared__ double ldsp[];
-  constexpr int wpb = SHL ? kPanelWpb : 1;
+  const int wpb = (int)blockDim.x >> 6;
   char* sh = (char*)ldsp;
-  const float* Cl = panel_mx_stage<STAGE, SHL>(S, M, A.s, sh, (int)threadIdx.x, 64 * wpb);
+  const float* Cl = panel_mx_stage<STAGE, SHL>(S, M, A.s, sh, (int)threadIdx.x, (int)blockDim.x);
   __syncthreads();
   const int wid = (int)threadIdx.x >> 6, w = (int)blockIdx.x * wpb + wid;
   if (w >= W.nw) return;

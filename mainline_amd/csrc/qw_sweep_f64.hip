@@ -10,7 +10,7 @@ namespace qw {
 namespace {
 template <int NW, int NS, bool JP>
 void go(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st) {
-  constexpr int wpb = NW == 1 ? kPanelWpb : 1;
+  const int wpb = NW == 1 ? panel_wpb(W.nw) : 1;
   const size_t lds = panel_lds_bytes(S.ne, S.na, S.nsh, S.ntab, NS, NW, wpb);
   hipLaunchKernelGGL((k_sweep_p<NW, NS, JP>), dim3((unsigned)((W.nw + wpb - 1) / wpb)), dim3(64 * NW * wpb), lds,
                      st, S, W, A, u);

@@ -10,9 +10,10 @@ namespace {
 // FP32 LCAO (qw_panel_mx.hpp)
 template <int NS, int DEPTH, bool JP, bool STAGE>
 void go_p(const DevSys& S, const MixedTables& M, const DevWalkers& W, const SweepArgs& A, int u, hipStream_t st) {
-  const size_t lds = panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, STAGE ? S.nb : 0, S.nsp, JP);
-  hipLaunchKernelGGL((k_sweep_mxp<NS, DEPTH, JP, STAGE>), dim3((unsigned)((W.nw + kPanelWpb - 1) / kPanelWpb)),
-                     dim3(64 * kPanelWpb), lds, st, S, M, W, A, u);
+  const int wpb = STAGE ? kPanelWpb : panel_wpb(W.nw);  // (staged coefficients: always shared by four)
+  const size_t lds = panel_mx_lds_bytes(S.na, S.nsh, S.ntab, NS, DEPTH, STAGE ? S.nb : 0, S.nsp, JP, wpb);
+  hipLaunchKernelGGL((k_sweep_mxp<NS, DEPTH, JP, STAGE>), dim3((unsigned)((W.nw + wpb - 1) / wpb)),
+                     dim3(64 * wpb), lds, st, S, M, W, A, u);
 }
 // the form for thousands of shells: one instantiation for every size and trial function
 template <int DEPTH>
