@@ -246,7 +246,7 @@ __device__ __forceinline__ void local_body(const DevSys& S, const DevWalkers& W,
 }
 
 template <typename TM, bool MD, bool PP, bool JP>
-__global__ __launch_bounds__(64) void k_local(DevSys S, DevWalkers W, LocalArgs A) {
+__global__ __launch_bounds__(64, MD ? 3 : 1) void k_local(DevSys S, DevWalkers W, LocalArgs A) {
   extern __shared__ double lds[];
   local_body<TM, MD, PP, JP>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, lds);
 }

@@ -4,7 +4,7 @@
 // The ratio at a quadrature point of electron k is linear in the basis values there:
 //   sum_j inv(k, j) phi_j(r) = sum_b chi_b(r) D_b,  D_b = sum_j C[b][j] inv(k, j),
 // and D does not depend on the point.  So for each selected (atom, electron) pair D is formed
-// once, and a lane then takes one quadrature point (of several pairs at a time): it walks the
+// once (in large bases for the shells near its points only), and a lane then takes one quadrature point (of several pairs at a time): it walks the
 // shells near it adding chi_b D_b, and the Jastrow partners, with no sums over lanes and no
 // orbital at all.  The pair's own unmoved position is one more point (its Jastrow value).
 //
@@ -13,7 +13,7 @@
 // against 1.58 one at a time, three and four 1.56 and 1.75 (registers), eight coefficient loads
 // instead of four 1.40.  Contracting the orbitals at every point instead, four points at a time with the
 // wave over orbitals, partners and shells in turn, held 255 registers (two waves per SIMD; now
-// 123, four) and waited on coefficient loads.  Measured: local energy of the 64-electron
+// 161, three) and waited on coefficient loads.  Measured: local energy of the 64-electron
 // pseudopotential molecule, 4096 walkers 4.56 -> 1.27 ms, of N2 (10 electrons, 2048 walkers)
 // 0.232 -> 0.046 ms; 500 configurations of the 64-electron molecule 1.89 -> 0.62 ms.
 #pragma once
@@ -25,6 +25,11 @@ namespace qw {
 constexpr int kPPShells = 2;  // shells whose table rows are in flight together
 
 constexpr int kPPPairs = 8;  // pairs whose points the lanes share at most
+// Functions of a chunk up to which D is formed for all of them.  Above, only for those of shells that
+// reach a point: 32 atoms of 40 functions, 256 walkers, rules of 4, 6 and 12 points, a step pair 13.9,
+// 14.0 and 16.8 -> 9.6, 9.7 and 12.3 ms, 32 atoms of 13 8.7 -> 7.5 ms; 16 atoms of 13 functions, 4096
+// walkers, were 7 % slower with the list.
+constexpr int kPPAll = 256;
 
 // chi . D of one shell (values of shell_val; src/basis_function/Cubic_spline_calc.cpp:25-140).
 __device__ __attribute__((noinline)) double shell_poly_dot(int sym, double f, double x, double y, double z, const double* d) {
@@ -64,7 +69,38 @@ __host__ __device__ inline int pp_pairs(int aip) {
 }
 // (gmax: pp_pairs of the system's smallest quadrature, DevSys::pp_g).
 __host__ __device__ inline size_t pp_lds_doubles(int gmax, int chunk_nf, int nsp) {
-  return (size_t)gmax * (chunk_nf | 1) + (size_t)gmax * ((nsp + 2) & ~1) + 64 + (64 + kPPPairs);
+  return (size_t)gmax * (chunk_nf | 1) + (size_t)gmax * ((nsp + 2) & ~1) + 64 + (64 + kPPPairs) +
+         (chunk_nf > kPPAll ? (chunk_nf + 3) / 4 : 0);
+}
+
+// The functions (from f0 on) of the shells [sh0, sh1) that reach a point of the pairs list[0..np-1] into
+// fl, in order; returns their count.  reach: the pairs' smallest and largest distance of a point from
+// its atom, so the points lie between two spheres about the atom.
+__device__ inline int pp_reached(const DevSys& S, int sh0, int sh1, int f0, const int2* list, const double* reach, int np,
+                                 unsigned short* fl, int lane) {
+  int n = 0;
+  for (int s0 = sh0; s0 < sh1; s0 += kWave) {
+    const int sh = s0 + lane;
+    int nf = 0, f = 0;
+    if (sh < sh1) {
+      const ShellDesc d = S.shells[sh];
+      const double* b = S.atom_pos + 3 * d.atom;
+      const double rc = fmin(d.rcut, d.objthr);
+      f = d.f0 - f0;
+      for (int p = 0; p < np; p++) {
+        const double* a = S.atom_pos + 3 * list[p].x;
+        const double x = a[0] - b[0], y = a[1] - b[1], z = a[2] - b[2], lo = reach[2 * p], hi = reach[2 * p + 1];
+        const double r = sqrt(x * x + y * y + z * z);
+        // (rounding of the points' own distances is far below the margin; a NaN reaches everything)
+        if (!(fmax(r - hi, lo - r) >= rc + 1e-6 * (1.0 + r + hi))) nf = d.nf;
+      }
+    }
+    int tot;
+    const int at = n + wave_excl_scan(nf, lane, &tot);
+    for (int i = 0; i < nf; i++) fl[at + i] = (unsigned short)(f + i);
+    n += tot;
+  }
+  return n;
 }
 
 // Jastrow value of electron e at p, terms of every other electron and atom (this lane's own e, p).
@@ -111,8 +147,8 @@ __device__ inline double jastrow_at(const DevSys& S, int e, const double p[3], c
 template <typename TM, bool MD, bool JP>
 __device__ inline double pp_pairs_energy(const DevSys& S, const DevWalkers& W, const LocalArgs& A, int w,
                                          const QW_CONST PPType& P, const double* pos, const double rot[9],
-                                         const int2* list, int g, double* dl, double* rowl, double* vx, const double* bw,
-                                         double md_den, int lane) {
+                                         const int2* list, int g, double* dl, double* rowl, double* vx,
+                                         unsigned short* fl, const double* bw, double md_den, int lane) {
   const int nsp = S.nsp, ne = S.ne, ldd = S.chunk_nf | 1, ldr = (nsp + 2) & ~1, npt = P.aip + 1;
   __syncthreads();
   // the pairs' inverse rows
@@ -160,6 +196,23 @@ __device__ inline double pp_pairs_energy(const DevSys& S, const DevWalkers& W, c
     const double nr = sqrt(nd[0] * nd[0] + nd[1] * nd[1] + nd[2] * nd[2]);
     cs = (nd[0] * od[0] + nd[1] * od[1] + nd[2] * od[2]) / (nr * orr);
     wq = P.w[q];
+    if (S.chunk_nf > kPPAll) vx[lane] = nr;
+  }
+  if (S.chunk_nf > kPPAll) {
+    __syncthreads();
+    double lo = 0, hi = 0;
+    if (lane < g) {
+      lo = hi = vx[lane * npt];
+      for (int i = 1; i < P.aip; i++) {
+        lo = fmin(lo, vx[lane * npt + i]);
+        hi = fmax(hi, vx[lane * npt + i]);
+      }
+    }
+    __syncthreads();
+    if (lane < g) {  // (read until the energies of the points take its place)
+      vx[2 * lane] = lo;
+      vx[2 * lane + 1] = hi;
+    }
   }
   double R = 0;
   for (int ch = 0; ch < S.nchunk; ch++) {
@@ -168,15 +221,24 @@ __device__ inline double pp_pairs_energy(const DevSys& S, const DevWalkers& W, c
     const int f0 = shs[sh0].f0, f1 = shs[sh1 - 1].f0 + shs[sh1 - 1].nf;
     __syncthreads();
     // D of the chunk's functions, up to four pairs of one spin at a time (each coefficient load
-    // serves them all); Ct: the coefficients with the functions contiguous
+    // serves them all); Ct: the coefficients with the functions contiguous.  In a large chunk only
+    // those of shells that reach a point.
+    const bool all = f1 - f0 <= kPPAll;
     for (int p0 = 0; p0 < g;) {
       const int s = list[p0].y < S.nup ? 0 : 1, n = S.nmo[s];
       int np = 1;
       while (np < 4 && p0 + np < g && (list[p0 + np].y < S.nup ? 0 : 1) == s) np++;
       const double* r0 = rowl + p0 * ldr;
       const double *r1 = r0 + (np > 1 ? ldr : 0), *r2 = r0 + (np > 2 ? 2 * ldr : 0), *r3 = r0 + (np > 3 ? 3 * ldr : 0);
-      for (int f = f0 + lane; f < f1; f += kWave) {
-        const double* c = S.Ct[s] + f;
+      int nf = f1 - f0;
+      if (!all) {
+        __syncthreads();
+        nf = pp_reached(S, sh0, sh1, f0, list + p0, vx + 2 * p0, np, fl, lane);
+        __syncthreads();
+      }
+      for (int i = lane; i < nf; i += kWave) {
+        const int f = all ? i : fl[i];
+        const double* c = S.Ct[s] + f0 + f;
         double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
 #pragma unroll 4
         for (int j = 0; j < n; j++) {
@@ -186,7 +248,7 @@ __device__ inline double pp_pairs_energy(const DevSys& S, const DevWalkers& W, c
           a2 += v * r2[j];
           a3 += v * r3[j];
         }
-        double* o = dl + p0 * ldd + (f - f0);
+        double* o = dl + p0 * ldd + f;
         o[0] = a0;
         if (np > 1) o[ldd] = a1;
         if (np > 2) o[2 * ldd] = a2;
@@ -279,6 +341,7 @@ __device__ inline double pp_energy(const DevSys& S, const DevWalkers& W, const L
   double* rowl = dl + (size_t)S.pp_g * (S.chunk_nf | 1);
   double* vx = rowl + (size_t)S.pp_g * ((S.nsp + 2) & ~1);
   int2* list = (int2*)(vx + 64);
+  unsigned short* fl = (unsigned short*)(list + 64 + kPPPairs);
   double rot[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
   if (A.mode == 0) {
     if (A.rot)
@@ -306,7 +369,7 @@ __device__ inline double pp_energy(const DevSys& S, const DevWalkers& W, const L
       int done = 0;
       while (cnt - done >= G || (drain && cnt > done)) {
         const int g = min(G, cnt - done);
-        vnl += pp_pairs_energy<TM, MD, JP>(S, W, A, w, P, pos, rot, list + done, g, dl, rowl, vx, bw, md_den, lane);
+        vnl += pp_pairs_energy<TM, MD, JP>(S, W, A, w, P, pos, rot, list + done, g, dl, rowl, vx, fl, bw, md_den, lane);
         done += g;
       }
       if (done) {
