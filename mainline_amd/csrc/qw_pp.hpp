@@ -4,8 +4,8 @@
 // The ratio at a quadrature point of electron k is linear in the basis values there:
 //   sum_j inv(k, j) phi_j(r) = sum_b chi_b(r) D_b,  D_b = sum_j C[b][j] inv(k, j),
 // and D does not depend on the point.  So for each selected (atom, electron) pair D is formed
-// once (in large bases for the shells near its points only), and a lane then takes one quadrature point (of several pairs at a time): it walks the
-// shells near it adding chi_b D_b, and the Jastrow partners, with no sums over lanes and no
+// once (in large bases for the shells near its points only), and a lane then takes one quadrature
+// point (of several pairs at a time): it walks the shells near it adding chi_b D_b, and the Jastrow partners, with no sums over lanes and no
 // orbital at all.  The pair's own unmoved position is one more point (its Jastrow value).
 //
 // What bounds it: the latency of the shells' table rows and coefficients at three wavefronts per
@@ -15,7 +15,10 @@
 // wave over orbitals, partners and shells in turn, held 255 registers (two waves per SIMD; now
 // 161, three) and waited on coefficient loads.  Measured: local energy of the 64-electron
 // pseudopotential molecule, 4096 walkers 4.56 -> 1.27 ms, of N2 (10 electrons, 2048 walkers)
-// 0.232 -> 0.046 ms; 500 configurations of the 64-electron molecule 1.89 -> 0.62 ms.
+// 0.232 -> 0.046 ms; 500 configurations of the 64-electron molecule 1.89 -> 0.62 ms.  Several
+// determinants: with every lane searching all occupations for its orbital, 60 determinants of 64 electrons and
+// 50 orbitals took 1.75 times what contracting the points took; gathered by half-waves 0.7 times
+// (128 evaluations 15.0 -> 5.9 ms).
 #pragma once
 #include "qw_jastrow.hpp"
 #include "qw_kernels.hpp"
@@ -24,6 +27,7 @@ namespace qw {
 
 constexpr int kPPShells = 2;  // shells whose table rows are in flight together
 
+constexpr int kPPDets = 8;   // determinants whose rows are in flight together
 constexpr int kPPPairs = 8;  // pairs whose points the lanes share at most
 // Functions of a chunk up to which D is formed for all of them.  Above, only for those of shells that
 // reach a point: 32 atoms of 40 functions, 256 walkers, rules of 4, 6 and 12 points, a step pair 13.9,
@@ -152,23 +156,39 @@ __device__ inline double pp_pairs_energy(const DevSys& S, const DevWalkers& W, c
   const int nsp = S.nsp, ne = S.ne, ldd = S.chunk_nf | 1, ldr = (nsp + 2) & ~1, npt = P.aip + 1;
   __syncthreads();
   // the pairs' inverse rows
-  for (int p = 0; p < g; p++) {
-    const int e = list[p].y, s = e < S.nup ? 0 : 1, k = e - (s ? S.nup : 0), n = s ? S.ndn : S.nup;
-    if constexpr (MD) {
-      // the determinants' rows weighted and gathered onto the spin's orbital list
-      const int nd = S.ndet, ns = S.nsig;
-      const double* inv = W.invd + ((size_t)w * 2 + s) * nd * ns * ns + (size_t)k * ns;
-      const QW_CONST int* oc = cptr(S.occ) + (size_t)s * nd * ns;
-      for (int m = lane; m < S.nmo[s]; m += kWave) {
-        double v = 0;
-        for (int d = 0; d < nd; d++) {
-          double t = 0;
-          for (int j = 0; j < n; j++) t += oc[d * ns + j] == m ? inv[(size_t)d * ns * ns + j] : 0.0;
-          v += bw[d] * t;
+  if constexpr (MD) {
+    // the determinants' rows weighted and gathered onto the spin's orbital list, one half-wave per
+    // pair (at most 32 electrons of a spin): a determinant's orbitals are distinct, so its lanes add to
+    // distinct places, determinant after determinant
+    for (int i = lane; i < g * ldr; i += kWave) rowl[i] = 0.0;
+    const int nd = S.ndet, ns = S.nsig, j = lane & 31;
+    for (int p0 = 0; p0 < g; p0 += 2) {
+      const int p = p0 + (lane >> 5), e = list[min(p, g - 1)].y, s = e < S.nup ? 0 : 1, k = e - (s ? S.nup : 0);
+      const bool on = p < g && j < (s ? S.ndn : S.nup);
+      const double* inv = W.invd + ((size_t)w * 2 + s) * nd * ns * ns + (size_t)k * ns + j;
+      const int* oc = S.occ + (size_t)s * nd * ns + j;
+      double* row = rowl + p * ldr;
+      for (int d0 = 0; d0 < nd; d0 += kPPDets) {
+        double v[kPPDets];
+        int m[kPPDets];
+#pragma unroll
+        for (int i = 0; i < kPPDets; i++) {
+          const int d = min(d0 + i, nd - 1);
+          v[i] = on ? inv[(size_t)d * ns * ns] : 0.0;
+          m[i] = on ? oc[d * ns] : 0;
         }
-        rowl[p * ldr + m] = v / md_den;
+#pragma unroll
+        for (int i = 0; i < kPPDets; i++) {
+          wave_sync();
+          if (on && d0 + i < nd) row[m[i]] += bw[d0 + i] * v[i];
+        }
       }
-    } else {
+    }
+    __syncthreads();
+    for (int i = lane; i < g * ldr; i += kWave) rowl[i] /= md_den;
+  } else {
+    for (int p = 0; p < g; p++) {
+      const int e = list[p].y, s = e < S.nup ? 0 : 1, k = e - (s ? S.nup : 0), n = s ? S.ndn : S.nup;
       const TM* row = inv_store<TM>(W) + (((size_t)w * 2 + s) * nsp + k) * nsp;
       for (int j = lane; j < n; j += kWave) rowl[p * ldr + j] = (double)row[j];
     }
