@@ -227,7 +227,7 @@ qw_status qw_kernel_times(const qw_engine* e, char* buf, int buflen, double* avg
 qw_status qw_engine_walker_bytes(const qw_engine* e, int nw, unsigned long long* bytes);
 
 /* Launch choices the engine made (no reference counterpart): out4 = LCAO coefficient loads in
- * flight chosen by the online tuner (0 while it is still measuring), HIP graphs used for DMC
+ * flight chosen by the online tuner for the sweeps launched last (0 while it is still measuring), HIP graphs used for DMC
  * steps (0/1), block-per-walker kernels for more than 64 electrons of a spin (0/1), register
  * tile width of the inverse. */
 qw_status qw_engine_tuning(const qw_engine* e, int* out4);

@@ -129,7 +129,8 @@ qw_status make_engine(SysTables T, const qw_engine_opts* opts, qw_engine** out) 
   if (const char* t = std::getenv("QW_TUNE")) e->tune_enabled = t[0] != '0';
   if (const char* v = std::getenv("QW_INV")) e->inv_rows = std::strcmp(v, "rows") == 0;
   if (const char* c = std::getenv("QW_SWEEP"))
-    if (e->sweep_choice_ok(std::atoi(c))) e->tune_u = std::atoi(c);
+    if (e->sweep_choice_ok(std::atoi(c)))
+      for (auto& t : e->tune) t.u = std::atoi(c);
   *out = e.release();
   return QW_OK;
 }
@@ -169,7 +170,7 @@ extern "C" void qw_engine_destroy(qw_engine* e) { delete e; }
 
 extern "C" qw_status qw_engine_tuning(const qw_engine* e, int* out4) {
   if (!e || !out4) return QW_ERR_ARG;
-  out4[0] = e->tune_u;
+  out4[0] = e->tune[e->tune_last].u;
   out4[1] = e->use_graphs() ? 1 : 0;
   out4[2] = e->big ? 1 : 0;
   out4[3] = e->ns;

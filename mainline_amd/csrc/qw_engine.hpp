@@ -209,6 +209,8 @@ struct qw_engine {
       if (eval_ws) (void)hipFree(eval_ws);
     }
     for (auto& e : evs) pool.push_back(e.a), pool.push_back(e.b);
+    for (auto& t : tune)
+      for (auto& x : t.ev) pool.push_back(x.second.first), pool.push_back(x.second.second);
     for (auto ev : pool) (void)hipEventDestroy(ev);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -650,11 +652,12 @@ struct qw_engine {
       return;
     }
     if (precision == QW_PREC_FP64) {
-      const int u = pick_u();
-      tuned_launch([&] {
-        if (depth == 1) launch_sweep_f64(S, W, A, u, stream);
-        else launch_sweep_vmc64_big(S, W, A, stream);  // (up to 64 electrons of a spin: vmc_sweeps)
-      });
+      if (depth == 2) {  // (up to 64 electrons of a spin: vmc_sweeps); no choice of launch
+        launch("k_sweep", [&] { launch_sweep_vmc64_big(S, W, A, stream); });
+        return;
+      }
+      const int u = pick_u(kTuneSweep);
+      tuned_launch(kTuneSweep, [&] { launch_sweep_f64(S, W, A, u, stream); });
       return;
     }
     if (big) big_sweep(A, depth);
@@ -667,14 +670,21 @@ struct qw_engine {
   // sweep launches of an engine simply run with each candidate in turn (kTuneReps times),
   // timed with events; the fastest is kept for the engine's lifetime.  QW_TUNE=0 keeps the
   // default; QW_SWEEP=<choice> forces one.
+  // A choice is kept per family of kernels: FP64 VMC steps (k_sweeps), whose loads in flight mean
+  // something else than the DMC sweep's, and everything else.
   static constexpr int kTuneReps = 2;
+  enum { kTuneSweep, kTuneVmc64, kTuneFamilies };
+  struct SweepTune {
+    int u = 0;    // chosen launch, 0 while measuring
+    int n = 0;    // candidate launches issued
+    int cur = 0;  // candidate of the launch being issued
+    std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev;
+  };
   bool tune_enabled = true;
-  int tune_u = 0;      // chosen launch, 0 while measuring
-  int tune_n = 0;      // candidate launches issued
-  int tune_cur = 0;    // candidate of the launch being issued
+  SweepTune tune[kTuneFamilies];
+  int tune_last = kTuneSweep;  // the family launched last
   bool cl_ok = false;  // LDS-staged coefficients fit this device and system
   std::vector<int> tune_cands;
-  std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> tune_ev;
   int u_default() const { return precision == QW_PREC_FP64 ? 4 : 8; }
   // (The LDS-staged launches can be forced but are not tried: at 64 electrons of a spin and 8192
   // walkers one takes 3.3 ms against 1.28, so trying them cost a new engine's first run 14 %.)
@@ -686,17 +696,20 @@ struct qw_engine {
     if (std::count(cands().begin(), cands().end(), u)) return true;
     return cl_ok && (u == 104 || u == 108 || u == 116);
   }
-  int pick_u() {
-    if (tune_u) return tune_u;
+  int pick_u(int family) {
+    SweepTune& t = tune[family];
+    tune_last = family;
+    if (t.u) return t.u;
     if (!tune_enabled || capturing || (big && precision != QW_PREC_FP64) || (precision != QW_PREC_FP64 && precision != QW_PREC_MIXED_FP32))
       return u_default();
-    tune_cur = cands()[tune_n % cands().size()];
-    return tune_cur;
+    t.cur = cands()[t.n % cands().size()];
+    return t.cur;
   }
   // Launches a sweep; while the launch choice is being tuned the launch is bracketed by events.
   template <typename F>
-  void tuned_launch(F f) {
-    const bool measuring = !tune_u && tune_enabled && !capturing && tune_cur != 0;
+  void tuned_launch(int family, F f) {
+    SweepTune& T = tune[family];
+    const bool measuring = !T.u && tune_enabled && !capturing && T.cur != 0;
     if (!measuring) {
       launch("k_sweep", f);
       return;
@@ -705,16 +718,16 @@ struct qw_engine {
     HIPCHK(hipEventRecord(a, stream));
     launch("k_sweep", f);
     HIPCHK(hipEventRecord(b, stream));
-    tune_ev.push_back({tune_cur, {a, b}});
-    tune_cur = 0;
+    T.ev.push_back({T.cur, {a, b}});
+    T.cur = 0;
     const size_t nc = cands().size();
-    if (++tune_n < (int)(nc * kTuneReps)) return;
+    if (++T.n < (int)(nc * kTuneReps)) return;
     HIPCHK(hipEventSynchronize(b));
     double best = 1e300;
     for (size_t i = 0; i < nc; i++) {
       const int u = tune_cands[i];
       double t = 1e300;
-      for (auto& x : tune_ev)
+      for (auto& x : T.ev)
         if (x.first == u) {
           float ms = 0;
           HIPCHK(hipEventElapsedTime(&ms, x.second.first, x.second.second));
@@ -722,11 +735,11 @@ struct qw_engine {
         }
       if (t < best) {
         best = t;
-        tune_u = u;
+        T.u = u;
       }
     }
-    for (auto& x : tune_ev) pool.push_back(x.second.first), pool.push_back(x.second.second);
-    tune_ev.clear();
+    for (auto& x : T.ev) pool.push_back(x.second.first), pool.push_back(x.second.second);
+    T.ev.clear();
   }
   void ensure_tneg() {
     if (tneg && tnegcap >= nw) return;
@@ -946,8 +959,8 @@ struct qw_engine {
   // nsw sweeps of both spins in one launch (one determinant, FP64, up to 64 electrons of a spin)
   void vmc_sweeps(double tau, int nsw) {
     const SweepArgs A{0, 0, 0, tau, seed, step, 0u, 0, 0, dstep};
-    const int u = pick_u();
-    tuned_launch([&] { launch_sweeps_vmc64(S, W, A, nsw, ns, u, stream); });
+    const int u = pick_u(kTuneVmc64);
+    tuned_launch(kTuneVmc64, [&] { launch_sweeps_vmc64(S, W, A, nsw, ns, u, stream); });
   }
   // one VMC step: ndecorr sweeps of both spin channels, then the local energy
   void vmc_step(const qw_method_desc& m, RunState& R) {

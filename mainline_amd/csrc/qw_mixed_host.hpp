@@ -112,8 +112,8 @@ void mixed_sweep(qw_engine& e, const SweepArgs& A0, int depth) {
     A.k0 = k0;
     A.k1 = std::min(A0.k1, k0 + e.refresh);
     A.dets = A0.dets && A.k1 == A0.k1;
-    const int choice = e.pick_u();
-    e.tuned_launch([&] { launch_sweep_mx(e.S, e.MT, e.W, A, depth, e.ns, mode, choice, e.stream); });
+    const int choice = e.pick_u(e.kTuneSweep);
+    e.tuned_launch(e.kTuneSweep, [&] { launch_sweep_mx(e.S, e.MT, e.W, A, depth, e.ns, mode, choice, e.stream); });
     mixed_lu(e, A.s);
   }
 }
