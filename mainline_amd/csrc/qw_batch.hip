@@ -301,7 +301,7 @@ struct qw_batch {
         else
           lds_sweep = std::max(lds_sweep, panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, B.depth, 0, e.S.nsp, e.S.usual));
       } else if (precision == QW_PREC_FP64) {
-        const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp, kCapF64, sizeof(double));
+        const size_t per = sweep_w_lds_bytes(e.S.ne, e.S.na, e.S.nsh, e.S.ntab, e.S.nsp);
         // walkers per block while their LDS leaves room for two blocks per compute unit
         B.wpb = (int)std::max<size_t>(1, std::min<size_t>(kBatchWpb, (80u << 10) / per));
         B.lds_w = (int)per;

@@ -39,21 +39,20 @@ __device__ __forceinline__ void batch_vmc(const QW_CONST BatchSlot& B, const Swe
   const int t = (int)threadIdx.x, lane = t & 63, wid = t >> 6;
   if (B.ns == 0) {
     if (wid >= B.wpb) return;
-    const BigPtrs<double> P{B.W.inv, B.W.mo, {B.S.C[0], B.S.C[1]}, B.S.spline};
     char* base = lds + (size_t)wid * B.lds_w;
     const int w = blk * B.wpb + wid;
-    if (B.nr == 2) sweep_w_body<double, double, 2, 2, kBatchWpb>(gref(B.S), gref(B.W), P, A, kCapF64, w, lane, base);
-    else sweep_w_body<double, double, 2, 4, kBatchWpb>(gref(B.S), gref(B.W), P, A, kCapF64, w, lane, base);
+    if (B.nr == 2) sweep_w_body<2, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, base);
+    else sweep_w_body<4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, base);
     return;
   }
   const int w = blk * kBatchWpb + wid;
   // one choice of loads in flight serves the batch (every choice gives the same results)
   switch (B.ns) {
-    case 4: sweep_fp64_body<4, 2, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
-    case 8: sweep_fp64_body<8, 2, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
-    case 16: sweep_fp64_body<16, 2, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
-    case 32: sweep_fp64_body<32, 2, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
-    default: sweep_fp64_body<64, 2, 8, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
+    case 4: sweep_fp64_body<4, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
+    case 8: sweep_fp64_body<8, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
+    case 16: sweep_fp64_body<16, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
+    case 32: sweep_fp64_body<32, 4, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
+    default: sweep_fp64_body<64, 8, kBatchWpb>(gref(B.S), gref(B.W), A, w, lane, wid, lds); break;
   }
 }
 

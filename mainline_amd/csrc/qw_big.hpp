@@ -1,12 +1,11 @@
 // Walker kernels for more than 64 electrons of one spin (up to 256).
 //
-//   k_sweep_w<TI, R, DEPTH, NR>  moves of one spin channel by one 64-lane wavefront per walker
+//   k_sweep_w<NR>       FP64 VMC moves of one spin channel by one 64-lane wavefront per walker
 //                       (src/method/Split_sample.cpp:302-540,
 //                       src/program_utils/MatrixAlgebrac.cpp:766-838): lane l owns rows and MOs
 //                       l, l+64, ... (NR of them); the inverse stays in device memory (too
 //                       large for one wavefront's registers) and each Sherman-Morrison update
-//                       streams the lane's rows; TI = inverse / MO cache element type, R =
-//                       Jastrow arithmetic
+//                       streams the lane's rows
 //   k_inv_grid<G>       FP64 pivoted Gauss-Jordan over a G x G thread grid (up to 128 per spin)
 //   k_inv_panel         the same Gauss-Jordan for 129 to 256 per spin, panel by panel with
 //                       the working matrix in device memory (src/program_utils/MatrixAlgebrac.cpp:
@@ -21,41 +20,6 @@ constexpr int kBigMaxSpin = 256;
 // registers); above, k_inv_panel.
 constexpr int kGridMaxSpin = 128;
 
-// Spline table element type that goes with an inverse / MO cache element type.
-template <typename TI>
-struct SplineOf {
-  using type = double;
-};
-template <>
-struct SplineOf<float> {
-  using type = float;
-};
-template <typename TI>
-using TS_SPLINE_T = typename SplineOf<TI>::type;
-
-// Jastrow objects of the arithmetic type R.
-template <typename R>
-__device__ inline const JRad<R>* jee(const DevSys& S);
-template <>
-__device__ inline const JRad<double>* jee<double>(const DevSys& S) { return S.ee; }
-template <>
-__device__ inline const JRad<float>* jee<float>(const DevSys& S) { return S.eef; }
-template <typename R>
-__device__ inline const JRad<R>* jei(const DevSys& S);
-template <>
-__device__ inline const JRad<double>* jei<double>(const DevSys& S) { return S.eit; }
-template <>
-__device__ inline const JRad<float>* jei<float>(const DevSys& S) { return S.eitf; }
-
-// Pointers of one precision for the big kernels.
-template <typename TI>
-struct BigPtrs {
-  TI* inv;           // [nw][2][nsp][nsp]
-  TI* mo;            // [nw][ne][5][nsp]
-  const TI* C[2];    // [nb][nspin] coefficients
-  const void* spline;  // double or float table, matching TI
-};
-
 // ---------------------------------------------------------------- one wavefront per walker
 // The same moves with one 64-lane wavefront per walker: lane l owns rows and MOs l, l+64, ...
 // (NR of them, nsigma <= 64 NR), so the whole move runs without block barriers and a compute
@@ -63,36 +27,36 @@ struct BigPtrs {
 // recompute writes it); row k and the accepted point's MO values go through LDS.
 
 // LDS of one walker: positions | system tables | basis tile | inverse row k and new MO values.
-__host__ __device__ inline size_t sweep_w_lds_bytes(int ne, int na, int nsh, int ntab, int nsp, int cap, int tsize) {
+__host__ __device__ inline size_t sweep_w_lds_bytes(int ne, int na, int nsh, int ntab, int nsp) {
   return ((((size_t)3 * ne * sizeof(double) + 15) & ~(size_t)15) + ((sys_lds_bytes(na, nsh, ntab) + 15) & ~(size_t)15) +
-          (size_t)5 * cap * tsize + (size_t)cap * sizeof(int) + (size_t)2 * nsp * tsize + 15) &
+          (size_t)kCapF64 * (5 * sizeof(double) + sizeof(int)) + (size_t)2 * nsp * sizeof(double) + 15) &
          ~(size_t)15;
 }
 
 // The sweep of walker w by one wavefront (base: its LDS region of sweep_w_lds_bytes); WPB > 1:
 // other wavefronts of the block run other walkers (wavefront-level barriers only).
-template <typename TI, typename R, int DEPTH, int NR, int WPB>
-__device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& W, const BigPtrs<TI>& P,
-                                             const SweepArgs& A, int cap, int w, int lane, char* base) {
+template <int NR, int WPB>
+__device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int w, int lane,
+                                             char* base) {
+  constexpr int cap = kCapF64;
   if (w >= W.nw) return;
   const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
   // rows of the inverse and of the MO cache start 16-byte aligned when nsp is a multiple of
   // the values per 16 bytes
-  constexpr int per = 16 / sizeof(TI);
-  typedef TI tvr __attribute__((ext_vector_type(per)));
+  constexpr int per = 2;
+  typedef double tvr __attribute__((ext_vector_type(per)));
   const bool vrow = nsp % per == 0;
   double* pos = (double*)base;
   SysLds V;
   char* q = sys_lds_carve(S, base + (((size_t)3 * ne * sizeof(double) + 15) & ~(size_t)15), V);
-  TI* chi = (TI*)q;
+  double* chi = (double*)q;
   int* roff = (int*)(chi + 5 * cap);
-  TI* rowk = (TI*)(roff + cap);
-  TI* phi0 = rowk + nsp;
+  double* rowk = (double*)(roff + cap);
+  double* phi0 = rowk + nsp;
   for (int i = lane; i < 3 * ne; i += kWave) pos[i] = W.pos[(size_t)w * ne * 3 + i];
   stage_sys(S, V, lane);
-  TI* ig = P.inv + ((size_t)w * 2 + s) * nsp * nsp;
-  TI* mog = P.mo + (size_t)w * ne * 5 * nsp;
-  const TS_SPLINE_T<TI>* spline = (const TS_SPLINE_T<TI>*)P.spline;
+  double* ig = W.inv + ((size_t)w * 2 + s) * nsp * nsp;
+  double* mog = W.mo + (size_t)w * ne * 5 * nsp;
   double logdet = W.logdet[2 * w + s], sgn = W.sgn[2 * w + s];
   int nacc = 0;
   const double tau = A.tau, stau = sqrt(tau);
@@ -105,8 +69,8 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const int j = lane + kWave * r;
-      const TI v = j < n ? ig[(size_t)k * nsp + j] : (TI)0;
-      rk[r] = (double)v;
+      const double v = j < n ? ig[(size_t)k * nsp + j] : 0;
+      rk[r] = v;
       if (j < nsp) rowk[j] = v;
     }
     double gd[3] = {0, 0, 0};
@@ -114,17 +78,17 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
     for (int r = 0; r < NR; r++) {
       const int j = lane + kWave * r;
       if (j < n)
-        for (int c = 0; c < 3; c++) gd[c] += rk[r] * (double)mog[((size_t)e * 5 + 1 + c) * nsp + j];
+        for (int c = 0; c < 3; c++) gd[c] += rk[r] * mog[((size_t)e * 5 + 1 + c) * nsp + j];
     }
     for (int c = 0; c < 3; c++) gd[c] = wsum(gd[c]);
-    R g0[3];
-    const double u0 = (double)jastrow_e_t<R, false>(S, jee<R>(S), jei<R>(S), e, r0, pos, g0, nullptr, lane, V.epos, 4);
-    const double d0[3] = {gd[0] + (double)g0[0], gd[1] + (double)g0[1], gd[2] + (double)g0[2]};
-    TI acc[NR][5];
+    double g0[3];
+    const double u0 = jastrow_e_t<double, false>(S, S.ee, S.eit, e, r0, pos, g0, nullptr, lane, V.epos, 4);
+    const double d0[3] = {gd[0] + g0[0], gd[1] + g0[1], gd[2] + g0[2]};
+    double acc[NR][5];
     double r1[3], d1[3], ln1 = 0, Rt = 0;
     bool accepted = false;
     double acc_first = 0;
-    for (int dep = 1; dep <= DEPTH && !accepted; dep++) {
+    for (int dep = 1; dep <= 2 && !accepted; dep++) {
       const double tt = dep == 1 ? tau : tau * 0.5, st = dep == 1 ? stau : sqrt(tau * 0.5);
       double g[3], dr[3], rn[3], dn[3];
       gauss3(A.seed, (unsigned)w, step_of(A.step, A.stepp), (unsigned)e, (dep == 1 ? TAG_GAUSS1 : TAG_GAUSS2) | (A.sweep << 8), g);
@@ -132,31 +96,31 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
       for (int d = 0; d < 3; d++) rn[d] = r0[d] + (g[d] * st + dr[d]);
 #pragma unroll
       for (int r = 0; r < NR; r++)
-        for (int c = 0; c < 5; c++) acc[r][c] = (TI)0;
+        for (int c = 0; c < 5; c++) acc[r][c] = 0;
       const int nact = basis_active(S, V, rn, lane);
       walker_sync<WPB>();
       for (int i0 = 0; i0 < nact;) {
         int nfun;
         const int take =
-            basis_batch_lap<TI, TS_SPLINE_T<TI>>(S, V, spline, rn, i0, nact, n, chi, cap, roff, cap, &nfun, lane);
+            basis_batch_lap<double, double>(S, V, S.spline, rn, i0, nact, n, chi, cap, roff, cap, &nfun, lane);
         walker_sync<WPB>();
 #pragma unroll
         for (int r = 0; r < NR; r++)
-          if (lane + kWave * r < n) lcao_batch<TI, 4>(P.C[s] + kWave * r, roff, chi, cap, nfun, acc[r], lane);
+          if (lane + kWave * r < n) lcao_batch<double, 4>(S.C[s] + kWave * r, roff, chi, cap, nfun, acc[r], lane);
         walker_sync<WPB>();
         i0 += take;
       }
       double tv[4] = {0, 0, 0, 0};
 #pragma unroll
       for (int r = 0; r < NR; r++)
-        for (int c = 0; c < 4; c++) tv[c] += rk[r] * (double)acc[r][c];
+        for (int c = 0; c < 4; c++) tv[c] += rk[r] * acc[r][c];
       for (int c = 0; c < 4; c++) tv[c] = wsum(tv[c]);
       const double t0 = tv[0];
-      R g2[3];
-      const double un = (double)jastrow_e_t<R, false>(S, jee<R>(S), jei<R>(S), e, rn, pos, g2, nullptr, lane, V.epos, 4);
-      dn[0] = tv[1] / t0 + (double)g2[0];
-      dn[1] = tv[2] / t0 + (double)g2[1];
-      dn[2] = tv[3] / t0 + (double)g2[2];
+      double g2[3];
+      const double un = jastrow_e_t<double, false>(S, S.ee, S.eit, e, rn, pos, g2, nullptr, lane, V.epos, 4);
+      dn[0] = tv[1] / t0 + g2[0];
+      dn[1] = tv[2] / t0 + g2[1];
+      dn[2] = tv[3] / t0 + g2[2];
       const double lnn = log(fabs(t0)) + (un - u0);
       const bool neg = t0 < 0;
       double acc_p;
@@ -191,14 +155,14 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
 #pragma unroll
       for (int r = 0; r < NR; r++) {
         const int j = lane + kWave * r;
-        if (j < nsp) phi0[j] = j < n ? acc[r][0] : (TI)0;
+        if (j < nsp) phi0[j] = j < n ? acc[r][0] : 0;
       }
       walker_sync<WPB>();
 #pragma unroll
       for (int r = 0; r < NR; r++) {
         const int i = lane + kWave * r;
         if (i >= n) continue;
-        TI* row = ig + (size_t)i * nsp;
+        double* row = ig + (size_t)i * nsp;
         // 16-byte accesses to the lane's row where the rows start 16-byte aligned (the same
         // arithmetic in the same order as the one-value loop that finishes the row)
         const int jv = vrow ? n / per * per : 0;
@@ -207,26 +171,26 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
           for (int j = 0; j < jv; j += per) {
             tvr u;
 #pragma unroll
-            for (int q = 0; q < per; q++) u[q] = (TI)((double)rowk[j + q] * f);
+            for (int q = 0; q < per; q++) u[q] = rowk[j + q] * f;
             *(tvr*)(row + j) = u;
           }
-          for (int j = jv; j < n; j++) row[j] = (TI)((double)rowk[j] * f);
+          for (int j = jv; j < n; j++) row[j] = rowk[j] * f;
         } else {
           double tk = 0;
           for (int j = 0; j < jv; j += per) {
             const tvr u = *(const tvr*)(row + j);
 #pragma unroll
-            for (int q = 0; q < per; q++) tk += (double)u[q] * (double)phi0[j + q];
+            for (int q = 0; q < per; q++) tk += u[q] * phi0[j + q];
           }
-          for (int j = jv; j < n; j++) tk += (double)row[j] * (double)phi0[j];
+          for (int j = jv; j < n; j++) tk += row[j] * phi0[j];
           const double pk = tk * (-1.0 / Rt);
           for (int j = 0; j < jv; j += per) {
             tvr u = *(const tvr*)(row + j);
 #pragma unroll
-            for (int q = 0; q < per; q++) u[q] = (TI)((double)u[q] + (double)rowk[j + q] * pk);
+            for (int q = 0; q < per; q++) u[q] = u[q] + rowk[j + q] * pk;
             *(tvr*)(row + j) = u;
           }
-          for (int j = jv; j < n; j++) row[j] = (TI)((double)row[j] + (double)rowk[j] * pk);
+          for (int j = jv; j < n; j++) row[j] = row[j] + rowk[j] * pk;
         }
         for (int c = 0; c < 5; c++) mog[((size_t)e * 5 + c) * nsp + i] = acc[r][c];
       }
@@ -251,8 +215,8 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
     for (int r = 0; r < NR; r++) {
       const int t = lane + kWave * r;
       if (t >= n) continue;
-      const TI* row = ig + (size_t)t * nsp;
-      const TI* mr = mog + (size_t)(off + t) * 5 * nsp;
+      const double* row = ig + (size_t)t * nsp;
+      const double* mr = mog + (size_t)(off + t) * 5 * nsp;
       double dv[4] = {0, 0, 0, 0};
       const int jv = vrow ? n / per * per : 0;
       for (int j = 0; j < jv; j += per) {
@@ -262,14 +226,14 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
         for (int c = 0; c < 4; c++) m[c] = *(const tvr*)(mr + (size_t)(c + 1) * nsp + j);
 #pragma unroll
         for (int q = 0; q < per; q++) {
-          const double iv = (double)u[q];
+          const double iv = u[q];
 #pragma unroll
-          for (int c = 0; c < 4; c++) dv[c] += (double)m[c][q] * iv;
+          for (int c = 0; c < 4; c++) dv[c] += m[c][q] * iv;
         }
       }
       for (int j = jv; j < n; j++) {
-        const double iv = (double)row[j];
-        for (int c = 0; c < 4; c++) dv[c] += (double)mr[(size_t)(c + 1) * nsp + j] * iv;
+        const double iv = row[j];
+        for (int c = 0; c < 4; c++) dv[c] += mr[(size_t)(c + 1) * nsp + j] * iv;
       }
       double* o = W.dgl + ((size_t)w * ne + off + t) * 4;
       for (int c = 0; c < 4; c++) o[c] = dv[c];
@@ -277,10 +241,10 @@ __device__ __forceinline__ void sweep_w_body(const DevSys& S, const DevWalkers& 
   }
 }
 
-template <typename TI, typename R, int DEPTH, int NR>
-__global__ __launch_bounds__(64) void k_sweep_w(DevSys S, DevWalkers W, BigPtrs<TI> P, SweepArgs A, int cap) {
+template <int NR>
+__global__ __launch_bounds__(64) void k_sweep_w(DevSys S, DevWalkers W, SweepArgs A) {
   extern __shared__ double lds[];
-  sweep_w_body<TI, R, DEPTH, NR, 1>(S, W, P, A, cap, (int)blockIdx.x, (int)threadIdx.x, (char*)lds);
+  sweep_w_body<NR, 1>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, (char*)lds);
 }
 
 // ---------------------------------------------------------------- k_inv_grid

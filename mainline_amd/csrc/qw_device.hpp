@@ -501,54 +501,6 @@ __device__ inline void shell_val(int sym, double f, double x, double y, double z
   }
 }
 
-// Basis values of the shells [sh0, sh1) at point p, written to chi[c*ld + (f - f0)]
-// (c = value, d/dx, d/dy, d/dz, laplacian), zero beyond each shell's cutoff.
-// Lanes take shells round-robin.  Table indices are clamped to the table.
-template <typename T>
-__device__ inline void basis_lap(const DevSys& S, const double p[3], int sh0, int sh1, int f0, T* chi, int ld, int lane) {
-  for (int sh = sh0 + lane; sh < sh1; sh += kWave) {
-    const ShellDesc d = S.shells[sh];
-    const double* ap = S.atom_pos + 3 * d.atom;
-    double x = p[0] - ap[0], y = p[1] - ap[1], z = p[2] - ap[2];
-    double r2 = x * x + y * y + z * z, r = sqrt(r2);
-    T* o = chi + (d.f0 - f0);
-    if (r < d.rcut && r < d.objthr) {
-      int iv = (int)(r * S.tab_inv[d.table]);
-      iv = iv < 0 ? 0 : (iv >= S.nint ? S.nint - 1 : iv);
-      const double* c = S.spline + ((size_t)d.table * S.nint + iv) * 4;
-      double h = r - iv * S.tab_sp[d.table];
-      double f = c[0] + h * (c[1] + h * (c[2] + h * c[3]));
-      double fd = (c[1] + h * (2 * c[2] + h * (3 * c[3]))) / r;
-      double f2 = 2 * c[2] + 6 * h * c[3];
-      shell_lap<T>(d.sym, f, fd, f2, x, y, z, o, ld);
-    } else {
-      for (int i = 0; i < d.nf; i++)
-        for (int c5 = 0; c5 < 5; c5++) o[c5 * ld + i] = (T)0;
-    }
-  }
-}
-
-template <typename T>
-__device__ inline void basis_val(const DevSys& S, const double p[3], int sh0, int sh1, int f0, T* chi, int lane) {
-  for (int sh = sh0 + lane; sh < sh1; sh += kWave) {
-    const ShellDesc d = S.shells[sh];
-    const double* ap = S.atom_pos + 3 * d.atom;
-    double x = p[0] - ap[0], y = p[1] - ap[1], z = p[2] - ap[2];
-    double r = sqrt(x * x + y * y + z * z);
-    T* o = chi + (d.f0 - f0);
-    if (r < d.rcut && r < d.objthr) {
-      int iv = (int)(r * S.tab_inv[d.table]);
-      iv = iv < 0 ? 0 : (iv >= S.nint ? S.nint - 1 : iv);
-      const double* c = S.spline + ((size_t)d.table * S.nint + iv) * 4;
-      double h = r - iv * S.tab_sp[d.table];
-      double f = c[0] + h * (c[1] + h * (c[2] + h * c[3]));
-      shell_val<T>(d.sym, f, x, y, z, o);
-    } else {
-      for (int i = 0; i < d.nf; i++) o[i] = (T)0;
-    }
-  }
-}
-
 // Exclusive prefix sum across the wave of small counts (0 <= v < 16, the function count of one
 // shell) from four ballots; *total receives the wave sum.
 __device__ inline int wave_excl_scan(int v, int lane, int* total) {

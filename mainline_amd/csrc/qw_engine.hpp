@@ -664,9 +664,9 @@ struct qw_engine {
     else mixed_sweep(*this, A, depth);
   }
 
-  // ---- online tuning of the sweep launch: LCAO coefficient loads in flight (U) and, on the
-  // FP32 mixed path, whether a block stages the coefficients in LDS for several walkers
-  // (choice 100 + U).  The candidates do the same arithmetic in the same order, so the first
+  // ---- online tuning of the sweep launch: LCAO coefficient loads in flight (U; on the FP32
+  // mixed path 100 + U forces the launch whose blocks stage the coefficients in LDS for four
+  // walkers).  The candidates do the same arithmetic in the same order, so the first
   // sweep launches of an engine simply run with each candidate in turn (kTuneReps times),
   // timed with events; the fastest is kept for the engine's lifetime.  QW_TUNE=0 keeps the
   // default; QW_SWEEP=<choice> forces one.
@@ -686,8 +686,10 @@ struct qw_engine {
   bool cl_ok = false;  // LDS-staged coefficients fit this device and system
   std::vector<int> tune_cands;
   int u_default() const { return precision == QW_PREC_FP64 ? 4 : 8; }
-  // (The LDS-staged launches can be forced but are not tried: at 64 electrons of a spin and 8192
-  // walkers one takes 3.3 ms against 1.28, so trying them cost a new engine's first run 14 %.)
+  // (The LDS-staged launches can be forced but are not tried: from 1 to 24 electrons of a spin the
+  // fastest of them takes 0.98 to 1.04 times the fastest other, 1024 and 8192 walkers, DMC and VMC; at
+  // 32, 48 and 64 and 8192 walkers 1.2, 2.5 and 2.5 times, so trying them cost a new engine's first
+  // run 14 %.)
   const std::vector<int>& cands() {
     if (tune_cands.empty()) tune_cands = precision == QW_PREC_FP64 ? std::vector<int>{2, 4, 8} : std::vector<int>{4, 8, 16};
     return tune_cands;

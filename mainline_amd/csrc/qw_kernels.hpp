@@ -30,7 +30,7 @@ struct DmcCtl {
 // ---------------------------------------------------------------- LCAO of one point
 // Lane j < n accumulates MO j: phi[c] = sum_b C[b][j] chi[c][b] over all basis chunks.
 // chi is an LDS tile of 5 x S.chunk_nf doubles.  Block-wide barriers separate the tile
-// producer (basis_lap) from the consumer.
+// producer (basis_lap_sparse) from the consumer.
 // flist: LDS tile of S.chunk_nf ints (indices of the active functions).
 __device__ inline void lcao_lap_n(const DevSys& S, int s, int n, const double p[3], double* chi, int* flist,
                                   double phi[5], int lane) {
@@ -586,9 +586,10 @@ __host__ __device__ inline size_t sweep_lds_bytes(int ne, int na, int nsh, int n
 // The sweep of walker w by wavefront `wid` of a block of WPB wavefronts, each with a whole
 // region of sweep_lds_bytes of its own (lds0: the block's LDS) and wavefront-level barriers
 // when WPB > 1: the same arithmetic as a one-walker block.
-template <int NS, int DEPTH, int U, int WPB>
+template <int NS, int U, int WPB>
 __device__ __forceinline__ void sweep_fp64_body(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int w,
                                                 int lane, int wid, char* lds0) {
+  constexpr int DEPTH = 2;  // delayed rejection (the DMC moves: qw_panel.hpp)
   if (w >= W.nw) return;
   const int ne = S.ne, s = A.s, n = s ? S.ndn : S.nup, nsp = S.nsp, off = s ? S.nup : 0;
   char* base = lds0;
@@ -658,12 +659,7 @@ __device__ __forceinline__ void sweep_fp64_body(const DevSys& S, const DevWalker
       dn[2] = t3 / t0 + gj[2];
       const bool neg = t0 < 0;
       double acc, lnn = 0;
-      if constexpr (DEPTH == 1) {
-        // |ratio|^2 exp(dtrans) as t0^2 exp(2 du + dtrans): one exponential, no logarithm
-        acc = (A.restrict_nodes && neg)
-                  ? 0.0
-                  : fmin(1.0, t0 * t0 * exp(2.0 * (un - u0) + (trans(rn, dn, r0, t) - trans(r0, d0, rn, t))));
-      } else if (dep == 1) {
+      if (dep == 1) {
         lnn = log(fabs(t0)) + (un - u0);
         double rr = exp(lnn);
         acc = (A.restrict_nodes && neg) ? 0.0
@@ -745,7 +741,7 @@ __device__ __forceinline__ void sweep_fp64_body(const DevSys& S, const DevWalker
 // on each other, so one launch takes them all.  What bounds it: the latency of a move's serial chain
 // (small systems leave most SIMDs one wavefront).  Measured, a step of two sweeps: 256 walkers with 2
 // electrons of a spin 179 us in four launches, 150 in one.
-template <int NS, int DEPTH, int U>
+template <int NS, int U>
 __global__ __launch_bounds__(64, 2) void k_sweeps(DevSys S, DevWalkers W, SweepArgs A, int nsw) {
   extern __shared__ double lds[];
   for (int i = 0; i < 2 * nsw; i++) {
@@ -758,7 +754,7 @@ __global__ __launch_bounds__(64, 2) void k_sweeps(DevSys S, DevWalkers W, SweepA
       __threadfence_block();
       __syncthreads();
     }
-    sweep_fp64_body<NS, DEPTH, U, 1>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, 0, (char*)lds);
+    sweep_fp64_body<NS, U, 1>(S, W, A, (int)blockIdx.x, (int)threadIdx.x, 0, (char*)lds);
   }
 }
 

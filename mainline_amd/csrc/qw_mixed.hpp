@@ -1,7 +1,7 @@
 // Mixed-precision path.
 //
-//   inverse of each spin channel and the MO cache in FP32; the inverse is held in VGPRs for a
-//   sweep and updated by FP32 Sherman-Morrison;
+//   inverse of each spin channel and the MO cache in FP32, updated by FP32 Sherman-Morrison (BF16
+//   modes: the inverse in VGPRs for a launch's moves; FP32 LCAO: qw_panel_mx.hpp and qw_big_mx.hpp);
 //   LCAO either FP32 on the VALU (lane = MO) or on MFMA (v_mfma_f32_16x16x32_bf16) with the
 //   operands split into BF16 terms and FP32 accumulation: x = x0 + x1 (+ x2), products kept
 //   down to the chosen order (3 products: "bf16x3", 6 products: "bf16x6"; Henry, Tang and

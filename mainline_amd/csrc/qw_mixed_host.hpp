@@ -65,7 +65,7 @@ void mixed_setup(qw_engine& e) {
     }
   }
   M.ready = 1;
-  // the LDS-staged sweep variant is a tuning candidate where its LDS fits one workgroup
+  // the LDS-staged sweep variant can be forced (QW_SWEEP) where its LDS fits one workgroup
   int maxlds = 0;
   if (hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, e.device) != hipSuccess) maxlds = 0;
   const size_t need = panel_mx_lds_bytes(e.S.na, e.S.nsh, e.S.ntab, e.ns, 2, e.S.nb, e.S.nsp, e.S.usual);

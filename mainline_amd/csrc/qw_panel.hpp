@@ -353,8 +353,6 @@ __device__ inline void lcao_join(const double acc[R][5], double phi[5]) {
 #pragma unroll
   for (int c = 0; c < 5; c++) {
     if constexpr (G == 2 && R == 2) phi[c] = swap32_add(acc[0][c], acc[1][c]);
-    else if constexpr (G == 4 && R == 4)
-      phi[c] = swap16_add(swap32_add(acc[0][c], acc[2][c]), swap32_add(acc[1][c], acc[3][c]));
     else if constexpr (G == 4 && R == 2)
       phi[c] = swap16_add(swap32_add(acc[0][c], acc[0][c]), swap32_add(acc[1][c], acc[1][c]));
     else {

@@ -10,11 +10,11 @@ void small(const DevSys& S, const DevWalkers& W, const SweepArgs& A, int nsw, in
   const size_t lds = sweep_lds_bytes(S.ne, S.na, S.nsh, S.ntab, ns, kCapF64, sizeof(double), 2);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(64), lds, st, S, W, A, nsw); };
   switch (ns) {
-    case 4: go(k_sweeps<4, 2, U>); break;
-    case 8: go(k_sweeps<8, 2, U>); break;
-    case 16: go(k_sweeps<16, 2, U>); break;
-    case 32: go(k_sweeps<32, 2, U>); break;
-    default: go(k_sweeps<64, 2, U>); break;
+    case 4: go(k_sweeps<4, U>); break;
+    case 8: go(k_sweeps<8, U>); break;
+    case 16: go(k_sweeps<16, U>); break;
+    case 32: go(k_sweeps<32, U>); break;
+    default: go(k_sweeps<64, U>); break;
   }
 }
 }  // namespace
@@ -29,11 +29,10 @@ void launch_sweeps_vmc64(const DevSys& S, const DevWalkers& W, const SweepArgs& 
 void launch_sweep_vmc64_big(const DevSys& S, const DevWalkers& W, const SweepArgs& A, hipStream_t st) {
   // one wavefront per walker, lanes over two (<= 128 per spin) or four rows
   const int n = S.nup > S.ndn ? S.nup : S.ndn;
-  const BigPtrs<double> P{W.inv, W.mo, {S.C[0], S.C[1]}, S.spline};
-  const size_t lds = sweep_w_lds_bytes(S.ne, S.na, S.nsh, S.ntab, S.nsp, kCapF64, sizeof(double));
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(kWave), lds, st, S, W, P, A, kCapF64); };
-  if (n <= 2 * kWave) go(k_sweep_w<double, double, 2, 2>);
-  else go(k_sweep_w<double, double, 2, 4>);
+  const size_t lds = sweep_w_lds_bytes(S.ne, S.na, S.nsh, S.ntab, S.nsp);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(W.nw), dim3(kWave), lds, st, S, W, A); };
+  if (n <= 2 * kWave) go(k_sweep_w<2>);
+  else go(k_sweep_w<4>);
 }
 
 }  // namespace qw
