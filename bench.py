@@ -342,16 +342,22 @@ def serving_leg(precision, njobs, rate, seed, tmp):
     return res
 
 
+# the kernel behind the "k_sweep" event times of a DMC run up to 64 electrons of a spin
+SWEEP_KERNEL = {"fp64": "k_sweep_p<1,64,", "mixed_fp32": "k_sweep_mxp<64,1,", "mixed_bf16": "k_sweep_mx<64,1,1>",
+                "mixed_bf16x6": "k_sweep_mx<64,1,2>"}
+
+
 def profile_traffic(precision, walkers):
     """HBM bytes per launch of the sweep kernel (FETCH_SIZE + WRITE_SIZE, scaled by a copy
     kernel's reading) from the counter runs summarised in profiles/traffic.tsv, when a run of
-    this precision and walker count is recorded there; None otherwise."""
+    this kernel, precision and walker count is recorded there; None otherwise."""
     path = os.path.join(ROOT, "profiles", "traffic.tsv")
     if not os.path.exists(path):
         return None
     for line in open(path):
         f = line.rstrip("\n").split("\t")
-        if len(f) >= 5 and not line.startswith("#") and f[1] == precision and int(f[2]) == walkers:
+        if (len(f) >= 5 and not line.startswith("#") and f[0].startswith(SWEEP_KERNEL[precision]) and f[1] == precision
+                and int(f[2]) == walkers):
             return float(f[3]) + float(f[4])
     return None
 

@@ -9,7 +9,7 @@
 // orbital at all.  The pair's own unmoved position is one more point (its Jastrow value).
 //
 // What bounds it: the latency of the shells' table rows and coefficients at three wavefronts per
-// SIMD (30 % of the vector issue slots are used); two shells' rows in flight together take 1.27 ms
+// SIMD (65 % of the vector issue slots are used); two shells' rows in flight together take 1.27 ms
 // against 1.58 one at a time, three and four 1.56 and 1.75 (registers), eight coefficient loads
 // instead of four 1.40.  Contracting the orbitals at every point instead, four points at a time with the
 // wave over orbitals, partners and shells in turn, held 255 registers (two waves per SIMD; now
