@@ -686,7 +686,7 @@ struct qw_engine {
   bool cl_ok = false;  // LDS-staged coefficients fit this device and system
   std::vector<int> tune_cands;
   int u_default() const { return precision == QW_PREC_FP64 ? 4 : 8; }
-  // (The LDS-staged launches can be forced but are not tried: from 1 to 24 electrons of a spin the
+  // (The LDS-staged launches can be forced but are not tried: from 2 to 24 electrons of a spin the
   // fastest of them takes 0.98 to 1.04 times the fastest other, 1024 and 8192 walkers, DMC and VMC; at
   // 32, 48 and 64 and 8192 walkers 1.2, 2.5 and 2.5 times, so trying them cost a new engine's first
   // run 14 %.)
