@@ -914,7 +914,7 @@ struct TmoveArgs {
 };
 
 // The quadrature point of atom a that the draw t selects for electron e, scanning the atom's
-// negative terms from the cumulative value c (the order and terms of k_local's nonlocal loop);
+// negative terms from the cumulative value c (the order and, to rounding, the terms of k_local's sums);
 // writes the new position.  All lanes take part (LCAO over the MOs, Jastrow over electrons).
 // MD: several determinants, ratios as weighted sums over the determinants (weights bw, sum
 // den, the walker's inverses md_inv; phq: LDS row for the MO values at a quadrature point).
@@ -942,6 +942,8 @@ __device__ inline void tmove_target(const DevSys& S, const DevWalkers& W, int w,
   const double ivk =
       (!MD && lane < n) ? (double)inv_store<TM>(W)[(((size_t)w * 2 + s) * nsp + k) * nsp + lane] : 0.0;
   int pick = -1;
+  // (a term within rounding of zero that k_local counted may come out positive here: no move)
+  for (int d = 0; d < 3; d++) np_out[d] = re[d];
   for (int q = 0; q < P.aip && pick < 0; q++) {
     const double qx = P.q[q][0] * rot[0] + P.q[q][1] * rot[3] + P.q[q][2] * rot[6];
     const double qy = P.q[q][0] * rot[1] + P.q[q][1] * rot[4] + P.q[q][2] * rot[7];
